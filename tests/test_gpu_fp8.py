@@ -172,3 +172,32 @@ def test_fp8_layer_config5_full_size():
     assert torch.equal(st["counts"].cpu(), ref["counts"])
     assert int(st["counts"].sum()) == case.T * case.k
     assert rel_l2(out[tokens].float(), ref["out"]) <= FP8_LAYER_TOL
+
+
+# segment lengths at the edges of the tiled kernel's row variants (32, 64, 128, 192, 256 rows), of
+# its even split into tiles (257, 300, 513) and an empty one; K = 1 to 7 steps of its rings, and
+# one K past its limit (the streaming kernel's)
+@pytest.mark.parametrize("K", [128, 256, 384, 512, 896, 8320])
+@pytest.mark.parametrize("epilogue", [0, 1, 2], ids=["swiglu", "relu2", "none"])
+@pytest.mark.parametrize("gather", [False, True])
+def test_fp8_many_rows_equal_the_streaming_kernel(K, epilogue, gather):
+    """Bit for bit: the packed GEMM over long segments (tiled kernel) against the plain-weight one
+    (32 rows at a time), which sum the same blocks in the same order."""
+    from nexttransformer_amd import _native as nat
+    from nexttransformer_amd import ops
+    g = torch.Generator().manual_seed(K + epilogue)
+    counts = [1, 32, 33, 0, 64, 65, 128, 129, 192, 193, 256, 257, 300, 513]
+    S, n_out, rows = len(counts), 128, sum(counts)
+    R = 2 * n_out if epilogue == nat.EPI_SWIGLU else n_out
+    a_rows = 700 if gather else rows
+    src = (torch.randint(0, a_rows, (rows,), generator=g, dtype=torch.int32).cuda() if gather
+           else None)
+    aq, as_ = ops.quantize_fp8_rowwise(_mixed_rows(a_rows, K, 5).cuda())
+    w = torch.randn(S, R, K, generator=g).cuda() * 0.05
+    w[2] *= 1e-3
+    wq, ws = ops.quantize_fp8_blockwise(w)
+    seg = _segments(counts).cuda()
+    plain = ops.grouped_gemm_fp8(aq, as_, src, seg, wq, ws, epilogue, rows, False)
+    tiled = ops.grouped_gemm_fp8(aq, as_, src, seg, ops.pack_expert_weights_fp8(wq, epilogue), ws,
+                                 epilogue, rows, True)
+    assert torch.equal(plain, tiled)
