@@ -327,6 +327,23 @@ int nt_moe_grouped_gemm_bf16_packed_keep(const uint16_t* a, int64_t ld_a, int64_
                                          nt_moe_stream_t stream);
 
 /*
+ * The routed experts' packed product and the shared expert's with the same epilogue (the expert
+ * loop and shared_experts(hidden), megatron_moe.py:145,150) in one call: the results of two
+ * nt_moe_grouped_gemm_bf16_packed calls (_keep with pre and shared_pre), one launch where the
+ * routed segments are short. shared_a bf16 [shared_rows, shared_K] (row stride shared_ld_a),
+ * shared_offsets device {0, shared_rows}, shared_w packed [1, rows, shared_K]; the shared widths
+ * may differ from the routed ones. pre and shared_pre: both or neither (SWIGLU, RELU2).
+ * Conditions as nt_moe_grouped_gemm_bf16_packed(_keep) for each product; shared_rows >= 1.
+ */
+int nt_moe_grouped_gemm_bf16_packed_shared(
+    const uint16_t* a, int64_t ld_a, int64_t a_rows, const int32_t* src_row,
+    const int32_t* seg_offsets, int32_t num_segments, int64_t total_rows, const uint16_t* w_packed,
+    int32_t K, int32_t n_out, uint16_t* c, uint16_t* pre, const uint16_t* shared_a,
+    int64_t shared_ld_a, int64_t shared_rows, const int32_t* shared_offsets,
+    const uint16_t* shared_w, int32_t shared_K, int32_t shared_n_out, uint16_t* shared_c,
+    uint16_t* shared_pre, int32_t epilogue, nt_moe_stream_t stream);
+
+/*
  * FP8 path (OCP E4M3FN, the format of gfx950's matrix cores). The reference has no fp8
  * experts -- its MasterLinear runs bf16/fp32 matmuls (megatron_moe.py:58-78) -- so these entry
  * points are the fp8 variant of the same expert computation (megatron_moe.py:145) for the

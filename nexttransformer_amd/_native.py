@@ -68,6 +68,9 @@ SIGNATURES = {
     "nt_moe_router_operands": (_i32, [_p, _i64, _i32, _i32, _i32, _p, _i64, _i32, _p, _p, _i32,
                                        _i32, _p]),
     "nt_moe_pack_expert_weights_bf16": (_i32, [_p, _i64, _i32, _i32, _i32, _p, _p]),
+    "nt_moe_grouped_gemm_bf16_packed_shared": (_i32, [_p, _i64, _i64, _p, _p, _i32, _i64, _p, _i32,
+                                                      _i32, _p, _p, _p, _i64, _i64, _p, _p, _i32,
+                                                      _i32, _p, _p, _i32, _p]),
     "nt_moe_grouped_gemm_bf16_packed": (_i32, [_p, _i64, _i64, _p, _p, _i32, _i64, _p, _i32, _i32,
                                                _i32, _p, _p]),
     "nt_moe_quantize_fp8_rowwise": (_i32, [_p, _i64, _i64, _i32, _p, _i64, _p, _p]),

@@ -807,6 +807,42 @@ int nt_moe_grouped_gemm_bf16_packed_keep(const uint16_t* a, int64_t ld_a, int64_
                   "grouped_gemm_packed_keep");
 }
 
+int nt_moe_grouped_gemm_bf16_packed_shared(
+    const uint16_t* a, int64_t ld_a, int64_t a_rows, const int32_t* src_row,
+    const int32_t* seg_offsets, int32_t num_segments, int64_t total_rows, const uint16_t* w_packed,
+    int32_t K, int32_t n_out, uint16_t* c, uint16_t* pre, const uint16_t* shared_a,
+    int64_t shared_ld_a, int64_t shared_rows, const int32_t* shared_offsets,
+    const uint16_t* shared_w, int32_t shared_K, int32_t shared_n_out, uint16_t* shared_c,
+    uint16_t* shared_pre, int32_t epilogue, nt_moe_stream_t stream) {
+  NT_REQUIRE((pre == nullptr) == (shared_pre == nullptr),
+             "grouped_gemm_packed_shared: both products keep their pre-activations or neither");
+  NT_REQUIRE(!pre || epilogue != NT_MOE_EPI_NONE,
+             "grouped_gemm_packed_shared: pre-activations need the SWIGLU or RELU2 epilogue");
+  int rc = check_packed(a, ld_a, a_rows, src_row, seg_offsets, num_segments, total_rows, w_packed,
+                        K, n_out, epilogue, c);
+  if (rc) return rc;
+  NT_REQUIRE(shared_rows >= 1, "grouped_gemm_packed_shared: shared_rows must be positive");
+  rc = check_packed(shared_a, shared_ld_a, shared_rows, nullptr, shared_offsets, 1, shared_rows,
+                    shared_w, shared_K, shared_n_out, epilogue, shared_c);
+  if (rc) return rc;
+  if (pre) {
+    const int64_t f = epilogue == NT_MOE_EPI_SWIGLU ? 2 : 1;
+    NT_REQUIRE(total_rows * f * n_out * 2 < ((int64_t)1 << 31) &&
+                   shared_rows * f * shared_n_out * 2 < ((int64_t)1 << 31),
+               "grouped_gemm_packed_shared: the pre-activations must stay below 2 GiB");
+    NT_REQUIRE(aligned16(pre) && aligned16(shared_pre),
+               "grouped_gemm_packed_shared: the pre-activations must be 16-byte aligned");
+  }
+  const FewPart routed{a, ld_a, a_rows, src_row, w_packed, K, n_out, c, pre};
+  const FewPart shared{shared_a, shared_ld_a, shared_rows, nullptr, shared_w,
+                       shared_K, shared_n_out, shared_c, shared_pre};
+  return launched(launch_grouped_gemm_bf16_packed_shared(routed, seg_offsets, num_segments,
+                                                         total_rows, shared, shared_rows,
+                                                         shared_offsets, epilogue,
+                                                         reinterpret_cast<hipStream_t>(stream)),
+                  "grouped_gemm_packed_shared");
+}
+
 int nt_moe_quantize_fp8_rowwise(const uint16_t* x, int64_t ld_x, int64_t rows, int32_t d,
                                 uint8_t* q, int64_t ld_q, float* scale, nt_moe_stream_t stream) {
   NT_REQUIRE(rows >= 0 && rows < ((int64_t)1 << 31), "quantize_fp8_rowwise: bad row count");

@@ -179,6 +179,30 @@ hipError_t launch_grouped_gemm_bf16_packed(const uint16_t* a, int64_t ld_a, int6
                                            const uint16_t* wp, int K, int n_out, int epilogue,
                                            uint16_t* c, hipStream_t stream);
 int packed_gemm_min_k();
+// One product of grouped_gemm_few.hip: rows of a (gathered through src_row when given) against
+// packed weights w of K columns and n_out outputs; pre (up projections) also takes the fc1
+// pre-activations.
+struct FewPart {
+  const uint16_t* a;
+  int64_t ld_a, a_rows;
+  const int32_t* src_row;
+  const uint16_t* w;
+  int K, n_out;
+  uint16_t* c;
+  uint16_t* pre;
+};
+// Routed and shared product (grouped_gemm_packed.hip); shared_offsets: device [0, shared_rows].
+hipError_t launch_grouped_gemm_bf16_packed_shared(const FewPart& routed, const int32_t* seg_offsets,
+                                                  int num_segments, int64_t total_rows,
+                                                  const FewPart& shared, int64_t shared_rows,
+                                                  const int32_t* shared_offsets, int epilogue,
+                                                  hipStream_t stream);
+// The packed GEMM for few rows per segment; with `shared`, also shared_rows rows (one segment, no
+// gather) of a second product with the same epilogue, in the same launch.
+hipError_t launch_grouped_gemm_bf16_few(const FewPart& routed, const int32_t* seg_offsets,
+                                        int num_segments, int64_t total_rows,
+                                        const FewPart* shared, int64_t shared_rows, int epilogue,
+                                        hipStream_t stream);
 // The ping-pong packed GEMM (grouped_gemm_pp.hip): same operands and results as the packed
 // kernel; pre (the fc1 pre-activations, SWIGLU / RELU2 only) may be null.
 bool pp_gemm_supported(int K, int num_segments);

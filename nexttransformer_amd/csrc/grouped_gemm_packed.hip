@@ -794,12 +794,27 @@ static bool packed_edge(int K, int n_out, int epilogue) {
   return (K / kBK) % 2 != 0 || NB % kTileBlocks != 0;
 }
 
+// Whether the kernel for few rows per segment takes a shape (grouped_gemm_few.hip): up to 32 rows
+// per segment on average, where it won on every shape measured (1 to 25 % at 32 rows, 10 to 50 %
+// below 8); up to 64 where a segment's weights are 1 MB or more (128 experts of 6 and 3 MB at 49
+// rows 153 / 87 -> 146 / 85 us, 32 experts of 2 and 1 MB at 64 rows 19.4 / 12.8 -> 18.9 / 11.9,
+// 256 experts of 1.6 MB at 48 rows 87 / 102 -> 85 / 93), since with smaller weights each
+// workgroup's start and stores weigh more than its stream (0.8 MB at 48 rows 48 / 53 -> 52 / 55).
+static bool few_rows(int num_segments, int64_t total_rows, int K, int n_out, int epilogue) {
+  const int64_t weights = (int64_t)(epilogue == NT_MOE_EPI_SWIGLU ? 2 : 1) * n_out * K * 2;
+  return total_rows <= (weights >= (1 << 20) ? 64 : 32) * (int64_t)num_segments;
+}
+
 hipError_t launch_grouped_gemm_bf16_packed(const uint16_t* a, int64_t ld_a, int64_t a_rows,
                                            const int32_t* src_row, const int32_t* seg_offsets,
                                            int num_segments, int64_t total_rows,
                                            const uint16_t* wp, int K, int n_out, int epilogue,
                                            uint16_t* c, hipStream_t stream) {
   if (total_rows == 0) return hipSuccess;
+  if (few_rows(num_segments, total_rows, K, n_out, epilogue))
+    return launch_grouped_gemm_bf16_few(FewPart{a, ld_a, a_rows, src_row, wp, K, n_out, c, nullptr},
+                                        seg_offsets, num_segments, total_rows, nullptr, 0,
+                                        epilogue, stream);
   if (use_pp() && pp_gemm_supported(K, num_segments))
     return launch_grouped_gemm_bf16_pp(a, ld_a, a_rows, src_row, seg_offsets, num_segments,
                                        total_rows, wp, K, n_out, epilogue, c, nullptr, stream);
@@ -837,6 +852,10 @@ hipError_t launch_grouped_gemm_bf16_packed_keep(const uint16_t* a, int64_t ld_a,
                                                 int n_out, int epilogue, uint16_t* c,
                                                 uint16_t* pre, hipStream_t stream) {
   if (total_rows == 0) return hipSuccess;
+  if (few_rows(num_segments, total_rows, K, n_out, epilogue))
+    return launch_grouped_gemm_bf16_few(FewPart{a, ld_a, a_rows, src_row, wp, K, n_out, c, pre},
+                                        seg_offsets, num_segments, total_rows, nullptr, 0,
+                                        epilogue, stream);
   if (use_pp() && pp_gemm_supported(K, num_segments))
     return launch_grouped_gemm_bf16_pp(a, ld_a, a_rows, src_row, seg_offsets, num_segments,
                                        total_rows, wp, K, n_out, epilogue, c, pre, stream);
@@ -862,6 +881,32 @@ hipError_t launch_grouped_gemm_bf16_packed_keep(const uint16_t* a, int64_t ld_a,
   NT_PK(NT_MOE_EPI_RELU2);
 #undef NT_PK
 #undef NT_PKE
+}
+
+// The routed product and the shared expert's (one segment of shared_rows rows, no gather, the same
+// epilogue): one launch where the routed rows are few, else one after the other. Past 2048 shared
+// rows (top-1 and top-2 routing over many experts) also one after the other: the shared tiles
+// are then too much work for the kernel for few rows (d 2048, 3072 wide, 3001 rows alone 125 us
+// against 47) to hide under the routed weight stream.
+hipError_t launch_grouped_gemm_bf16_packed_shared(const FewPart& routed, const int32_t* seg_offsets,
+                                                  int num_segments, int64_t total_rows,
+                                                  const FewPart& shared, int64_t shared_rows,
+                                                  const int32_t* shared_offsets, int epilogue,
+                                                  hipStream_t stream) {
+  if (total_rows > 0 && shared_rows <= 2048 &&
+      few_rows(num_segments, total_rows, routed.K, routed.n_out, epilogue))
+    return launch_grouped_gemm_bf16_few(routed, seg_offsets, num_segments, total_rows, &shared,
+                                        shared_rows, epilogue, stream);
+  auto one = [&](const FewPart& p, const int32_t* offsets, int segments, int64_t rows) {
+    return p.pre ? launch_grouped_gemm_bf16_packed_keep(p.a, p.ld_a, p.a_rows, p.src_row, offsets,
+                                                        segments, rows, p.w, p.K, p.n_out,
+                                                        epilogue, p.c, p.pre, stream)
+                 : launch_grouped_gemm_bf16_packed(p.a, p.ld_a, p.a_rows, p.src_row, offsets,
+                                                   segments, rows, p.w, p.K, p.n_out, epilogue,
+                                                   p.c, stream);
+  };
+  hipError_t err = one(routed, seg_offsets, num_segments, total_rows);
+  return err != hipSuccess ? err : one(shared, shared_offsets, 1, shared_rows);
 }
 
 }  // namespace ntmoe

@@ -367,3 +367,49 @@ def test_split_partial_tiles_match_plain(epilogue, n_out):
             torch.cuda.synchronize()
             assert torch.equal(c.view(torch.int16), plain.view(torch.int16)), K
             assert torch.equal(pre.view(torch.int16), z.view(torch.int16)), K
+
+
+# mean rows per segment on both sides of the rules (32, and 64 with 1 MB of weights per segment);
+# within them empty, one-row, 32 / 33, 64 / 65, 128 / 129-row and split (300) segments; the shared
+# width equal, smaller with a partial tile, or larger; K steps short of and past the rings' lengths
+@pytest.mark.parametrize("counts", [[1], [3, 0, 1, 2], [0, 1, 32, 33, 5, 0, 31, 2, 40],
+                                    [64, 65, 0, 128, 129, 1, 2, 3, 7, 9, 0, 0],
+                                    [300, 4, 0, 1, 0, 2, 0, 1, 30]], ids=str)
+@pytest.mark.parametrize("K,n_out,K_s,n_s,T", [(256, 64, 256, 64, 1), (320, 160, 320, 160, 65),
+                                               (1024, 512, 256, 96, 130), (448, 96, 512, 288, 33)])
+@pytest.mark.parametrize("epilogue", [0, 1, 2], ids=["swiglu", "relu2", "none"])
+@pytest.mark.parametrize("gather", [False, True])
+def test_few_rows_with_shared_expert_equal_the_tiled_kernel(counts, K, n_out, K_s, n_s, T,
+                                                            epilogue, gather):
+    """Bit for bit, outputs and kept pre-activations: the one-call routed + shared product over
+    short segments against the 256-row plain-weight kernel (the same per-element K order)."""
+    from nexttransformer_amd import _native as nat
+    from nexttransformer_amd import ops
+    g = torch.Generator().manual_seed(K + len(counts))
+    f = 2 if epilogue == nat.EPI_SWIGLU else 1
+    S, rows = len(counts), sum(counts)
+    off = torch.tensor([0] + counts).cumsum(0).to(torch.int32).cuda()
+    mk = lambda *s: torch.randn(s, generator=g).to(torch.bfloat16).cuda()
+    a = mk(70 if gather else rows, K)
+    src = torch.randint(0, 70, (rows,), generator=g, dtype=torch.int32).cuda() if gather else None
+    xs, w, ws = mk(T, K_s), mk(S, f * n_out, K), mk(1, f * n_s, K_s)
+    seg = torch.tensor([0, T], dtype=torch.int32).cuda()
+    pw, pws = ops.pack_expert_weights(w, epilogue), ops.pack_expert_weights(ws, epilogue)
+    keep = epilogue != nat.EPI_NONE
+    c, pre, cs, pres = ops.grouped_gemm_packed_shared(a, src, off, pw, epilogue, rows, xs, pws, keep)
+
+    def plain(rows_in, idx, offs, wt, n, total):
+        """(c, pre) of the plain-weight kernel, whose widths are multiples of 64: zero weight rows
+        added behind each half and their columns dropped again."""
+        wt = torch.nn.functional.pad(wt.view(wt.shape[0], f, n, -1), (0, 0, 0, -n % 64)).flatten(1, 2)
+        if not keep:
+            return ops.grouped_gemm(rows_in, idx, offs, wt, epilogue, total)[:, :n], None
+        out, z = ops.grouped_gemm_keep(rows_in, idx, offs, wt, epilogue, total)
+        return out[:, :n], z.view(total, f, -1)[:, :, :n].flatten(1)
+
+    ref, ref_pre = plain(a, src, off, w, n_out, rows)
+    ref_s, ref_pres = plain(xs, None, seg, ws, n_s, T)
+    assert torch.equal(c, ref) and torch.equal(cs, ref_s)
+    if keep:
+        assert torch.equal(pre, ref_pre) and torch.equal(pres, ref_pres)
+    assert torch.equal(ops.grouped_gemm_packed(a, src, off, pw, epilogue, rows), ref)
