@@ -461,6 +461,14 @@ int nt_moe_router_plan(const uint16_t* x, int64_t ld_x, const float* w_router_t,
     return fail(NT_MOE_ENOSPC, "router_plan: workspace %zu < %zu bytes", workspace_bytes, need);
   const size_t router_part = align256(router_workspace_need(T, d, E));
   void* plan_ws = reinterpret_cast<char*>(workspace) + router_part;
+  if (router_small(T, d, E, k)) {  // ranking and plan over the whole chip, three launches in all
+    const RoutePlanOut plan{counts, offsets, src_row, perm_w, combine_dest, combine_w};
+    return launched(launch_router(x, ld_x, w_router_t, logit_bias, T, d, E, k, score_fn, logits,
+                                  topk_ids, topk_w, prob_partial, z_partial,
+                                  reinterpret_cast<float*>(workspace), router_part, st, nullptr,
+                                  &plan),
+                    "router_plan");
+  }
   const bool from_counts = plan_from_counts(T, E);
   hipError_t err = launch_router(x, ld_x, w_router_t, logit_bias, T, d, E, k, score_fn, logits,
                                  topk_ids, topk_w, prob_partial, z_partial,

@@ -60,11 +60,23 @@ inline int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 
 // Kernel launchers (one per translation unit). They assume validated arguments and return
 // a hipError_t from the launch.
+// The route plan's outputs (nt_moe_route_plan); perm_w may be null.
+struct RoutePlanOut {
+  int32_t* counts;
+  int32_t* offsets;
+  int32_t* src_row;
+  float* perm_w;
+  int32_t* combine_dest;
+  float* combine_w;
+};
+// plan: also the route plan (only where router_small, with the router's whole workspace).
+bool router_small(int64_t T, int d, int E, int k);
 hipError_t launch_router(const uint16_t* x, int64_t ld_x, const float* wt, const float* bias,
                          int64_t T, int d, int E, int k, int score_fn, float* logits,
                          int32_t* topk_ids, float* topk_w, float* prob_partial,
                          float* z_partial, float* workspace, size_t workspace_bytes,
-                         hipStream_t stream, int32_t* block_counts = nullptr);
+                         hipStream_t stream, int32_t* block_counts = nullptr,
+                         const RoutePlanOut* plan = nullptr);
 hipError_t launch_topk_from_logits(const float* logits, int64_t T, int E, int k,
                                    int score_fn, int32_t* topk_ids, float* topk_w,
                                    float* prob_partial, float* z_partial, hipStream_t stream);

@@ -82,30 +82,13 @@ __device__ __forceinline__ void list_insert(float v, int e, float* lv, int* li) 
   }
 }
 
-// Top-k, weights, full scores and aux partials for the 64 tokens whose logits sit in the
-// LDS tile lg[64][E+1]; overwrites lg with the full scores s_te. Called by all 64 * LPT threads
-// of the block: LPT lanes per token, each scanning every LPT-th expert.
-template <int KMAX, int LPT = 4>
-__device__ __forceinline__ void topk_and_scores(float* lg, float* zt, int64_t t0, int64_t T, int E, int k,
-                                int score_fn, int32_t* __restrict__ topk_ids,
-                                float* __restrict__ topk_w, float* __restrict__ prob_partial,
-                                float* __restrict__ z_partial, int32_t* __restrict__ block_counts) {
-  static_assert(LPT == 1 || LPT == 2 || LPT == 4 || LPT == 8 || LPT == 16, "lanes per token");
-  // The block's assignments per expert, for the route plan: a 64-bit mask per expert (bit tt
-  // for token tt; LDS ORs, so the result does not depend on their order) gives the counts
-  // (popcount) and each assignment's rank among the block's tokens that chose its expert
-  // (popcount of the lower bits) -- block_counts[blk][e] and, after the table,
-  // ranks[t k + j] (route_ranks_offset).
-  unsigned long long* msk =
-      reinterpret_cast<unsigned long long*>(reinterpret_cast<unsigned char*>(zt) + kRouteBlock * 4);
-  if (block_counts)
-    for (int e = threadIdx.x; e < E; e += blockDim.x) msk[e] = 0ull;
-  const int ldl = E + 1;
-  const int tt = threadIdx.x / LPT;   // token within the block
-  const int sub = threadIdx.x % LPT;  // which of the LPT expert strides this lane scans
-  const int64_t t = t0 + tt;
-  float* row = lg + tt * ldl;
-
+// Top-k, weights and full scores of one token, by LPT consecutive lanes (lane sub of them scans
+// every LPT-th expert of the token's logits in LDS, row[0 .. E)); row is left holding the full
+// scores s_te, oi the selected experts in order. Returns the squared logsumexp.
+template <int KMAX, int LPT>
+__device__ __forceinline__ float rank_token(float* row, int sub, int64_t t, int64_t T, int E, int k,
+                                            int score_fn, int32_t* __restrict__ topk_ids,
+                                            float* __restrict__ topk_w, int (&oi)[KMAX]) {
   float lv[KMAX];
   int li[KMAX];
 #pragma unroll
@@ -137,7 +120,6 @@ __device__ __forceinline__ void topk_and_scores(float* lg, float* zt, int64_t t0
 
   // k rounds: best head of the LPT lists (xor butterfly), the owner pops it.
   float ov[KMAX];
-  int oi[KMAX];
 #pragma unroll
   for (int j = 0; j < KMAX; ++j) {
     float bv = lv[0];
@@ -207,7 +189,36 @@ __device__ __forceinline__ void topk_and_scores(float* lg, float* zt, int64_t t0
     const float inv = 1.f / spart;
     for (int e = sub; e < E; e += LPT) row[e] = inv / row[e];
   }
-  if (sub == 0) zt[tt] = lse * lse;
+  return lse * lse;
+}
+
+// Top-k, weights, full scores and aux partials for the 64 tokens whose logits sit in the
+// LDS tile lg[64][E+1]; overwrites lg with the full scores s_te. Called by all 64 * LPT threads
+// of the block: LPT lanes per token, each scanning every LPT-th expert.
+template <int KMAX, int LPT = 4>
+__device__ __forceinline__ void topk_and_scores(float* lg, float* zt, int64_t t0, int64_t T, int E, int k,
+                                int score_fn, int32_t* __restrict__ topk_ids,
+                                float* __restrict__ topk_w, float* __restrict__ prob_partial,
+                                float* __restrict__ z_partial, int32_t* __restrict__ block_counts) {
+  static_assert(LPT == 1 || LPT == 2 || LPT == 4 || LPT == 8 || LPT == 16, "lanes per token");
+  // The block's assignments per expert, for the route plan: a 64-bit mask per expert (bit tt
+  // for token tt; LDS ORs, so the result does not depend on their order) gives the counts
+  // (popcount) and each assignment's rank among the block's tokens that chose its expert
+  // (popcount of the lower bits) -- block_counts[blk][e] and, after the table,
+  // ranks[t k + j] (route_ranks_offset).
+  unsigned long long* msk =
+      reinterpret_cast<unsigned long long*>(reinterpret_cast<unsigned char*>(zt) + kRouteBlock * 4);
+  if (block_counts)
+    for (int e = threadIdx.x; e < E; e += blockDim.x) msk[e] = 0ull;
+  const int ldl = E + 1;
+  const int tt = threadIdx.x / LPT;   // token within the block
+  const int sub = threadIdx.x % LPT;  // which of the LPT expert strides this lane scans
+  const int64_t t = t0 + tt;
+  float* row = lg + tt * ldl;
+
+  int oi[KMAX];
+  const float z = rank_token<KMAX, LPT>(row, sub, t, T, E, k, score_fn, topk_ids, topk_w, oi);
+  if (sub == 0) zt[tt] = z;
   __syncthreads();
   if (block_counts && t < T) {
 #pragma unroll
@@ -1006,6 +1017,401 @@ __global__ __launch_bounds__(1024) void router_topk_kernel(
                             z_partial, block_counts);
 }
 
+// ---- Ranking over the whole chip --------------------------------------------------------------
+// router_topk_kernel ranks 64 tokens per workgroup, so a batch of a few hundred tokens keeps a
+// few CUs busy (48 tokens of 256 experts: 26 us on one CU, bound by its instruction rate). For
+// batches of up to kRankAssignments selections the same per-token ranking runs 16 tokens per
+// workgroup (router_rank_kernel, which also sums the chunk planes), leaving the scores in the
+// workspace; router_finish_kernel then does what crosses tokens: the aux partials (one workgroup
+// per 64 tokens, the sums in router_topk_kernel's order) and the route plan (one workgroup per
+// 256 tokens, from the ranking workgroups' per-expert counts, one byte each). Router and plan, us
+// before (plane sum, 64-token top-k, plan from its counts) -> after, same bits: 256 experts d 1280
+// 1 / 48 / 777 / 3001 / 8192 tokens 37 / 40 / 59 / 87 / 128 -> 22 / 24 / 38 / 61 / 118 (with
+// router_path's wider use of the planes); 128 experts d 4096 64 / 4096 tokens 33 / 110 -> 23 / 95;
+// 32 experts d 1024 1 / 4095 tokens 19 / 33 -> 15 / 22. Past kRankAssignments selections (T =
+// 8192 at top-8) the fused kernels, or the 64-token top-k over logits, fill the chip.
+constexpr int64_t kRankAssignments = 65536;
+constexpr int kRankTokens = 16;   // per workgroup of 256 threads, 16 lanes each
+constexpr int kPlanTokens = 256;  // per plan workgroup
+// Bytes per row of the counts table [ceil(T / 16)][pitch].
+__host__ __device__ inline int rank_count_pitch(int E) { return (E + 15) & ~15; }
+
+// v of another lane of the 16-lane row: xor 1 and 2 within quads; then, for values alike in a
+// quad (half row), the other quad's (half's).
+template <int STEP>
+__device__ __forceinline__ int row_other(int v) {
+  constexpr int ctrl = STEP == 0 ? 0xB1 : (STEP == 1 ? 0x4E : (STEP == 2 ? 0x141 : 0x140));
+  return __builtin_amdgcn_update_dpp(v, v, ctrl, 0xf, 0xf, false);
+}
+template <int STEP>
+__device__ __forceinline__ float row_other(float v) {
+  return __builtin_bit_cast(float, row_other<STEP>(__builtin_bit_cast(int, v)));
+}
+// Sum over the 16 lanes of a row, in the order of an xor butterfly 1, 2, 4, 8.
+__device__ __forceinline__ float row_sum(float v) {
+  v += row_other<0>(v);
+  v += row_other<1>(v);
+  v += row_other<2>(v);
+  v += row_other<3>(v);
+  return v;
+}
+
+// rank_token for 16 lanes per token with the token's logits in registers: lane sub holds experts
+// sub + 16 i in l[i] (NPL of them). k rounds of an arg-max over the row's registers (a selected
+// logit becomes NaN, which is never taken), all lane exchanges as DPP moves: the list insertions,
+// LDS re-reads and permutes of rank_token are a chain of latencies that nothing hides in a small
+// batch (one token of 256 experts, planes summed here too: 18.6 us that way, 10.3 us this way;
+// of 32 experts 5.3 and 3.4 us). Same bits.
+template <int KMAX, int NPL>
+__global__ __launch_bounds__(256) void router_rank_kernel(
+    const float* __restrict__ planes, int nchunk, const float* __restrict__ bias, int64_t T, int E,
+    int k, int score_fn, float* __restrict__ logits, int32_t* __restrict__ topk_ids,
+    float* __restrict__ topk_w, float* __restrict__ scores, float* __restrict__ z,
+    uint8_t* __restrict__ block_counts) {
+  __shared__ __align__(16) float rows[kRankTokens][NPL * 16 + 1];
+  __shared__ int cnt[NT_MOE_MAX_EXPERTS];
+  cnt[threadIdx.x] = 0;
+  const int tt = threadIdx.x / 16, sub = threadIdx.x % 16;
+  const int64_t t = (int64_t)blockIdx.x * kRankTokens + tt;
+  const int64_t tc = t < T ? t : T - 1;  // rows past the batch rank its last token, unstored
+  const int64_t plane = T * E;
+  float* row = rows[tt];
+  // ((p0 + p1) + p2) + ... + bias: NB planes' loads of all the lane's experts in flight, without
+  // branches (indices clamped; what a clamped one reads is not added)
+  if (E % 4 == 0) {
+    constexpr int G = (NPL + 3) / 4, NB = G == 4 ? 4 : 8;
+    const floatx4* p[G];
+    floatx4 v[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int e = 4 * (sub + 16 * g);
+      p[g] = reinterpret_cast<const floatx4*>(planes + tc * E + (e < E ? e : 0));
+      v[g] = *p[g];
+    }
+    for (int c0 = 1; c0 < nchunk; c0 += NB) {
+      floatx4 part[NB][G];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const int64_t c = c0 + j < nchunk ? c0 + j : nchunk - 1;
+#pragma unroll
+        for (int g = 0; g < G; ++g) part[j][g] = p[g][c * (plane / 4)];
+      }
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        if (c0 + j < nchunk) {
+#pragma unroll
+          for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[g][q] = v[g][q] + part[j][g][q];
+        }
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int e = 4 * (sub + 16 * g);
+      if (e < E) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (bias) v[g][q] = v[g][q] + bias[e + q];
+          row[e + q] = v[g][q];
+        }
+        if (logits && t < T) *reinterpret_cast<floatx4*>(logits + t * E + e) = v[g];
+      }
+    }
+  } else {
+    float v[NPL];
+#pragma unroll
+    for (int i = 0; i < NPL; ++i) {
+      const int e = sub + 16 * i;
+      v[i] = planes[tc * E + (e < E ? e : E - 1)];
+    }
+    for (int c = 1; c < nchunk; ++c) {
+      float part[NPL];
+#pragma unroll
+      for (int i = 0; i < NPL; ++i) {
+        const int e = sub + 16 * i;
+        part[i] = planes[(int64_t)c * plane + tc * E + (e < E ? e : E - 1)];
+      }
+#pragma unroll
+      for (int i = 0; i < NPL; ++i) v[i] = v[i] + part[i];
+    }
+#pragma unroll
+    for (int i = 0; i < NPL; ++i) {
+      const int e = sub + 16 * i;
+      if (e < E) {
+        if (bias) v[i] = v[i] + bias[e];
+        row[e] = v[i];
+        if (logits && t < T) logits[t * E + e] = v[i];
+      }
+    }
+  }
+  __syncthreads();
+  float l[NPL], sel[NPL];
+#pragma unroll
+  for (int i = 0; i < NPL; ++i) {
+    const int e = sub + 16 * i;
+    l[i] = e < E ? row[e] : __builtin_nanf("");
+    sel[i] = l[i];
+  }
+  float ov[KMAX];
+  int oi[KMAX];
+#pragma unroll
+  for (int j = 0; j < KMAX; ++j) {
+    float bv = -INFINITY;
+    int bi = 0x7fffffff;
+#pragma unroll
+    for (int i = NPL - 1; i >= 0; --i) {  // descending, so the lower expert wins a tie
+      const bool c = sel[i] >= bv;
+      bv = c ? sel[i] : bv;
+      bi = c ? sub + 16 * i : bi;
+    }
+    auto take = [&](float v2, int i2) {
+      const bool c = rank_before(v2, i2, bv, bi);
+      bv = c ? v2 : bv;
+      bi = c ? i2 : bi;
+    };
+    take(row_other<0>(bv), row_other<0>(bi));
+    take(row_other<1>(bv), row_other<1>(bi));
+    take(row_other<2>(bv), row_other<2>(bi));
+    take(row_other<3>(bv), row_other<3>(bi));
+    ov[j] = bv;
+    oi[j] = bi;
+#pragma unroll
+    for (int i = 0; i < NPL; ++i) sel[i] = sub + 16 * i == bi ? __builtin_nanf("") : sel[i];
+  }
+  // Routing weights over the k selected: softmax, or sigmoid normalised over the selected.
+  const float top = ov[0];
+  float wsum = 0.f, wv[KMAX];
+#pragma unroll
+  for (int j = 0; j < KMAX; ++j) {
+    const float s = score_fn == NT_MOE_SCORE_SOFTMAX ? expf(ov[j] - top) : 1.f / (1.f + expf(-ov[j]));
+    wv[j] = j < k ? s : 0.f;
+    wsum += wv[j];
+  }
+  const float winv = 1.f / wsum;
+  // Full scores for the load-balance loss, logsumexp for the z-loss.
+  float part = 0.f, spart = 0.f;
+#pragma unroll
+  for (int i = 0; i < NPL; ++i) {
+    if (sub + 16 * i < E) {
+      const float ex = expf(l[i] - top);
+      part += ex;
+      if (score_fn == NT_MOE_SCORE_SIGMOID) {
+        const float den = 1.f + expf(-l[i]);
+        spart += 1.f / den;
+        l[i] = den;
+      } else {
+        l[i] = ex;
+      }
+    }
+  }
+  part = row_sum(part);
+  spart = row_sum(spart);
+  const float lse = top + logf(part);
+  const float inv = 1.f / (score_fn == NT_MOE_SCORE_SOFTMAX ? part : spart);
+  if (t < T) {
+#pragma unroll
+    for (int i = 0; i < NPL; ++i)
+      if (sub + 16 * i < E)
+        scores[t * E + sub + 16 * i] = score_fn == NT_MOE_SCORE_SOFTMAX ? l[i] * inv : inv / l[i];
+    if (sub == 0) z[t] = lse * lse;
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j) {
+      if (j < k && j == sub) {
+        topk_ids[t * k + j] = oi[j];
+        topk_w[t * k + j] = wv[j] * winv;
+        if ((unsigned)oi[j] < (unsigned)E) atomicAdd(&cnt[oi[j]], 1);
+      }
+    }
+  }
+  __syncthreads();
+  const int pitch = rank_count_pitch(E);
+  if ((int)threadIdx.x < pitch)
+    block_counts[(int64_t)blockIdx.x * pitch + threadIdx.x] = (uint8_t)cnt[threadIdx.x];
+}
+
+// Workgroups 0 .. nplan - 1: the route plan of 256 tokens each (plan_kernel's outputs;
+// integer sums, so the same bits). The rest: the aux partials of one 64-token block each.
+template <bool PLAN>
+__global__ __launch_bounds__(256) void router_finish_kernel(
+    const float* __restrict__ scores, const float* __restrict__ z, int64_t T, int E, int k,
+    float* __restrict__ prob_partial, float* __restrict__ z_partial, int nplan,
+    const int32_t* __restrict__ topk_ids, const float* __restrict__ topk_w,
+    const uint8_t* __restrict__ block_counts, RoutePlanOut out) {
+  const int tid = threadIdx.x, lane = lane_id(), w = wave_id();
+  if (!PLAN || (int)blockIdx.x >= nplan) {
+    const int64_t blk = (int64_t)blockIdx.x - nplan, t0 = blk * kRouteBlock;
+    const int nvalid = (int)(T - t0 < kRouteBlock ? T - t0 : kRouteBlock);
+    int P = 64;  // lanes per expert, as in topk_and_scores of a 1024-thread workgroup
+    while (P > 1 && E * P > 1024) P >>= 1;
+    for (int base = 0; base < E * P; base += 256) {
+      const int idx = base + tid, e = idx / P, p = idx % P;
+      float s = 0.f;
+      if (e < E) {
+        for (int r0 = p; r0 < nvalid; r0 += 16 * P) {  // 16 loads in flight
+          float v[16];
+#pragma unroll
+          for (int j = 0; j < 16; ++j) {
+            const int r = r0 + j * P;
+            v[j] = r < nvalid ? scores[(t0 + r) * E + e] : 0.f;
+          }
+#pragma unroll
+          for (int j = 0; j < 16; ++j)
+            if (r0 + j * P < nvalid) s += v[j];
+        }
+      }
+      for (int m = P >> 1; m >= 1; m >>= 1) s += __shfl_xor(s, m);
+      if (e < E && p == 0) prob_partial[blk * E + e] = s;
+    }
+    if (tid < 64) {
+      float s = tid < nvalid ? z[t0 + tid] : 0.f;
+#pragma unroll
+      for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m);
+      if (tid == 0) z_partial[blk] = s;
+    }
+    return;
+  }
+  if constexpr (PLAN) {
+    __shared__ unsigned long long mask[4][NT_MOE_MAX_EXPERTS];  // this workgroup's tokens, by wave
+    __shared__ int tot_s[4][NT_MOE_MAX_EXPERTS], before_s[4][NT_MOE_MAX_EXPERTS];
+    __shared__ int base[NT_MOE_MAX_EXPERTS];
+    __shared__ int wave_tot[4];
+    const int64_t first = (int64_t)blockIdx.x * kPlanTokens;
+    const int64_t t = first + tid;
+    const bool live = t < T;
+    int ev[NT_MOE_MAX_TOPK];
+    float wv[NT_MOE_MAX_TOPK];
+#pragma unroll
+    for (int j = 0; j < NT_MOE_MAX_TOPK; ++j) {
+      ev[j] = 0x7fffffff;
+      wv[j] = 0.f;
+      if (live && j < k) {
+        ev[j] = topk_ids[t * k + j];
+        wv[j] = topk_w[t * k + j];
+      }
+    }
+    for (int e = tid; e < E; e += 256) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) mask[q][e] = 0ull;
+    }
+    // Column sums of the counts table, over all rows and over those before this workgroup's
+    // tokens: 16 bytes (experts) per thread per row, two 16-bit sums to a word (a column's total
+    // is at most T), then the threads of one column group added by shuffles and across waves.
+    const int pitch = rank_count_pitch(E), cg = pitch / 16;  // column groups of 16 experts
+    const int rows = (int)((T + kRankTokens - 1) / kRankTokens);
+    const int before_rows = (int)(first / kRankTokens);
+    // cg groups (1 to 16) padded to a power of two, so a group's threads are lanes apart by it
+    int gp = 1;
+    while (gp < cg) gp <<= 1;
+    const int g = tid & (gp - 1);
+    uint32_t at[8] = {}, ab[8] = {};
+    if (g < cg) {
+      const int step = 256 / gp;
+      for (int r0 = tid / gp; r0 < rows; r0 += 8 * step) {
+        u32x4 v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int r = r0 + j * step;
+          v[j] = r < rows ? *reinterpret_cast<const u32x4*>(block_counts + (int64_t)r * pitch + g * 16)
+                          : u32x4{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const bool b4 = r0 + j * step < before_rows;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const uint32_t lo = v[j][q] & 0x00ff00ffu, hi = (v[j][q] >> 8) & 0x00ff00ffu;
+            at[2 * q] += lo;
+            at[2 * q + 1] += hi;
+            ab[2 * q] += b4 ? lo : 0u;
+            ab[2 * q + 1] += b4 ? hi : 0u;
+          }
+        }
+      }
+    }
+    for (int m = gp; m < 64; m <<= 1) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        at[q] += __shfl_xor(at[q], m);
+        ab[q] += __shfl_xor(ab[q], m);
+      }
+    }
+    if (lane < gp && g < cg) {  // word 2 q + h holds experts 16 g + 4 q + h and + 2
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int e = 16 * g + 4 * (q >> 1) + (q & 1);
+        tot_s[w][e] = at[q] & 0xffffu;
+        tot_s[w][e + 2] = at[q] >> 16;
+        before_s[w][e] = ab[q] & 0xffffu;
+        before_s[w][e + 2] = ab[q] >> 16;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NT_MOE_MAX_TOPK; ++j)
+      if ((unsigned)ev[j] < (unsigned)E) atomicOr(&mask[w][ev[j]], 1ull << lane);
+    __syncthreads();
+    int total = 0, before = 0;  // thread tid owns expert tid
+    if (tid < E) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        total += tot_s[q][tid];
+        before += before_s[q][tid];
+      }
+    }
+    int incl = total;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int u = __shfl_up(incl, o);
+      if (lane >= o) incl += u;
+    }
+    if (lane == 63) wave_tot[w] = incl;
+    __syncthreads();
+    int carry = 0;
+    for (int q = 0; q < w; ++q) carry += wave_tot[q];
+    const int excl = carry + incl - total;
+    if (tid < E) {
+      base[tid] = excl + before;
+      if (blockIdx.x == 0) {
+        out.counts[tid] = total;
+        out.offsets[tid] = excl;
+      }
+    }
+    if (blockIdx.x == 0 && tid == 0)
+      out.offsets[E] = wave_tot[0] + wave_tot[1] + wave_tot[2] + wave_tot[3];
+    __syncthreads();
+    if (!live) return;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    int dv[NT_MOE_MAX_TOPK];
+#pragma unroll
+    for (int j = 0; j < NT_MOE_MAX_TOPK; ++j) {
+      dv[j] = 0;
+      if (j < k) {
+        if ((unsigned)ev[j] < (unsigned)E) {
+          int dest = base[ev[j]] + __popcll(mask[w][ev[j]] & below);
+          for (int q = 0; q < w; ++q) dest += __popcll(mask[q][ev[j]]);
+          out.src_row[dest] = (int32_t)t;
+          if (out.perm_w) out.perm_w[dest] = wv[j];
+          dv[j] = dest;
+        } else {
+          ev[j] = 0x7ffffffe;  // ignored id: sorts last, row 0 as a harmless target
+        }
+      }
+    }
+    // Ascending expert order; equal keys (only ignored ids) keep their slot order.
+#pragma unroll
+    for (int j = 0; j < NT_MOE_MAX_TOPK; ++j) {
+      if (j < k) {
+        int pos = 0;
+#pragma unroll
+        for (int i = 0; i < NT_MOE_MAX_TOPK; ++i)
+          pos += (ev[i] < ev[j] || (ev[i] == ev[j] && i < j)) ? 1 : 0;
+        out.combine_dest[t * k + pos] = dv[j];
+        out.combine_w[t * k + pos] = wv[j];
+      }
+    }
+  }
+}
+
 int kmax_for(int k) { return k <= 2 ? 2 : (k <= 4 ? 4 : 8); }
 
 // Expert blocks of 32 (a power of two: the fused kernel's waves per token row set the top-k's
@@ -1102,19 +1508,36 @@ enum RouterPath { kFused = 0, kLogits = 1, kPlanes = 2, kStream = 3 };
 // when it gives every other SIMD a wave. Measured on MI355X, router alone: T = 16384, d = 1280,
 // E = 256 streamed 142 us (logits + top-k 230); T = 32768, d = 2048, E = 64 fused 122 us
 // (streamed 133); T = 8192, d = 2048, E = 128 logits + top-k 121 us (streamed 131).
+// Up to kPlanesTokens tokens the planes also take the shapes where they are the faster: their
+// grid splits the features, so they run at the chip's rate (about 57 TFLOP/s, plus 7 us for
+// writing and summing the planes), while the logits and the streamed kernel take whole rounds of
+// 64-token workgroups (8.3 and 10.5 us per 128-feature chunk of a workgroup's range). Router and
+// plan with want_logits, E = 256, d = 1280: 4095 tokens streamed 130 us, planes 72; 8192 tokens
+// 128 and 118; 3001 tokens logits 69, planes 63, but 2048 tokens (one full round) 44 and 51.
+constexpr int64_t kPlanesTokens = 8192;  // (T k <= kRankAssignments for every k)
+
 int router_path(int64_t T, int d, int E) {
   const int mode = router_mode_override();
   const int nchunk = ceil_div(d, kRouterChunk);
   const int64_t blocks = ceil_div(T, kRouteBlock);
-  const int64_t logit_waves = blocks * (int64_t)ceil_div(E, 32) * 2 * logit_ranges(d);
+  const int64_t logit_wgs = blocks * (int64_t)ceil_div(E, 32);
+  const int64_t logit_waves = logit_wgs * 2 * logit_ranges(d);
   const int64_t plane_bytes = (int64_t)nchunk * T * E * (int64_t)sizeof(float);
   if (mode == 2) return kPlanes;
   if (mode == 1) return E <= 128 ? kFused : kLogits;
   if (mode == 3) return E > 128 && E <= 256 ? kStream : kLogits;
   if (E <= 128 && blocks >= num_cus()) return kFused;
-  if (E > 128 && E <= 256 && blocks * 8 >= 2LL * num_cus()) return kStream;
-  if (nchunk <= 16 && logit_waves >= 2LL * num_cus()) return kLogits;
-  if (plane_bytes <= (512LL << 20)) return kPlanes;
+  const bool planes_fit = plane_bytes <= (512LL << 20);
+  const double planes_us = 2.0 * T * d * E / 57e6 + 7;
+  auto planes_win = [&](double us_per_round, int64_t workgroups) {
+    return planes_fit && T <= kPlanesTokens &&
+           planes_us < us_per_round * ceil_div(workgroups, num_cus());
+  };
+  if (E > 128 && E <= 256 && blocks * 8 >= 2LL * num_cus())
+    return planes_win(10.5 * nchunk, blocks) ? kPlanes : kStream;
+  if (nchunk <= 16 && logit_waves >= 2LL * num_cus())
+    return planes_win(8.3 * ceil_div(nchunk, logit_ranges(d)), logit_wgs) ? kPlanes : kLogits;
+  if (planes_fit) return kPlanes;
   return nchunk <= 16 ? kLogits : (E <= 128 ? kFused : kStream);
 }
 
@@ -1179,13 +1602,57 @@ hipError_t launch_stream(const uint16_t* x, int64_t ld_x, const float* wt, const
   }
 }
 
+size_t plane_bytes_of(int64_t T, int E) { return (size_t)T * (size_t)E * sizeof(float); }
+
+// router_rank_kernel over the planes (or logits) in `planes`, then router_finish_kernel; the
+// scores take ws's first plane (which may be `planes`), the z terms follow the planes.
+hipError_t launch_rank_finish(const float* planes, int nchunk, const float* bias, int64_t T, int E,
+                              int k, int score_fn, float* logits, int32_t* ids, float* w,
+                              float* pp, float* zp, float* scores, float* z,
+                              const RoutePlanOut* plan, hipStream_t stream) {
+  uint8_t* bc = reinterpret_cast<uint8_t*>(z + (T + 3) / 4 * 4);
+  auto pick = [&](auto kmax_c) {
+    constexpr int KM = decltype(kmax_c)::value;
+    return E <= 32 ? router_rank_kernel<KM, 2>
+                   : (E <= 64 ? router_rank_kernel<KM, 4>
+                              : (E <= 128 ? router_rank_kernel<KM, 8> : router_rank_kernel<KM, 16>));
+  };
+  auto rank = k <= 2 ? pick(std::integral_constant<int, 2>())
+                     : (k <= 4 ? pick(std::integral_constant<int, 4>())
+                               : pick(std::integral_constant<int, NT_MOE_MAX_TOPK>()));
+  hipLaunchKernelGGL(rank, dim3((unsigned)ceil_div(T, kRankTokens)), dim3(256), 0, stream, planes,
+                     nchunk, bias, T, E, k, score_fn, logits, ids, w, scores, z, bc);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  const int nplan = plan ? ceil_div(T, kPlanTokens) : 0;
+  const dim3 grid((unsigned)(nplan + ceil_div(T, kRouteBlock)));
+  if (plan)
+    hipLaunchKernelGGL(router_finish_kernel<true>, grid, dim3(256), 0, stream, scores, z, T, E, k,
+                       pp, zp, nplan, ids, w, bc, *plan);
+  else
+    hipLaunchKernelGGL(router_finish_kernel<false>, grid, dim3(256), 0, stream, scores, z, T, E, k,
+                       pp, zp, 0, ids, w, bc, RoutePlanOut{});
+  return hipGetLastError();
+}
+
 }  // namespace
 
-// Workspace the router uses for this shape: the chunk planes, one T x E logits plane, or none.
+// Whether the router ranks over the whole chip (router_rank_kernel, router_finish_kernel, which
+// then also writes the route plan): the shapes on the planes and logits paths.
+bool router_small(int64_t T, int d, int E, int k) {
+  const int path = router_path(T, d, E);
+  return (path == kPlanes || path == kLogits) && E <= NT_MOE_MAX_EXPERTS &&
+         T * k <= kRankAssignments;
+}
+
+// Workspace the router uses for this shape: the chunk planes or one T x E logits plane, then (for
+// router_small) the tokens' z terms and the ranking workgroups' counts; or none.
 size_t router_workspace_need(int64_t T, int d, int E) {
   const int path = router_path(T, d, E);
-  const size_t plane = (size_t)T * (size_t)E * sizeof(float);
-  return path == kPlanes ? plane * ceil_div(d, kRouterChunk) : (path == kLogits ? plane : 0);
+  const int planes = path == kPlanes ? ceil_div(d, kRouterChunk) : (path == kLogits ? 1 : 0);
+  if (!planes) return 0;
+  const size_t z = (plane_bytes_of(T, E) * planes + 15) / 16 * 16;
+  return z + (size_t)(T + 3) / 4 * 16 + (size_t)ceil_div(T, kRankTokens) * rank_count_pitch(E);
 }
 
 // Runs the path for the shape when its buffers are there; without enough workspace the fused
@@ -1194,10 +1661,13 @@ hipError_t launch_router(const uint16_t* x, int64_t ld_x, const float* wt, const
                          int64_t T, int d, int E, int k, int score_fn, float* logits,
                          int32_t* topk_ids, float* topk_w, float* prob_partial,
                          float* z_partial, float* workspace, size_t workspace_bytes,
-                         hipStream_t stream, int32_t* block_counts) {
+                         hipStream_t stream, int32_t* block_counts, const RoutePlanOut* plan) {
   const int nchunk = ceil_div(d, kRouterChunk);
   const int path = router_path(T, d, E);
-  const size_t plane = (size_t)T * (size_t)E * sizeof(float);
+  const size_t plane = plane_bytes_of(T, E);
+  const bool small = router_small(T, d, E, k) && workspace &&
+                     workspace_bytes >= router_workspace_need(T, d, E);
+  if (plan && !small) return hipErrorInvalidValue;
   hipError_t err;
   if (path == kPlanes && workspace && workspace_bytes >= plane * nchunk) {
     hipLaunchKernelGGL(router_mfma_partial_kernel,
@@ -1206,6 +1676,10 @@ hipError_t launch_router(const uint16_t* x, int64_t ld_x, const float* wt, const
                        dim3(128), 0, stream, x, ld_x, wt, T, d, E, workspace);
     err = hipGetLastError();
     if (err != hipSuccess) return err;
+    if (small)
+      return launch_rank_finish(workspace, nchunk, bias, T, E, k, score_fn, logits, topk_ids,
+                                topk_w, prob_partial, z_partial, workspace,
+                                workspace + (nchunk * T * E + 3) / 4 * 4, plan, stream);
     if (E % 4 == 0) {
       const int64_t n4 = T * E / 4;
       router_sum_planes_kernel<<<dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, stream>>>(
@@ -1237,6 +1711,11 @@ hipError_t launch_router(const uint16_t* x, int64_t ld_x, const float* wt, const
 #undef NT_LOGITS
     err = hipGetLastError();
     if (err != hipSuccess) return err;
+    if (small)
+      return launch_rank_finish(lbuf, 1, nullptr, T, E, k, score_fn, nullptr, topk_ids, topk_w,
+                                prob_partial, z_partial, workspace,
+                                workspace + (T * E + 3) / 4 * 4, plan,
+                                stream);
     return launch_topk_any(lbuf, 1, nullptr, T, E, k, score_fn, nullptr, topk_ids, topk_w,
                            prob_partial, z_partial, block_counts, stream);
   }

@@ -4,6 +4,8 @@ Bar: routing (top-k ids, per-expert counts, offsets, permutation order, combine 
 bit-exact; logits are bit-exact to the fixed-order C restatement; outputs are within relative
 L2 1e-2 of the fp32 reference computed from the same bf16 inputs and bf16-rounded weights.
 """
+import math
+
 import pytest
 import torch
 
@@ -344,3 +346,47 @@ def test_forward_is_deterministic():
     for out, aux in runs[1:]:
         assert torch.equal(out.view(torch.int16), runs[0][0].view(torch.int16))
         assert torch.equal(aux, runs[0][1])
+
+
+# the 16-token ranking workgroups, 64-token partials and 256-token plan workgroups at their edges;
+# experts at the register counts' edges (32, 64, 128, 256) and not multiples of 4 or 16; the
+# largest batch that ranks this way (T k = 65536) and the next
+RANK_CASES = [(1, 2, 1), (15, 5, 5), (16, 16, 2), (17, 17, 3), (63, 32, 4), (64, 33, 8),
+              (65, 64, 8), (255, 65, 1), (256, 128, 8), (257, 129, 6), (300, 250, 5),
+              (777, 256, 8), (8192, 128, 8), (8193, 128, 8), (2049, 8, 8)]
+
+
+@pytest.mark.parametrize("T,E,k", RANK_CASES, ids=str)
+@pytest.mark.parametrize("score_fn", [0, 1], ids=["softmax", "sigmoid"])
+def test_ranking_over_the_chip_equals_the_block_top_k(T, E, k, score_fn):
+    """router_plan against topk_from_logits and route_plan on its own logits, bit for bit (ids,
+    weights, aux partials, plan), with ties, rows that are -inf in all but a few experts or in
+    all, and NaN nowhere selected; the selection also against the CPU oracle."""
+    from nexttransformer_amd import ops
+    d = 64
+    g = torch.Generator().manual_seed(T + E)
+    # integers: every logit exact, many of them equal
+    x = torch.randint(-2, 3, (T, d), generator=g).to(torch.bfloat16)
+    w = torch.randint(-2, 3, (E, d), generator=g).float()
+    bias = torch.zeros(E)
+    bias[::3] = -math.inf
+    if E > 2:
+        bias[1] = 0.5
+    dev = "cuda:0"
+    out = ops.router_plan(x.to(dev), w.t().contiguous().to(dev), bias.to(dev), k, score_fn, True)
+    logits, ids, tw, pp, zp = out[:5]
+    assert torch.equal(logits.cpu(), orc.router_logits_fixed(x, w, bias))
+    ref = ops.topk_from_logits(logits, k, score_fn)
+    bits = lambda t: t.contiguous().view(torch.int32)
+    for got, want in zip((ids, tw, pp, zp), ref):
+        assert torch.equal(bits(got), bits(want))
+    assert torch.equal(ids.cpu(), orc.topk(logits, k, score_fn)[0])
+    plan = ops.route_plan(ids, tw, E, None, False)[:6]
+    for got, want in zip(out[5:], plan):
+        assert torch.equal(bits(got), bits(want))
+    # rows of -inf only: the lowest experts, as the block top-k has it
+    bias[:] = -math.inf
+    out = ops.router_plan(x.to(dev), w.t().contiguous().to(dev), bias.to(dev), k, score_fn, True)
+    ref = ops.topk_from_logits(out[0], k, score_fn)
+    assert torch.equal(out[1], ref[0])
+    assert torch.equal(out[1], torch.arange(k, device=dev, dtype=torch.int32).expand(T, k))
