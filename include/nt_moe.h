@@ -522,6 +522,45 @@ int nt_moe_router_bwd(const float* logits, const int32_t* topk_ids, const float*
                       int32_t k, int32_t score_fn, const float* grad_aux, float aux_coeff,
                       float z_coeff, float* grad_logits, nt_moe_stream_t stream);
 
+/*
+ * The routed experts' activation backward from the hidden gradient before the routing weight,
+ * grad_h[r] = g_t W2_s (g the output's gradient, t the row's token), per expert-major row r with
+ * routing weight row_w[r] (autograd of the weighted expert outputs and of the fc1 activation,
+ * megatron_moe.py:145-148, lm.py:29-35):
+ *   grad_fc1[r]   = act'(fc1[r]) * row_w[r] grad_h[r]   bf16 [rows, 2H] (SwiGLU) or [rows, H]
+ *   weighted_h[r] = row_w[r] h[r]                       bf16 [rows, H] (dW2 = sum_r g_t^T wh_r)
+ *   grad_row_w[r] = <h[r], grad_h[r]>                   fp32 [rows]
+ * fc1, h, grad_h contiguous bf16; H % 8 == 0; the bf16 buffers 16-byte aligned.
+ */
+int nt_moe_act_bwd_rows(const uint16_t* fc1, const uint16_t* h, const uint16_t* grad_h,
+                        const float* row_w, int64_t rows, int32_t H, int32_t activation,
+                        uint16_t* grad_fc1, uint16_t* weighted_h, float* grad_row_w,
+                        nt_moe_stream_t stream);
+
+/* nt_moe_router_bwd with the routing-weight gradients per expert-major row (nt_moe_act_bwd_rows)
+ * and combine_dest int32 [T, k], the token's rows in ascending expert order. */
+int nt_moe_router_bwd_rows(const float* logits, const int32_t* topk_ids, const float* topk_w,
+                           const float* grad_row_w, const int32_t* combine_dest,
+                           const int32_t* counts, int64_t T, int32_t E, int32_t k,
+                           int32_t score_fn, const float* grad_aux, float aux_coeff,
+                           float z_coeff, float* grad_logits, nt_moe_stream_t stream);
+
+/*
+ * Both expert weight gradients (autograd of the per-expert fc1 / fc2 products,
+ * megatron_moe.py:58-78,145), x and g bf16 [token_rows, d] gathered through src_row:
+ *   dw1[s] = sum_r dfc1[r]^T x[src_row[r]]   [F, d]
+ *   dw2[s] = sum_r g[src_row[r]]^T wh[r]     [d, H]
+ * over segment s's rows, fp32 (c_fp32) or bf16. splits1, splits2 and partial as
+ * nt_moe_grouped_wgrad_splitk (partial serves one product after the other: the larger need);
+ * F, d and H multiples of 64; one launch where both take the 256-wide tiles.
+ */
+int nt_moe_expert_wgrads(const uint16_t* dfc1, int64_t ld_dfc1, const uint16_t* x, int64_t ld_x,
+                         const uint16_t* g, int64_t ld_g, int64_t token_rows, const uint16_t* wh,
+                         int64_t ld_wh, const int32_t* src_row, const int32_t* seg_offsets,
+                         int32_t num_segments, int64_t total_rows, int32_t F, int32_t d, int32_t H,
+                         int32_t splits1, int32_t splits2, float* partial, size_t partial_bytes,
+                         int32_t c_fp32, void* dw1, void* dw2, nt_moe_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -68,6 +68,12 @@ SIGNATURES = {
     "nt_moe_router_operands": (_i32, [_p, _i64, _i32, _i32, _i32, _p, _i64, _i32, _p, _p, _i32,
                                        _i32, _p]),
     "nt_moe_pack_expert_weights_bf16": (_i32, [_p, _i64, _i32, _i32, _i32, _p, _p]),
+    "nt_moe_act_bwd_rows": (_i32, [_p, _p, _p, _p, _i64, _i32, _i32, _p, _p, _p, _p]),
+    "nt_moe_router_bwd_rows": (_i32, [_p, _p, _p, _p, _p, _p, _i64, _i32, _i32, _i32, _p, _f32,
+                                      _f32, _p, _p]),
+    "nt_moe_expert_wgrads": (_i32, [_p, _i64, _p, _i64, _p, _i64, _i64, _p, _i64, _p, _p, _i32,
+                                    _i64, _i32, _i32, _i32, _i32, _i32, _p, _sz, _i32, _p, _p,
+                                    _p]),
     "nt_moe_grouped_gemm_bf16_packed_shared": (_i32, [_p, _i64, _i64, _p, _p, _i32, _i64, _p, _i32,
                                                       _i32, _p, _p, _p, _i64, _i64, _p, _p, _i32,
                                                       _i32, _p, _p, _i32, _p]),

@@ -352,6 +352,84 @@ int nt_moe_grouped_wgrad_pair(const uint16_t* a0, int64_t lda0, const uint16_t* 
                   "grouped_wgrad_pair");
 }
 
+int nt_moe_expert_wgrads(const uint16_t* dfc1, int64_t ld_dfc1, const uint16_t* x, int64_t ld_x,
+                         const uint16_t* g, int64_t ld_g, int64_t token_rows, const uint16_t* wh,
+                         int64_t ld_wh, const int32_t* src_row, const int32_t* seg_offsets,
+                         int32_t num_segments, int64_t total_rows, int32_t F, int32_t d, int32_t H,
+                         int32_t splits1, int32_t splits2, float* partial, size_t partial_bytes,
+                         int32_t c_fp32, void* dw1, void* dw2, nt_moe_stream_t stream) {
+  NT_REQUIRE(src_row, "expert_wgrads: null buffer");
+  int rc = check_wgrad(dfc1, ld_dfc1, x, ld_x, token_rows, src_row, seg_offsets, num_segments,
+                       total_rows, F, d, dw1);
+  if (rc) return rc;
+  rc = check_wgrad(g, ld_g, wh, ld_wh, total_rows, nullptr, seg_offsets, num_segments, total_rows,
+                   d, H, dw2);
+  if (rc) return rc;
+  NT_REQUIRE(splits1 >= 1 && splits1 <= 256 && splits2 >= 1 && splits2 <= 256,
+             "expert_wgrads: splits must be in [1, 256]");
+  const size_t need1 = splits1 > 1 ? (size_t)splits1 * num_segments * F * d * sizeof(float) : 0;
+  const size_t need2 = splits2 > 1 ? (size_t)splits2 * num_segments * d * H * sizeof(float) : 0;
+  const size_t need = need1 > need2 ? need1 : need2;
+  if (need) {
+    NT_REQUIRE(partial && aligned16(partial), "expert_wgrads: null or unaligned partial");
+    if (partial_bytes < need)
+      return fail(NT_MOE_ENOSPC, "expert_wgrads: partial %zu < %zu bytes", partial_bytes, need);
+  }
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (splits1 == 1 && splits2 == 1)
+    return launched(launch_grouped_wgrad_pair(dfc1, ld_dfc1, x, ld_x, token_rows, src_row, F, d,
+                                              dw1, g, ld_g, wh, ld_wh, token_rows, src_row, d, H,
+                                              dw2, seg_offsets, num_segments, total_rows,
+                                              c_fp32 != 0, st, true),
+                    "expert_wgrads");
+  hipError_t err = launch_grouped_wgrad(dfc1, ld_dfc1, x, ld_x, token_rows, src_row, seg_offsets,
+                                        num_segments, total_rows, F, d, splits1, partial,
+                                        c_fp32 != 0, dw1, st);
+  if (err != hipSuccess) return launched(err, "expert_wgrads");
+  return launched(launch_grouped_wgrad(g, ld_g, wh, ld_wh, token_rows, src_row, seg_offsets,
+                                       num_segments, total_rows, d, H, splits2, partial,
+                                       c_fp32 != 0, dw2, st, true),
+                  "expert_wgrads");
+}
+
+int nt_moe_router_bwd_rows(const float* logits, const int32_t* topk_ids, const float* topk_w,
+                           const float* grad_row_w, const int32_t* combine_dest,
+                           const int32_t* counts, int64_t T, int32_t E, int32_t k,
+                           int32_t score_fn, const float* grad_aux, float aux_coeff,
+                           float z_coeff, float* grad_logits, nt_moe_stream_t stream) {
+  int rc = check_route_shape(T, k, E);
+  if (rc) return rc;
+  NT_REQUIRE(score_fn == NT_MOE_SCORE_SOFTMAX || score_fn == NT_MOE_SCORE_SIGMOID,
+             "router_bwd_rows: unknown score_fn %d", score_fn);
+  if (T == 0) return ok();
+  NT_REQUIRE(logits && topk_ids && topk_w && grad_row_w && combine_dest && counts && grad_logits,
+             "router_bwd_rows: null buffer");
+  return launched(launch_router_bwd(logits, topk_ids, topk_w, grad_row_w, counts, T, E, k,
+                                    score_fn, grad_aux, aux_coeff, z_coeff, grad_logits,
+                                    reinterpret_cast<hipStream_t>(stream), combine_dest),
+                  "router_bwd_rows");
+}
+
+int nt_moe_act_bwd_rows(const uint16_t* fc1, const uint16_t* h, const uint16_t* grad_h,
+                        const float* row_w, int64_t rows, int32_t H, int32_t activation,
+                        uint16_t* grad_fc1, uint16_t* weighted_h, float* grad_row_w,
+                        nt_moe_stream_t stream) {
+  NT_REQUIRE(rows >= 0 && H > 0 && H % 8 == 0,
+             "act_bwd_rows: H must be a positive multiple of 8, got %d", H);
+  NT_REQUIRE(activation == NT_MOE_ACT_SWIGLU || activation == NT_MOE_ACT_RELU2,
+             "act_bwd_rows: unknown activation %d", activation);
+  if (rows == 0) return ok();
+  NT_REQUIRE(fc1 && h && grad_h && row_w && grad_fc1 && weighted_h && grad_row_w,
+             "act_bwd_rows: null buffer");
+  NT_REQUIRE(aligned16(fc1) && aligned16(h) && aligned16(grad_h) && aligned16(grad_fc1) &&
+                 aligned16(weighted_h),
+             "act_bwd_rows: the bf16 buffers must be 16-byte aligned");
+  return launched(launch_act_bwd_rows(fc1, h, grad_h, row_w, rows, H, activation, grad_fc1,
+                                      weighted_h, grad_row_w,
+                                      reinterpret_cast<hipStream_t>(stream)),
+                  "act_bwd_rows");
+}
+
 int nt_moe_router_bwd(const float* logits, const int32_t* topk_ids, const float* topk_w,
                       const float* grad_w, const int32_t* counts, int64_t T, int32_t E,
                       int32_t k, int32_t score_fn, const float* grad_aux, float aux_coeff,

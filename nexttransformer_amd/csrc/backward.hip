@@ -5,8 +5,11 @@
 //   y_r = act(a_r W1_s^T) W2_s^T for each assignment row r (expert s, token t = src_row[r])
 //   out_t = shared_t + sum_j w_tj y_{dest_tj};  aux = lb + z from the full scores and counts
 // Given g = d loss / d out and the aux loss's gradient, this file provides
-//   combine_bwd:  dy_r = w_tj g_t (bf16, expert-major rows) and dw_tj = <g_t, y_r> (fp32)
-//   act_bwd:      d fc1 from d h and the fc1 pre-activations (SwiGLU or ReLU^2)
+//   act_bwd_rows: for the routed rows, d fc1, the routing-weight gradients and w_r h_r from
+//                 u_r = g_t W2_s (what ops.moe_backward uses)
+//   combine_bwd:  dy_r = w_tj g_t (bf16, expert-major rows) and dw_tj = <g_t, y_r> (fp32), for
+//                 callers that differentiate the combine alone
+//   act_bwd:      d fc1 from d h and the fc1 pre-activations (SwiGLU or ReLU^2): the shared expert
 //   router_bwd:   d logits from dw (the k-selected normalisation) plus the load-balance and
 //                 z-loss terms (MCore TopKRouter, megatron_moe.py:43-45)
 // The dgrad GEMMs run on the packed grouped GEMM with transposed packed weights, and the
@@ -139,6 +142,92 @@ __global__ __launch_bounds__(256) void act_bwd_kernel(const uint16_t* __restrict
   }
 }
 
+// The activation backward of the routed rows from the unscaled hidden gradient u_r = g_t W2
+// (t = src_row[r], g_t the output's gradient before the routing weight), one wave per row:
+//   dw_r   = <h_r, u_r>                       (= <g_t, y_r>, fp32)
+//   dfc1_r = act'(fc1_r) * (w_r u_r)          (bf16)
+//   wh_r   = w_r h_r                          (bf16: dW2 = sum_r g_t^T wh_r)
+// so the backward needs no [rows, d] copy of w_r g_t and no second read of y: at d = 1280 and
+// H = 320 the rows move 5 H bf16 instead of 3 d for that copy and 3 H for the activation alone
+// (combine_bwd + act_bwd 137 + 40 us at 131072 rows, this kernel 70 = 6.0 TB/s; d 1024, H 512
+// SwiGLU, 65536 rows 52 + 56 -> 88 = 5.3 TB/s). Bound by HBM. Rows go two per wave and turn: their
+// loads overlap. Training steps 1069 -> 1040 us (32 experts) and 2315 -> 2187 us (T3 cell, where
+// the gathered down dgrad also splits its partial N tile: 192 -> 162 us).
+template <int ACT>
+__global__ __launch_bounds__(256) void act_bwd_rows_kernel(
+    const uint16_t* __restrict__ fc1, const uint16_t* __restrict__ h, const uint16_t* __restrict__ u,
+    const float* __restrict__ row_w, int64_t rows, int H, uint16_t* __restrict__ dfc1,
+    uint16_t* __restrict__ wh, float* __restrict__ dw) {
+  constexpr bool SW = ACT == NT_MOE_ACT_SWIGLU;
+  constexpr int R = 2;
+  const int lane = lane_id(), vecs = H >> 3;
+  const int F = SW ? 2 * H : H;
+  const int64_t step = (int64_t)gridDim.x * 4 * R;
+  for (int64_t r0 = ((int64_t)blockIdx.x * 4 + wave_id()) * R; r0 < rows; r0 += step) {
+    float dot[R] = {};
+    for (int v0 = 0; v0 < vecs; v0 += 64) {
+      const int v = v0 + lane;
+      u32x4 uv[R], hv[R], fv[R], gv[R];
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const int64_t r = r0 + q < rows ? r0 + q : rows - 1;
+        const int64_t at = r * vecs + (v < vecs ? v : 0), fat = r * (F >> 3) + (v < vecs ? v : 0);
+        uv[q] = reinterpret_cast<const u32x4*>(u)[at];
+        hv[q] = reinterpret_cast<const u32x4*>(h)[at];
+        fv[q] = reinterpret_cast<const u32x4*>(fc1)[fat];
+        if (SW) gv[q] = reinterpret_cast<const u32x4*>(fc1)[fat + vecs];
+      }
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const int64_t r = r0 + q;
+        if (r >= rows) break;
+        const float w = row_w[r];
+        u32x4 df, dg, ow;
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float a[2], b[2], uu[2], hh[2], of[2], og[2];
+#pragma unroll
+          for (int x = 0; x < 2; ++x) {
+            auto at = [&](const u32x4& p) {
+              return x ? __builtin_bit_cast(float, p[i] & 0xffff0000u)
+                       : bf16_bits_to_f32(p[i] & 0xffffu);
+            };
+            uu[x] = at(uv[q]);
+            hh[x] = at(hv[q]);
+            a[x] = at(fv[q]);
+            s = __builtin_fmaf(hh[x], uu[x], s);
+            const float d = w * uu[x];
+            if (SW) {
+              b[x] = at(gv[q]);
+              const float sg = sigmoidf_(a[x]);
+              of[x] = d * b[x] * sg * (1.f + a[x] * (1.f - sg));
+              og[x] = d * (a[x] * sg);
+            } else {
+              of[x] = d * 2.f * (a[x] > 0.f ? a[x] : 0.f);
+            }
+          }
+          df[i] = pack_bf16x2(of[0], of[1]);
+          if (SW) dg[i] = pack_bf16x2(og[0], og[1]);
+          ow[i] = pack_bf16x2(w * hh[0], w * hh[1]);
+        }
+        if (v < vecs) {
+          dot[q] += s;
+          reinterpret_cast<u32x4*>(dfc1)[r * (F >> 3) + v] = df;
+          if (SW) reinterpret_cast<u32x4*>(dfc1)[r * (F >> 3) + vecs + v] = dg;
+          reinterpret_cast<u32x4*>(wh)[r * vecs + v] = ow;
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+#pragma unroll
+      for (int m = 32; m >= 1; m >>= 1) dot[q] += __shfl_xor(dot[q], m);
+      if (lane == 0 && r0 + q < rows) dw[r0 + q] = dot[q];
+    }
+  }
+}
+
 // One wave per token; lane l holds experts l, l + 64, ... (E <= 256).
 //   selected (softmax over the k):     dl_j = w_j (dw_j - sum_i w_i dw_i)
 //   selected (sigmoid, normalised):    dl_j = s_j (1 - s_j) / S (dw_j - sum_i w_i dw_i)
@@ -149,10 +238,13 @@ __global__ __launch_bounds__(256) void act_bwd_kernel(const uint16_t* __restrict
 // with c_lb = aux_coeff E / (k T^2), c_z = z_coeff, and g_lb, g_z read from grad_aux (the
 // gradient of the forward's aux = {lb + z, lb, z}; NULL = no aux gradient).
 // PER = experts per lane (E <= 64 PER): the per-token work is sized by E, not by the largest E.
+// dw in top-k slot order [T, k], or with row_dest (combine_dest, the token's rows in ascending
+// expert order) one value per expert-major row.
 template <int PER>
 __global__ __launch_bounds__(256) void router_bwd_kernel(
     const float* __restrict__ logits, const int32_t* __restrict__ topk_ids,
     const float* __restrict__ topk_w, const float* __restrict__ dw,
+    const int32_t* __restrict__ row_dest,
     const int32_t* __restrict__ counts, int64_t T, int E, int k, int score_fn,
     const float* __restrict__ grad_aux, float aux_coeff, float z_coeff,
     float* __restrict__ dlogits) {
@@ -218,8 +310,21 @@ __global__ __launch_bounds__(256) void router_bwd_kernel(
       e = topk_ids[t * k + lane];
       if ((unsigned)e >= (unsigned)E) e = -1;
       wj = topk_w[t * k + lane];
-      dwj = dw[t * k + lane];
       lj = e >= 0 ? row[e] : 0.f;
+    }
+    if (row_dest) {  // slot j's row is the token's combine row #{i : ids_i < ids_j}
+      int pos = 0;
+      for (int j = 0; j < k; ++j) {
+        const int ej = __shfl(e, j);
+        pos += ej >= 0 && ej < e ? 1 : 0;
+      }
+      if (lane < k && e >= 0) {
+        const int64_t A = T * k;
+        const int r = row_dest[t * k + pos];
+        dwj = dw[r < 0 ? 0 : (r >= A ? A - 1 : r)];
+      }
+    } else if (lane < k) {
+      dwj = dw[t * k + lane];
     }
     float wdw = wj * dwj, ssel = lane < k && e >= 0 ? sigmoidf_(lj) : 0.f;
 #pragma unroll
@@ -340,10 +445,24 @@ hipError_t launch_act_bwd(const uint16_t* fc1, const uint16_t* dh, int64_t rows,
   return hipGetLastError();
 }
 
+hipError_t launch_act_bwd_rows(const uint16_t* fc1, const uint16_t* h, const uint16_t* u,
+                               const float* row_w, int64_t rows, int H, int activation,
+                               uint16_t* dfc1, uint16_t* wh, float* dw, hipStream_t stream) {
+  if (rows == 0) return hipSuccess;
+  int64_t blocks = (rows + 7) / 8;
+  const int64_t cap = (int64_t)num_cus() * 16;
+  if (blocks > cap) blocks = cap;
+  auto kern = activation == NT_MOE_ACT_SWIGLU ? act_bwd_rows_kernel<NT_MOE_ACT_SWIGLU>
+                                              : act_bwd_rows_kernel<NT_MOE_ACT_RELU2>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, stream, fc1, h, u, row_w, rows, H,
+                     dfc1, wh, dw);
+  return hipGetLastError();
+}
+
 hipError_t launch_router_bwd(const float* logits, const int32_t* topk_ids, const float* topk_w,
                              const float* dw, const int32_t* counts, int64_t T, int E, int k,
                              int score_fn, const float* grad_aux, float aux_coeff, float z_coeff,
-                             float* dlogits, hipStream_t stream) {
+                             float* dlogits, hipStream_t stream, const int32_t* row_dest) {
   if (T == 0) return hipSuccess;
   int64_t blocks = (T + 3) / 4;
   const int64_t cap = (int64_t)num_cus() * 32;
@@ -351,7 +470,7 @@ hipError_t launch_router_bwd(const float* logits, const int32_t* topk_ids, const
   auto kern = E <= 64 ? router_bwd_kernel<1>
                       : (E <= 128 ? router_bwd_kernel<2> : router_bwd_kernel<NT_MOE_MAX_EXPERTS / 64>);
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, stream, logits, topk_ids, topk_w,
-                     dw, counts, T, E, k, score_fn, grad_aux, aux_coeff, z_coeff, dlogits);
+                     dw, row_dest, counts, T, E, k, score_fn, grad_aux, aux_coeff, z_coeff, dlogits);
   return hipGetLastError();
 }
 

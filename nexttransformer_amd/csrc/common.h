@@ -108,11 +108,12 @@ hipError_t launch_grouped_gemm_bf16_packed_keep(const uint16_t* a, int64_t ld_a,
                                                 int64_t total_rows, const uint16_t* wp, int K,
                                                 int n_out, int epilogue, uint16_t* c,
                                                 uint16_t* pre, hipStream_t stream);
+// gather_a: b_src_row (of b_rows rows) gathers A's rows instead of B's.
 hipError_t launch_grouped_wgrad(const uint16_t* a, int64_t lda, const uint16_t* b, int64_t ldb,
                                 int64_t b_rows, const int32_t* b_src_row,
                                 const int32_t* seg_offsets, int num_segments, int64_t total_rows,
                                 int N, int M, int splits, float* partial, bool c_f32, void* c,
-                                hipStream_t stream);
+                                hipStream_t stream, bool gather_a = false);
 // Two products over the same segments without split K: one launch of the 256 x 256 kernel
 // when both take it, else one launch_grouped_wgrad after the other.
 hipError_t launch_grouped_wgrad_pair(const uint16_t* a0, int64_t lda0, const uint16_t* b0,
@@ -121,19 +122,24 @@ hipError_t launch_grouped_wgrad_pair(const uint16_t* a0, int64_t lda0, const uin
                                      const uint16_t* b1, int64_t ldb1, int64_t b_rows1,
                                      const int32_t* b_src_row1, int N1, int M1, void* c1,
                                      const int32_t* seg_offsets, int num_segments,
-                                     int64_t total_rows, bool c_f32, hipStream_t stream);
+                                     int64_t total_rows, bool c_f32, hipStream_t stream,
+                                     bool gather_a1 = false);
 hipError_t launch_combine_bwd(const uint16_t* g, int64_t ld_g, const uint16_t* y,
                               const int32_t* topk_ids, const int32_t* combine_dest,
                               const float* combine_w, int64_t T, int d, int k, uint16_t* dy,
                               float* dw, hipStream_t stream);
 hipError_t launch_act_bwd(const uint16_t* fc1, const uint16_t* dh, int64_t rows, int H,
                           int activation, uint16_t* dfc1, hipStream_t stream);
+hipError_t launch_act_bwd_rows(const uint16_t* fc1, const uint16_t* h, const uint16_t* u,
+                               const float* row_w, int64_t rows, int H, int activation,
+                               uint16_t* dfc1, uint16_t* wh, float* dw, hipStream_t stream);
 hipError_t launch_first_operand(const float* grad_logits, int E, const uint16_t* dfc1s, int Fs,
                                 int64_t T, int Ep, int Kc, uint16_t* out, hipStream_t stream);
 hipError_t launch_router_bwd(const float* logits, const int32_t* topk_ids, const float* topk_w,
                              const float* dw, const int32_t* counts, int64_t T, int E, int k,
                              int score_fn, const float* grad_aux, float aux_coeff, float z_coeff,
-                             float* dlogits, hipStream_t stream);
+                             float* dlogits, hipStream_t stream,
+                             const int32_t* row_dest = nullptr);
 hipError_t launch_route_plan(const uint16_t* x, int64_t ld_x, const int32_t* topk_ids,
                              const float* topk_w, int64_t T, int d, int k, int E, int32_t* counts,
                              int32_t* offsets, int32_t* ranks, int32_t* block_counts,

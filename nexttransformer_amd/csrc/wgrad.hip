@@ -47,7 +47,8 @@ __device__ __forceinline__ uint32_t hi_pair(uint32_t a, uint32_t b) {
 template <bool OUT_F32>
 __global__ __launch_bounds__(256) void grouped_wgrad_kernel(
     const uint16_t* __restrict__ a, int64_t lda, const uint16_t* __restrict__ b, int64_t ldb,
-    int64_t b_rows, const int32_t* __restrict__ b_src_row, const int32_t* __restrict__ seg_offsets,
+    int64_t b_rows, const int32_t* __restrict__ b_src_row, bool gather_a,
+    const int32_t* __restrict__ seg_offsets,
     int num_segments, int64_t total_rows, int N, int M, int splits, void* __restrict__ c) {
   __shared__ __align__(16) uint16_t lds[2][2][kWSlab];  // [buffer][operand A, B][col][row]
   const int ntn = (N + kWT - 1) / kWT, ntm = (M + kWT - 1) / kWT;
@@ -92,9 +93,9 @@ __global__ __launch_bounds__(256) void grouped_wgrad_kernel(
     const int col = (op == 0 ? n0 : m0) + 8 * cg, width = op == 0 ? N : M;
     const uint16_t* base = (op == 0 ? a : b) + (col < width ? col : width - 8);
     const int64_t ld = op == 0 ? lda : ldb;
-    // Gathered B rows: the row indices of a slab are loaded one slab ahead of its data (idx), so
+    // Gathered rows (B's, or A's with gather_a): the row indices of a slab are loaded one slab ahead of its data (idx), so
     // the data loads do not wait on an index load.
-    const bool gather = op == 1 && b_src_row != nullptr;
+    const bool gather = op == (gather_a ? 0 : 1) && b_src_row != nullptr;
     int32_t idx[8];
     auto load_idx = [&](int64_t r0) {
 #pragma unroll
@@ -241,7 +242,8 @@ struct TrGeo {
   static_assert(kCopiesA >= 1 && kCopiesB >= 1, "copies per wave");
 };
 
-template <int TN, int TM, bool GATHER, bool OUT_F32>
+// GATHER: 0 neither operand's rows gathered, 1 B's, 2 A's (through b_src_row, of b_rows rows).
+template <int TN, int TM, int GATHER, bool OUT_F32>
 __global__ __launch_bounds__(256, 2) void grouped_wgrad_tr_kernel(
     const uint16_t* __restrict__ a, int64_t lda, const uint16_t* __restrict__ b, int64_t ldb,
     int64_t b_rows, const int32_t* __restrict__ b_src_row, const int32_t* __restrict__ seg_offsets,
@@ -290,14 +292,15 @@ __global__ __launch_bounds__(256, 2) void grouped_wgrad_tr_kernel(
   const int rows = (int)(hi - lo);
   const int n_slabs = (rows + kTK - 1) / kTK;
   if (n_slabs > 0) {
-    // A: this tile's rows of the segment (a row past hi is out of range: zeros)
-    const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(a + lo * lda), 0, (int)((int64_t)rows * lda * 2), kBufWord3);
-    // B: the whole matrix (gathered rows) or this tile's rows; an explicit out-of-range offset
-    // for rows past hi
-    const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(GATHER ? b : b + lo * ldb), 0,
-        (int)(GATHER ? b_rows * ldb * 2 : (int64_t)rows * ldb * 2), kBufWord3);
+    // An operand's rows of the segment (a row past hi is out of range: zeros), or the whole
+    // matrix (gathered rows; an explicit out-of-range offset for rows past hi).
+    auto rsrc = [&](const uint16_t* p, int64_t ld, bool gathered) {
+      return __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(gathered ? p : p + lo * ld), 0,
+          (int)(gathered ? b_rows * ld * 2 : (int64_t)rows * ld * 2), kBufWord3);
+    };
+    const __amdgpu_buffer_rsrc_t ar = rsrc(a, lda, GATHER == 2);
+    const __amdgpu_buffer_rsrc_t br = rsrc(b, ldb, GATHER == 1);
     const __amdgpu_buffer_rsrc_t ir = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(GATHER ? b_src_row + lo : seg_offsets), 0, GATHER ? rows * 4 : 0, kBufWord3);
 
@@ -310,12 +313,12 @@ __global__ __launch_bounds__(256, 2) void grouped_wgrad_tr_kernel(
       const int col = col0 + 8 * cg;
       return col < width ? col : width - 8;
     };
-    int a_voff[G::kCopiesA], b_coloff[G::kCopiesB], b_row[G::kCopiesB];
+    int a_coloff[G::kCopiesA], a_row[G::kCopiesA], b_coloff[G::kCopiesB], b_row[G::kCopiesB];
 #pragma unroll
     for (int i = 0; i < G::kCopiesA; ++i) {
       constexpr int cpr = TN / 8, rpi = 64 / cpr;
-      const int row = (wave * G::kCopiesA + i) * rpi + lane / cpr;
-      a_voff[i] = row * (int)lda * 2 + chunk_col(row, cpr, n0, N) * 2;
+      a_row[i] = (wave * G::kCopiesA + i) * rpi + lane / cpr;
+      a_coloff[i] = chunk_col(a_row[i], cpr, n0, N) * 2;
     }
 #pragma unroll
     for (int i = 0; i < G::kCopiesB; ++i) {
@@ -335,23 +338,21 @@ __global__ __launch_bounds__(256, 2) void grouped_wgrad_tr_kernel(
     auto issue_copies = [&](int t) __attribute__((always_inline)) {
       unsigned char* st = smem + (t % kTRing) * G::kStage;
       const int r0 = t * kTK;
+      // byte offset of slab row `row` of an operand (rows past hi: out of range)
+      auto voff = [&](bool gathered, int row, int64_t ld, int coloff) {
+        if (!gathered) return row * (int)ld * 2 + coloff + r0 * (int)ld * 2;
+        int g = idx_ring[(t % kTIdx) * kTK + row];
+        g = g < 0 ? 0 : (g >= b_rows ? (int)b_rows - 1 : g);
+        return r0 + row < rows ? g * (int)ld * 2 + coloff : 0x7fffffff;
+      };
 #pragma unroll
       for (int i = 0; i < G::kCopiesA; ++i)
         buffer_to_lds16(ar, st + (wave * G::kCopiesA + i) * 1024,
-                          a_voff[i] + r0 * (int)lda * 2);
+                        voff(GATHER == 2, a_row[i], lda, a_coloff[i]));
 #pragma unroll
-      for (int i = 0; i < G::kCopiesB; ++i) {
-        const int r = r0 + b_row[i];
-        int voff;
-        if (GATHER) {
-          int g = idx_ring[(t % kTIdx) * kTK + b_row[i]];
-          g = g < 0 ? 0 : (g >= b_rows ? (int)b_rows - 1 : g);
-          voff = r < rows ? g * (int)ldb * 2 + b_coloff[i] : 0x7fffffff;
-        } else {
-          voff = r < rows ? r * (int)ldb * 2 + b_coloff[i] : 0x7fffffff;
-        }
-        buffer_to_lds16(br, st + G::kSlabA + (wave * G::kCopiesB + i) * 1024, voff);
-      }
+      for (int i = 0; i < G::kCopiesB; ++i)
+        buffer_to_lds16(br, st + G::kSlabA + (wave * G::kCopiesB + i) * 1024,
+                        voff(GATHER == 1, b_row[i], ldb, b_coloff[i]));
     };
     // Vector memory operations per slab and wave after its copies: the next slab's index load
     // and copies.
@@ -542,6 +543,7 @@ struct T2Product {
   void* c;
   int64_t lda, ldb, b_rows;
   int N, M, blocks;
+  bool gather_a;  // b_src_row (of b_rows rows) gathers A's rows instead of B's
 };
 struct T2Args {
   T2Product p[2];
@@ -577,6 +579,7 @@ __global__ __launch_bounds__(256, 1) void grouped_wgrad_t256_kernel(T2Args args)
   const int num_segments = args.num_segments, splits = args.splits;
   const int64_t total_rows = args.total_rows;
   const bool gather = b_src_row != nullptr;
+  const bool gather_a = second ? args.p[1].gather_a : args.p[0].gather_a;
   const int ntn = (N + TN - 1) / TN, ntm = (M + TM - 1) / TM;
   const int per_seg = ntn * ntm;
   const int split = blk / (num_segments * per_seg);
@@ -609,11 +612,20 @@ __global__ __launch_bounds__(256, 1) void grouped_wgrad_t256_kernel(T2Args args)
   const int rows = (int)(hi - lo);
   const int n_slabs = (rows + kTK - 1) / kTK;
   if (n_slabs > 0) {
+    // The copies take the operands as a linear and a (possibly) gathered one: A and B, or with
+    // gather_a B and A. Only their LDS places and columns differ, so one loop serves both.
+    const bool ga = gather && gather_a;
+    const uint16_t* lin = ga ? b : a;
+    const uint16_t* gat = ga ? a : b;
+    const int64_t ld_lin = ga ? ldb : lda, ld_gat = ga ? lda : ldb;
+    const int lin_dst = ga ? G::kSlab : 0, gat_dst = ga ? 0 : G::kSlab;
+    const int lin_col0 = ga ? m0 : n0, gat_col0 = ga ? n0 : m0;
+    const int lin_width = ga ? M : N, gat_width = ga ? N : M;
     const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(a + lo * lda), 0, (int)((int64_t)rows * lda * 2), kBufWord3);
+        (void*)(lin + lo * ld_lin), 0, (int)((int64_t)rows * ld_lin * 2), kBufWord3);
     const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(gather ? b : b + lo * ldb), 0,
-        (int)(gather ? b_rows * ldb * 2 : (int64_t)rows * ldb * 2), kBufWord3);
+        (void*)(gather ? gat : gat + lo * ld_gat), 0,
+        (int)(gather ? b_rows * ld_gat * 2 : (int64_t)rows * ld_gat * 2), kBufWord3);
     const __amdgpu_buffer_rsrc_t ir = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(gather ? b_src_row + lo : seg_offsets), 0, gather ? rows * 4 : 0, kBufWord3);
 
@@ -633,9 +645,9 @@ __global__ __launch_bounds__(256, 1) void grouped_wgrad_t256_kernel(T2Args args)
   #pragma unroll
       for (int i = 0; i < G::kCopies; ++i) {
         const int row = (wave * G::kCopies + i) * 2 + lane / 32;
-        a_voff[i] = row * (int)lda * 2 + chunk_col(row, n0, N) * 2;
+        a_voff[i] = row * (int)ld_lin * 2 + chunk_col(row, lin_col0, lin_width) * 2;
         b_row[i] = row;
-        b_coloff[i] = chunk_col(row, m0, M) * 2;
+        b_coloff[i] = chunk_col(row, gat_col0, gat_width) * 2;
       }
       // Index loads of slab t (GATHER): wave w loads rows 8 w .. 8 w + 7 with lanes 0-7.
       auto issue_idx = [&](int t) __attribute__((always_inline)) {
@@ -671,7 +683,7 @@ __global__ __launch_bounds__(256, 1) void grouped_wgrad_t256_kernel(T2Args args)
             const int g = gi[i];
             src = g < 0 ? 0 : (g >= b_rows ? (int)b_rows - 1 : g);
           }
-          bv[i] = r < rows ? src * (int)ldb * 2 + b_coloff[i] : 0x7fffffff;
+          bv[i] = r < rows ? src * (int)ld_gat * 2 + b_coloff[i] : 0x7fffffff;
         }
       };
       // Item k of the group published with slab p: A copies, B copies, the index load of slab
@@ -685,11 +697,11 @@ __global__ __launch_bounds__(256, 1) void grouped_wgrad_t256_kernel(T2Args args)
         const int t = p + kT2Lead;
         unsigned char* st = smem + (t % kT2Ring) * G::kStage;
         if constexpr (k < G::kCopies) {
-          buffer_to_lds16(ar, st + (wave * G::kCopies + k) * 1024,
-                          a_voff[k] + t * kTK * (int)lda * 2);
+          buffer_to_lds16(ar, st + lin_dst + (wave * G::kCopies + k) * 1024,
+                          a_voff[k] + t * kTK * (int)ld_lin * 2);
         } else if constexpr (k < 2 * G::kCopies) {
           constexpr int i = k - G::kCopies;
-          buffer_to_lds16(br, st + G::kSlab + (wave * G::kCopies + i) * 1024, bv[i]);
+          buffer_to_lds16(br, st + gat_dst + (wave * G::kCopies + i) * 1024, bv[i]);
         } else {
           issue_idx(p + kT2ILead);
         }
@@ -910,7 +922,7 @@ bool wgrad_regs_override() {
   return v;
 }
 
-template <int TN, int TM, bool GATHER, bool OUT_F32>
+template <int TN, int TM, int GATHER, bool OUT_F32>
 hipError_t launch_tr(const uint16_t* a, int64_t lda, const uint16_t* b, int64_t ldb,
                      int64_t b_rows, const int32_t* b_src_row, const int32_t* seg_offsets,
                      int num_segments, int64_t total_rows, int N, int M, int splits, void* c,
@@ -939,9 +951,10 @@ hipError_t launch_t256(const T2Args& args, hipStream_t stream) {
 }
 
 T2Product t256_product(const uint16_t* a, int64_t lda, const uint16_t* b, int64_t ldb,
-                       int64_t b_rows, const int32_t* b_src_row, int num_segments, int N, int M,
-                       int splits, void* c) {
+                       int64_t b_rows, const int32_t* b_src_row, bool gather_a, int num_segments,
+                       int N, int M, int splits, void* c) {
   T2Product p;
+  p.gather_a = gather_a;
   p.a = a;
   p.b = b;
   p.b_src_row = b_src_row;
@@ -964,13 +977,14 @@ bool wgrad_t256(int N, int M, int splits) { return N % 256 == 0 && M % 256 == 0 
 // not split, else 128 x 256 when N <= M, else 256 x 128.
 template <bool OUT_F32>
 hipError_t launch_tr_any(const uint16_t* a, int64_t lda, const uint16_t* b, int64_t ldb,
-                         int64_t b_rows, const int32_t* b_src_row, const int32_t* seg_offsets,
-                         int num_segments, int64_t total_rows, int N, int M, int splits, void* c,
-                         hipStream_t stream) {
-  const bool g = b_src_row != nullptr;
+                         int64_t b_rows, const int32_t* b_src_row, bool gather_a,
+                         const int32_t* seg_offsets, int num_segments, int64_t total_rows, int N,
+                         int M, int splits, void* c, hipStream_t stream) {
+  const int g = b_src_row == nullptr ? 0 : (gather_a ? 2 : 1);
   if (wgrad_t256(N, M, splits)) {
     T2Args args;
-    args.p[0] = t256_product(a, lda, b, ldb, b_rows, b_src_row, num_segments, N, M, splits, c);
+    args.p[0] = t256_product(a, lda, b, ldb, b_rows, b_src_row, gather_a, num_segments, N, M,
+                             splits, c);
     args.p[1] = args.p[0];
     args.seg_offsets = seg_offsets;
     args.total_rows = total_rows;
@@ -983,10 +997,11 @@ hipError_t launch_tr_any(const uint16_t* a, int64_t lda, const uint16_t* b, int6
   return launch_tr<TN, TM, GG, OUT_F32>(a, lda, b, ldb, b_rows, b_src_row, seg_offsets,         \
                                         num_segments, total_rows, N, M, splits, c, stream);
   if (N <= M) {
-    if (g) { NT_TR(128, 256, true) } else { NT_TR(128, 256, false) }
-  } else {
-    if (g) { NT_TR(256, 128, true) } else { NT_TR(256, 128, false) }
+    if (g == 2) { NT_TR(128, 256, 2) } else if (g == 1) { NT_TR(128, 256, 1) }
+    NT_TR(128, 256, 0)
   }
+  if (g == 2) { NT_TR(256, 128, 2) } else if (g == 1) { NT_TR(256, 128, 1) }
+  NT_TR(256, 128, 0)
 #undef NT_TR
 }
 
@@ -996,20 +1011,22 @@ hipError_t launch_grouped_wgrad(const uint16_t* a, int64_t lda, const uint16_t* 
                                 int64_t b_rows, const int32_t* b_src_row,
                                 const int32_t* seg_offsets, int num_segments, int64_t total_rows,
                                 int N, int M, int splits, float* partial, bool c_f32, void* c,
-                                hipStream_t stream) {
+                                hipStream_t stream, bool gather_a) {
+  gather_a = gather_a && b_src_row;
   const int64_t tiles = (int64_t)num_segments * ((N + kWT - 1) / kWT) * ((M + kWT - 1) / kWT);
   if (tiles == 0) return hipSuccess;
   // The transposing-read kernel addresses its operands through 32-bit buffer offsets.
   const int64_t lim = (int64_t)1 << 31;
-  if (!wgrad_regs_override() && total_rows * lda * 2 < lim &&
-      (b_src_row ? b_rows : total_rows) * ldb * 2 < lim) {
+  const int64_t rows_a = gather_a ? b_rows : total_rows;
+  const int64_t rows_b = b_src_row && !gather_a ? b_rows : total_rows;
+  if (!wgrad_regs_override() && rows_a * lda * 2 < lim && rows_b * ldb * 2 < lim) {
     hipError_t err;
     if (splits <= 1)
-      return c_f32 ? launch_tr_any<true>(a, lda, b, ldb, b_rows, b_src_row, seg_offsets,
+      return c_f32 ? launch_tr_any<true>(a, lda, b, ldb, b_rows, b_src_row, gather_a, seg_offsets,
                                          num_segments, total_rows, N, M, 1, c, stream)
-                   : launch_tr_any<false>(a, lda, b, ldb, b_rows, b_src_row, seg_offsets,
+                   : launch_tr_any<false>(a, lda, b, ldb, b_rows, b_src_row, gather_a, seg_offsets,
                                           num_segments, total_rows, N, M, 1, c, stream);
-    err = launch_tr_any<true>(a, lda, b, ldb, b_rows, b_src_row, seg_offsets, num_segments,
+    err = launch_tr_any<true>(a, lda, b, ldb, b_rows, b_src_row, gather_a, seg_offsets, num_segments,
                               total_rows, N, M, splits, static_cast<void*>(partial), stream);
     if (err != hipSuccess) return err;
     const int64_t count = (int64_t)num_segments * N * M;
@@ -1021,11 +1038,11 @@ hipError_t launch_grouped_wgrad(const uint16_t* a, int64_t lda, const uint16_t* 
   if (splits <= 1) {
     auto kern = c_f32 ? grouped_wgrad_kernel<true> : grouped_wgrad_kernel<false>;
     hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(256), 0, stream, a, lda, b, ldb, b_rows,
-                       b_src_row, seg_offsets, num_segments, total_rows, N, M, 1, c);
+                       b_src_row, gather_a, seg_offsets, num_segments, total_rows, N, M, 1, c);
     return hipGetLastError();
   }
   hipLaunchKernelGGL(grouped_wgrad_kernel<true>, dim3((unsigned)(tiles * splits)), dim3(256), 0,
-                     stream, a, lda, b, ldb, b_rows, b_src_row, seg_offsets, num_segments,
+                     stream, a, lda, b, ldb, b_rows, b_src_row, gather_a, seg_offsets, num_segments,
                      total_rows, N, M, splits, static_cast<void*>(partial));
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
@@ -1042,20 +1059,25 @@ hipError_t launch_grouped_wgrad_pair(const uint16_t* a0, int64_t lda0, const uin
                                      const uint16_t* b1, int64_t ldb1, int64_t b_rows1,
                                      const int32_t* b_src_row1, int N1, int M1, void* c1,
                                      const int32_t* seg_offsets, int num_segments,
-                                     int64_t total_rows, bool c_f32, hipStream_t stream) {
+                                     int64_t total_rows, bool c_f32, hipStream_t stream,
+                                     bool gather_a1) {
   if (num_segments == 0) return hipSuccess;
+  gather_a1 = gather_a1 && b_src_row1;
   const int64_t lim = (int64_t)1 << 31;
-  auto fits = [&](int64_t lda, int64_t ldb, int64_t b_rows, const int32_t* src, int N, int M) {
-    return wgrad_t256(N, M, 1) && total_rows * lda * 2 < lim &&
-           (src ? b_rows : total_rows) * ldb * 2 < lim;
+  auto fits = [&](int64_t lda, int64_t ldb, int64_t b_rows, const int32_t* src, bool ga, int N,
+                  int M) {
+    return wgrad_t256(N, M, 1) && (ga ? b_rows : total_rows) * lda * 2 < lim &&
+           (src && !ga ? b_rows : total_rows) * ldb * 2 < lim;
   };
-  if (!wgrad_regs_override() && fits(lda0, ldb0, b_rows0, b_src_row0, N0, M0) &&
-      fits(lda1, ldb1, b_rows1, b_src_row1, N1, M1)) {
+  if (!wgrad_regs_override() && fits(lda0, ldb0, b_rows0, b_src_row0, false, N0, M0) &&
+      fits(lda1, ldb1, b_rows1, b_src_row1, gather_a1, N1, M1)) {
     // one launch over both tile lists: the second product's tiles start as CUs free up from the
     // first's, and the launch has one tail instead of two
     T2Args args;
-    args.p[0] = t256_product(a0, lda0, b0, ldb0, b_rows0, b_src_row0, num_segments, N0, M0, 1, c0);
-    args.p[1] = t256_product(a1, lda1, b1, ldb1, b_rows1, b_src_row1, num_segments, N1, M1, 1, c1);
+    args.p[0] = t256_product(a0, lda0, b0, ldb0, b_rows0, b_src_row0, false, num_segments, N0, M0,
+                             1, c0);
+    args.p[1] = t256_product(a1, lda1, b1, ldb1, b_rows1, b_src_row1, gather_a1, num_segments, N1,
+                             M1, 1, c1);
     args.seg_offsets = seg_offsets;
     args.total_rows = total_rows;
     args.num_segments = num_segments;
@@ -1068,7 +1090,7 @@ hipError_t launch_grouped_wgrad_pair(const uint16_t* a0, int64_t lda0, const uin
                                         stream);
   if (err != hipSuccess) return err;
   return launch_grouped_wgrad(a1, lda1, b1, ldb1, b_rows1, b_src_row1, seg_offsets, num_segments,
-                              total_rows, N1, M1, 1, nullptr, c_f32, c1, stream);
+                              total_rows, N1, M1, 1, nullptr, c_f32, c1, stream, gather_a1);
 }
 
 }  // namespace ntmoe

@@ -782,7 +782,7 @@ def moe_forward(x, w_router_t, w1, w2, *, top_k, score_fn=nat.SCORE_SOFTMAX,
     `mark(name)`, when given, is called after each stage is enqueued (used to place timing
     events on the stream; without permute_rows the router and the route plan are one call, so
     the "router" stage holds both and "route_plan" is empty). keep (bf16 experts): the state also holds what moe_backward reads
-    (h, y, the shared expert's h, the router's aux partials and the fc1 pre-activations of
+    (h, the shared expert's h; also y, the router's aux partials and the fc1 pre-activations of
     the routed and the shared expert from their up projections' launches, with packed weights
     or plain ones that plain_keep_supported takes; otherwise moe_backward recomputes them).
     """
@@ -1084,6 +1084,111 @@ def _(a0, b0, b_src_row0, a1, b1, b_src_row1, seg_offsets, total_rows, out_fp32=
             a0.new_empty(S, a1.shape[1], b1.shape[1], dtype=dt))
 
 
+@_custom_op("ntmoe::act_bwd_rows")
+def act_bwd_rows(fc1: Tensor, h: Tensor, grad_h: Tensor, row_w: Tensor,
+                 activation: int) -> tuple[Tensor, Tensor, Tensor]:
+    """(grad_fc1 [rows, F], weighted_h [rows, H] = row_w h, grad_row_w fp32 [rows] = <h, grad_h>)
+    from grad_h = the output gradient's rows times W2, before the routing weights row_w."""
+    _on_gpu(fc1, h, grad_h, row_w)
+    for t in (fc1, h, grad_h):
+        _require(t.dtype == torch.bfloat16 and t.dim() == 2 and t.is_contiguous(),
+                 "act_bwd_rows: fc1, h and grad_h must be contiguous bf16 matrices")
+    rows, H = grad_h.shape
+    F = 2 * H if activation == nat.ACT_SWIGLU else H
+    _require(fc1.shape == (rows, F) and h.shape == (rows, H),
+             "act_bwd_rows: fc1 must be [rows, 2H] (SwiGLU) or [rows, H], h [rows, H]")
+    _require(row_w.dtype == torch.float32 and row_w.shape == (rows,) and row_w.is_contiguous(),
+             "act_bwd_rows: row_w must be contiguous fp32 [rows]")
+    dfc1, wh = torch.empty_like(fc1), torch.empty_like(h)
+    dw = torch.empty(rows, device=h.device, dtype=torch.float32)
+    st = nat.load().nt_moe_act_bwd_rows(ptr(fc1), ptr(h), ptr(grad_h), ptr(row_w), rows, H,
+                                        activation, ptr(dfc1), ptr(wh), ptr(dw),
+                                        _stream(h.device))
+    nat.check(st, "ntmoe::act_bwd_rows")
+    return dfc1, wh, dw
+
+
+@act_bwd_rows.register_fake
+def _(fc1, h, grad_h, row_w, activation):
+    return torch.empty_like(fc1), torch.empty_like(h), torch.empty_like(row_w)
+
+
+@_custom_op("ntmoe::router_bwd_rows")
+def router_bwd_rows(logits: Tensor, ids: Tensor, weights: Tensor, grad_row_w: Tensor,
+                    combine_dest: Tensor, counts: Tensor, score_fn: int,
+                    grad_aux: Optional[Tensor], aux_coeff: float, z_coeff: float) -> Tensor:
+    """router_bwd with the routing-weight gradients per expert-major row (act_bwd_rows)."""
+    _on_gpu(logits, ids, weights, grad_row_w, combine_dest, counts, grad_aux)
+    T, E = logits.shape
+    k = ids.shape[1]
+    _require(logits.dtype == torch.float32 and logits.is_contiguous(),
+             "router_bwd_rows: logits must be contiguous fp32 [T, E]")
+    _require(ids.dtype == torch.int32 and ids.shape == (T, k) and ids.is_contiguous()
+             and combine_dest.dtype == torch.int32 and combine_dest.shape == (T, k)
+             and combine_dest.is_contiguous() and weights.dtype == torch.float32
+             and weights.shape == (T, k) and weights.is_contiguous()
+             and grad_row_w.dtype == torch.float32 and grad_row_w.shape == (T * k,)
+             and grad_row_w.is_contiguous(),
+             "router_bwd_rows: bad ids / weights / grad_row_w / combine_dest")
+    _require(counts.dtype == torch.int32 and counts.shape == (E,), "router_bwd_rows: bad counts")
+    if grad_aux is not None:
+        _require(grad_aux.dtype == torch.float32 and grad_aux.shape == (3,)
+                 and grad_aux.is_contiguous(), "router_bwd_rows: grad_aux must be fp32 [3]")
+    out = torch.empty_like(logits)
+    st = nat.load().nt_moe_router_bwd_rows(
+        ptr(logits), ptr(ids), ptr(weights), ptr(grad_row_w), ptr(combine_dest), ptr(counts), T, E,
+        k, score_fn, ptr(grad_aux), float(aux_coeff), float(z_coeff), ptr(out),
+        _stream(logits.device))
+    nat.check(st, "ntmoe::router_bwd_rows")
+    return out
+
+
+@router_bwd_rows.register_fake
+def _(logits, ids, weights, grad_row_w, combine_dest, counts, score_fn, grad_aux, aux_coeff,
+      z_coeff):
+    return torch.empty_like(logits)
+
+
+@_custom_op("ntmoe::expert_wgrads")
+def expert_wgrads(dfc1: Tensor, x: Tensor, g: Tensor, wh: Tensor, src_row: Tensor,
+                  seg_offsets: Tensor, splits1: int = 1, splits2: int = 1,
+                  out_fp32: bool = False) -> tuple[Tensor, Tensor]:
+    """(dW1 [S, F, d] = sum over each segment's rows r of dfc1[r]^T x[src_row[r]], dW2 [S, d, H]
+    = sum of g[src_row[r]]^T wh[r]), bf16 or fp32; splits as grouped_wgrad."""
+    _on_gpu(dfc1, x, g, wh, src_row, seg_offsets)
+    for t in (dfc1, x, g, wh):
+        _require(t.dtype == torch.bfloat16 and t.dim() == 2 and t.stride(1) == 1,
+                 "expert_wgrads: operands must be bf16 matrices with contiguous rows")
+    _require(seg_offsets.dtype == torch.int32 and seg_offsets.dim() == 1
+             and seg_offsets.is_contiguous(), "expert_wgrads: seg_offsets must be int32 [S+1]")
+    rows, F = dfc1.shape
+    T, d = x.shape
+    H = wh.shape[1]
+    _require(g.shape == (T, d) and wh.shape[0] == rows, "expert_wgrads: g must be [T, d] like x, "
+             "wh [rows, H]")
+    _require(src_row.dtype == torch.int32 and src_row.shape == (rows,) and src_row.is_contiguous(),
+             "expert_wgrads: src_row must be contiguous int32 [rows]")
+    S = seg_offsets.shape[0] - 1
+    dt = torch.float32 if out_fp32 else torch.bfloat16
+    dw1 = torch.empty(S, F, d, device=x.device, dtype=dt)
+    dw2 = torch.empty(S, d, H, device=x.device, dtype=dt)
+    need = max(splits1 * F if splits1 > 1 else 0, splits2 * H if splits2 > 1 else 0) * S * d
+    partial = torch.empty(need, device=x.device, dtype=torch.float32) if need else None
+    st = nat.load().nt_moe_expert_wgrads(
+        ptr(dfc1), dfc1.stride(0), ptr(x), x.stride(0), ptr(g), g.stride(0), T, ptr(wh),
+        wh.stride(0), ptr(src_row), ptr(seg_offsets), S, rows, F, d, H, splits1, splits2,
+        ptr(partial), 4 * need, int(out_fp32), ptr(dw1), ptr(dw2), _stream(x.device))
+    nat.check(st, "ntmoe::expert_wgrads")
+    return dw1, dw2
+
+
+@expert_wgrads.register_fake
+def _(dfc1, x, g, wh, src_row, seg_offsets, splits1=1, splits2=1, out_fp32=False):
+    S, d = seg_offsets.shape[0] - 1, x.shape[1]
+    dt = torch.float32 if out_fp32 else torch.bfloat16
+    return (x.new_empty(S, dfc1.shape[1], d, dtype=dt), x.new_empty(S, d, wh.shape[1], dtype=dt))
+
+
 _CU_COUNT = {}
 
 
@@ -1255,13 +1360,14 @@ def moe_backward(grad_out, grad_aux, x, w_router_t, bw, state, *, top_k,
     multiples of 64.
 
     All on this library's kernels: the fc1 recompute (when the forward kept no pre-activations),
-    the dgrad of both projections (grouped GEMMs), the combine transpose and routing-weight
-    gradient, the activation backward, the router backward (routing-weight, load-balance and
+    the dgrad of both projections (grouped GEMMs; the down projection's on the output gradient's
+    gathered rows, before the routing weight), the activation backward with the routing weight and
+    its gradient (act_bwd_rows), the router backward (routing-weight, load-balance and
     z-loss terms), the token-side sum of the k input-gradient rows (the forward's combine kernel
     with unit weights; its first row, the shared expert's input gradient plus the router's,
     grad_logits . Wr, comes from one grouped GEMM over the concatenated K of BackwardWeights'
-    `first` operand), and every weight gradient on grouped_wgrad: dy^T h and d_fc1^T x over each
-    expert's rows (x gathered through src_row), the shared expert's over all T rows and the
+    `first` operand), and every weight gradient on the grouped_wgrad kernels: g^T (w h) and d_fc1^T x over each
+    expert's rows (g and x gathered through src_row), the shared expert's over all T rows and the
     router's grad_logits^T x (fp32 output over the two-term bf16 split of grad_logits, which
     carries g to about 2^-17 |g|; the router gradients are checked against fp64), the last
     two split along T in fixed order. `mark(name)` as in moe_forward.
@@ -1285,11 +1391,12 @@ def moe_backward(grad_out, grad_aux, x, w_router_t, bw, state, *, top_k,
     if fc1 is None:  # not kept by the forward: recompute the pre-activations
         fc1 = bw.w1(x, src, offsets, A)
     mark("fc1_recompute")
-    gy, gw = combine_bwd.raw(g, state["y"], ids, cdest, state["combine_w"])
-    mark("combine_bwd")
-    dh = bw.w2t(gy, None, offsets, A)
+    # u_r = g_t W2 (the rows gathered by the GEMM), before the routing weight: the activation
+    # backward then applies it, so no [A, d] rows of w_r g_t are written and y is not read again
+    h = state["h"]
+    u = bw.w2t(g, src, offsets, A)
     mark("dgrad_down")
-    dfc1 = act_bwd.raw(fc1, dh, activation)
+    dfc1, wh, gw = act_bwd_rows.raw(fc1, h, u, state["perm_w"], activation)
     mark("act_bwd")
     dxp = bw.w1t(dfc1, None, offsets, A)
     mark("dgrad_up")
@@ -1304,8 +1411,8 @@ def moe_backward(grad_out, grad_aux, x, w_router_t, bw, state, *, top_k,
         dhs = sb["w2t"](g, None, seg, T)
         dfc1s = act_bwd.raw(fc1s, dhs, activation)
         mark("shared")
-    dlogits = router_bwd.raw(state["logits"], ids, state["weights"], gw, state["counts"], score_fn,
-                         grad_aux, aux_coeff, z_coeff)
+    dlogits = router_bwd_rows.raw(state["logits"], ids, state["weights"], gw, cdest,
+                                  state["counts"], score_fn, grad_aux, aux_coeff, z_coeff)
     # the token-side first row: [dfc1s | g_hi | g_hi | g_lo] . [W1s^T | Wr_hi | Wr_lo | Wr_hi]^T
     wf, (Fs, Ep, Kc) = bw.first(w_router_t)
     a_cat = backward_first_operand.raw(dlogits, dfc1s, Ep, Kc)
@@ -1322,14 +1429,9 @@ def moe_backward(grad_out, grad_aux, x, w_router_t, bw, state, *, top_k,
     mark("dx_sum")
     # expert weight gradients over each expert's rows; the shared expert's over all T rows
     f32 = weight_grads_fp32
-    h = state["h"]
-    s1 = wgrad_splits(E, dfc1.shape[1], d, A // E, x.device)
-    s2 = wgrad_splits(E, d, h.shape[1], A // E, x.device)
-    if s1 == 1 and s2 == 1:  # both in one call (one launch where both take the 256-wide tiles)
-        res["w1"], res["w2"] = grouped_wgrad_pair.raw(dfc1, x, src, gy, h, None, offsets, A, f32)
-    else:
-        res["w1"] = grouped_wgrad.raw(dfc1, x, src, offsets, A, s1, f32)
-        res["w2"] = grouped_wgrad.raw(gy, h, None, offsets, A, s2, f32)
+    res["w1"], res["w2"] = expert_wgrads.raw(
+        dfc1, x, g, wh, src, offsets, wgrad_splits(E, dfc1.shape[1], d, A // E, x.device),
+        wgrad_splits(E, d, h.shape[1], A // E, x.device), f32)
     if sh:
         res["shared_w1"] = grouped_wgrad.raw(dfc1s, x, None, seg, T,
                                          wgrad_splits(1, dfc1s.shape[1], d, T, x.device), f32)

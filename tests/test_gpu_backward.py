@@ -583,3 +583,69 @@ def test_grouped_wgrad_pair_equals_two_calls(N0, M0, N1, M1):
                                    rtol=1e-2, atol=1e-2)
         torch.testing.assert_close(c1[s].double().cpu(), ref1.to(torch.bfloat16).double(),
                                    rtol=1e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 130, 8200])
+@pytest.mark.parametrize("H", [8, 64, 320, 512, 520, 1536])
+@pytest.mark.parametrize("activation", [0, 1], ids=["swiglu", "relu2"])
+def test_act_bwd_rows(rows, H, activation):
+    """Against float64: grad_fc1 within two bf16 ulps (fp32 arithmetic, one rounding), weighted_h
+    bit-exact, the dot within its fp32 summation bound; one, two and odd row counts, more rows
+    than the grid holds at once, widths below, at and past one pass of a wave."""
+    from nexttransformer_amd import ops
+    g = torch.Generator().manual_seed(rows + H)
+    F = 2 * H if activation == 0 else H
+    mk = lambda *s: torch.randn(s, generator=g).to(torch.bfloat16)
+    fc1, h, u, w = mk(rows, F), mk(rows, H), mk(rows, H), torch.rand(rows, generator=g)
+    dfc1, wh, dw = (t.cpu() for t in ops.act_bwd_rows(fc1.cuda(), h.cuda(), u.cuda(), w.cuda(),
+                                                      activation))
+    d = w[:, None].double() * u.double()
+    if activation == 0:
+        a, b = fc1.double().chunk(2, -1)
+        s = torch.sigmoid(a)
+        ref = torch.cat([d * b * s * (1 + a * (1 - s)), d * a * s], -1)
+    else:
+        ref = d * 2 * torch.relu(fc1.double())
+    # (1 + a (1 - s) cancels near its root: an absolute term of fp32 size there)
+    assert ((dfc1.double() - ref).abs() <= 2 ** -7 * ref.abs() + 1e-5).all()
+    assert torch.equal(wh, (w[:, None] * h.float()).to(torch.bfloat16))
+    terms = h.double() * u.double()
+    bound = (H + 1) * 2.0 ** -24 * terms.abs().sum(-1)
+    assert ((dw.double() - terms.sum(-1)).abs() <= bound).all()
+
+
+# tiles of every kernel: 128 x 256 and 256 x 128 (the gather on either side), 256 x 256 in pairs,
+# a partial tile, split K; segments empty, of one row, ending at and past a 32-row slab
+@pytest.mark.parametrize("F,d,H,splits", [(64, 64, 64, 1), (320, 1280, 320, 1), (512, 256, 256, 1),
+                                          (1024, 512, 512, 1), (128, 192, 448, 3), (256, 128, 64, 2)])
+@pytest.mark.parametrize("fp32", [False, True])
+def test_expert_wgrads_equal_grouped_wgrad_on_gathered_rows(F, d, H, splits, fp32):
+    from nexttransformer_amd import ops
+    g = torch.Generator().manual_seed(F + H)
+    counts = [0, 1, 31, 32, 33, 0, 200, 97]
+    rows, T = sum(counts), 150
+    off = torch.tensor([0] + counts).cumsum(0).to(torch.int32).cuda()
+    mk = lambda *s: torch.randn(s, generator=g).to(torch.bfloat16).cuda()
+    dfc1, x, go, wh = mk(rows, F), mk(T, d), mk(T, d), mk(rows, H)
+    src = torch.randint(0, T, (rows,), generator=g, dtype=torch.int32).cuda()
+    w1, w2 = ops.expert_wgrads(dfc1, x, go, wh, src, off, splits, splits, fp32)
+    idx = src.long()
+    assert torch.equal(w1, ops.grouped_wgrad(dfc1, x[idx], None, off, rows, splits, fp32))
+    assert torch.equal(w2, ops.grouped_wgrad(go[idx], wh, None, off, rows, splits, fp32))
+
+
+@pytest.mark.parametrize("T,E,k", [(1, 2, 1), (65, 8, 2), (130, 100, 5), (300, 256, 8)])
+@pytest.mark.parametrize("score_fn", [0, 1], ids=["softmax", "sigmoid"])
+def test_router_bwd_rows_equal_slot_order(T, E, k, score_fn):
+    """Bit for bit router_bwd, the routing-weight gradients given per expert-major row."""
+    from nexttransformer_amd import ops
+    g = torch.Generator().manual_seed(T)
+    logits = torch.randn(T, E, generator=g).cuda()
+    ids, w, _, _ = ops.topk_from_logits(logits, k, score_fn)
+    counts, _, _, _, dest, _, _ = ops.route_plan(ids, w, E, None, False)
+    rows = torch.randn(T * k, generator=g).cuda()
+    order = ids.argsort(1).argsort(1)  # a slot's place among the token's ascending experts
+    slots = rows[dest.long().gather(1, order)].contiguous()
+    aux = torch.tensor([0.5, 1.0, 2.0]).cuda()
+    got = ops.router_bwd_rows(logits, ids, w, rows, dest, counts, score_fn, aux, 0.01, 0.001)
+    assert torch.equal(got, ops.router_bwd(logits, ids, w, slots, counts, score_fn, aux, 0.01, 0.001))
