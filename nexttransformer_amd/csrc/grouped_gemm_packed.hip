@@ -123,15 +123,31 @@ struct Tile {
 
 // KEEP: also store the epilogue's input (the fc1 pre-activations: SwiGLU gate then value, 2 n_out
 // wide, or the ReLU^2 input, n_out wide) to Pre, for a backward pass.
+// SHARED: one more segment, the shared expert's, of the same K and n_out: rows 0 .. shared.rows - 1
+// of its own matrix (no gather), its own weights and outputs. Its tiles end the tile list, so its
+// rows (numbered from total_rows on in the tile walk) run beside the last experts' instead of in
+// launches of their own that leave CUs idle (T3 cell, 16384 tokens: up 162 + 34 us as two launches,
+// 180 as one, down 172 + 25 and 198; forward 631 -> 604 us with the launches' gaps; the d = 1792
+// cell at 3001 tokens: up 165 + 37 -> 162, down 110 + 15 -> 112, down dgrad 128 + 34 -> 124).
 // EDGE: shapes with an odd K-step count or a partial last N tile (the extra step, waves that
 // multiply nothing). Without it the kernel holds neither, so the common shapes' code stays small
 // enough for the instruction cache (both together double it).
-template <int EPI, bool GATHER, int WAVES, bool KEEP = false, bool EDGE = false>
+struct SharedSegment {
+  const uint16_t* a;
+  int64_t ld_a;
+  const uint16_t* w;
+  uint16_t* c;
+  uint16_t* pre;
+  int rows;
+};
+
+template <int EPI, bool GATHER, int WAVES, bool KEEP = false, bool EDGE = false,
+          bool SHARED = false>
 __global__ __launch_bounds__(WAVES * 64, 2) void grouped_gemm_packed_kernel(
     const uint16_t* __restrict__ A, int64_t ld_a, const int32_t* __restrict__ src_row,
     const int32_t* __restrict__ seg_offsets, int S, int total_rows, int64_t a_rows,
     const uint16_t* __restrict__ Wp, int K, int n_out, uint16_t* __restrict__ Cout,
-    uint16_t* __restrict__ Pre) {
+    uint16_t* __restrict__ Pre, SharedSegment shared) {
   using Gm = Geo<WAVES>;
   constexpr int kBM = Gm::kBM, kWaves = Gm::kWaves, kAQ = Gm::kAQ, kStage = Gm::kStage;
   constexpr int kWB = Gm::kWB, kNJ = Gm::kNJ, kIdxWaves = Gm::kIdxWaves;
@@ -140,8 +156,9 @@ __global__ __launch_bounds__(WAVES * 64, 2) void grouped_gemm_packed_kernel(
   unsigned char* xpose = smem + kSA * kStage + wave_id() * kXposeBytes;  // this wave's scratch
   int* src_tab = reinterpret_cast<int*>(smem + kSA * kStage + kWaves * kXposeBytes);  // [2][kBM]
   int* src_dummy = src_tab + 2 * kBM;                           // [kWaves][64] sink
-  int* tile_prefix = src_dummy + kWaves * 64;                   // [S+1]
-  int* seg_lo = tile_prefix + (S + 1);                          // [S+1]
+  const int S_all = SHARED ? S + 1 : S;                         // segments of the tile list
+  int* tile_prefix = src_dummy + kWaves * 64;                   // [S_all+1]
+  int* seg_lo = tile_prefix + (S_all + 1);                      // [S_all+1]
 
   const int lane = lane_id(), wave = wave_id();
   const int NB = (EPI == NT_MOE_EPI_SWIGLU ? 2 * n_out : n_out) / 32;  // packed 32-row blocks
@@ -184,10 +201,14 @@ __global__ __launch_bounds__(WAVES * 64, 2) void grouped_gemm_packed_kernel(
       run_max = __shfl(o, 63);
       run_tiles += __shfl(t, 63);
     }
+    if (SHARED && lane == 0) {
+      seg_lo[S + 1] = total_rows + shared.rows;
+      tile_prefix[S + 1] = tile_prefix[S] + (shared.rows + kBM - 1) / kBM * n_tiles;
+    }
   }
   __syncthreads();
 
-  const int total = __builtin_amdgcn_readfirstlane(tile_prefix[S]);
+  const int total = __builtin_amdgcn_readfirstlane(tile_prefix[S_all]);
   const int xcd = blockIdx.x % 8, local = blockIdx.x / 8, per_xcd = gridDim.x / 8;
   const int t_begin = (int)((int64_t)total * xcd / 8);
   const int t_end = (int)((int64_t)total * (xcd + 1) / 8);
@@ -207,9 +228,9 @@ __global__ __launch_bounds__(WAVES * 64, 2) void grouped_gemm_packed_kernel(
   // position. The segment is the last one whose tile prefix is <= tl: one ballot per 64 segments.
   auto locate_tl = [&](int tl, int half, Tile& t) {
     int cnt = 0;
-    for (int base = 0; base < S; base += 64) {
+    for (int base = 0; base < S_all; base += 64) {
       const int i = base + lane;
-      const bool le = i < S && tile_prefix[i] <= tl;
+      const bool le = i < S_all && tile_prefix[i] <= tl;
       cnt += __popcll(__ballot(le));
     }
     t.s = __builtin_amdgcn_readfirstlane(cnt - 1);
@@ -217,7 +238,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void grouped_gemm_packed_kernel(
     const int mt = lt / n_tiles;
     t.nt = lt - mt * n_tiles;
     t.seg_end = __builtin_amdgcn_readfirstlane(seg_lo[t.s + 1]);
-    t.m0 = __builtin_amdgcn_readfirstlane(seg_lo[t.s]) + mt * kBM;
+    const int seg_first = SHARED && t.s == S ? total_rows : seg_lo[t.s];
+    t.m0 = __builtin_amdgcn_readfirstlane(seg_first) + mt * kBM;
     if (half >= 0) {  // rows [m0, m0 + kBM/2) or [m0 + kBM/2, m0 + kBM) of the tile
       const int tile_end = t.seg_end < t.m0 + kBM ? t.seg_end : t.m0 + kBM;
       if (half) t.m0 += kBM / 2;
@@ -246,7 +268,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void grouped_gemm_packed_kernel(
 
   // Gather indices of tile t into table slot `slot`: the first kBM / 64 waves load 64 rows each,
   // straight to LDS; rows past the segment end repeat its last row (their results are dropped).
-  const char* abase = reinterpret_cast<const char*>(A);
+  const char* abase = reinterpret_cast<const char*>(A);  // (of the producer's tile)
+  auto is_shared = [&](const Tile& t) { return SHARED && t.s == S; };
   // Byte offsets of this lane's four A chunks (one per load instruction) for tile t.
   // Instruction q covers rows (wave kAQ + q) kRPI + [0, kRPI); a row's swizzle depends only on
   // q % 2 and the lane, so two per-lane values serve every instruction.
@@ -259,11 +282,17 @@ __global__ __launch_bounds__(WAVES * 64, 2) void grouped_gemm_packed_kernel(
     for (int q = 0; q < kAQ; ++q) {
       const int row = (wave * kAQ + q) * kRPI + lrow;
       int64_t r;
+      if (is_shared(t)) {  // in bounds: m0 and seg_end lie in [total_rows, total_rows + rows]
+        r = (t.m0 + row < t.seg_end ? t.m0 + row : t.seg_end - 1) - total_rows;
+        aoff[q] = (uint32_t)(r * shared.ld_a * 2) + aswz[q % 2];
+        continue;
+      }
       if (GATHER) r = src_tab[slot * kBM + row];
       else r = t.m0 + row < t.seg_end ? t.m0 + row : t.seg_end - 1;
       r = r < 0 ? 0 : (r >= a_rows ? a_rows - 1 : r);
       aoff[q] = (uint32_t)(r * ld_a * 2) + aswz[q % 2];
     }
+    if (SHARED) abase = reinterpret_cast<const char*>(is_shared(t) ? shared.a : A);
   };
   // This wave's packed weight blocks for tile t (clamped in a partial N tile): wave-uniform
   // addresses, to which each lane adds lane * 16 bytes.
@@ -274,7 +303,9 @@ __global__ __launch_bounds__(WAVES * 64, 2) void grouped_gemm_packed_kernel(
     for (int rb = 0; rb < kWB; ++rb) {
       int nb = t.nt * kTileBlocks + wv * kWB + rb;
       nb = nb < NB ? nb : NB - 1;
-      wb[rb] = Wp + ((int64_t)t.s * NB + nb) * (int64_t)nk * kBlockElems;
+      const uint16_t* seg_w =
+          is_shared(t) ? shared.w : Wp + (int64_t)t.s * NB * (int64_t)nk * kBlockElems;
+      wb[rb] = seg_w + (int64_t)nb * nk * kBlockElems;
     }
   };
   const uint32_t b_lane = lane * 16;
@@ -354,7 +385,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void grouped_gemm_packed_kernel(
 
   locate_static(0, pt);
   tq0 = pt;
-  if (GATHER && wave < kIdxWaves) {  // the first tile's gather indices, before anything else
+  if (GATHER && wave < kIdxWaves && !is_shared(pt)) {  // the first tile's gather indices first
     const int r = wave * 64 + lane;
     const int gr = pt.m0 + r < pt.seg_end ? pt.m0 + r : pt.seg_end - 1;
     __builtin_amdgcn_global_load_lds((gvoid*)(src_row + gr), (lvoid*)(src_tab + wave * 64), 4,
@@ -394,7 +425,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void grouped_gemm_packed_kernel(
       if (!real) total_steps = (p_idx + 1) * nks;
     }
     if (GATHER) {
-      const bool load_idx = real && wave < kIdxWaves;
+      const bool load_idx = real && wave < kIdxWaves && !is_shared(nx);
       const int r = (wave % kIdxWaves) * 64 + lane;
       const int gr = load_idx ? (nx.m0 + r < nx.seg_end ? nx.m0 + r : nx.seg_end - 1) : 0;
       int* dst = load_idx ? src_tab + (p_slot ^ 1) * kBM + wave * 64 : src_dummy + wave * 64;
@@ -410,12 +441,12 @@ __global__ __launch_bounds__(WAVES * 64, 2) void grouped_gemm_packed_kernel(
   for (int q = 0; q < 4; ++q)
     frag_off[q] = (lane & 31) * kRB + (swz(lane & 31, 4 * (lane >> 5) + q) << 4);
 
-  const __amdgpu_buffer_rsrc_t out_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      Cout, 0, (int)((int64_t)total_rows * n_out * 2), kBufferWord3);
   constexpr int kPreW = EPI == NT_MOE_EPI_SWIGLU ? 2 : 1;  // pre-activation width / n_out
-  __amdgpu_buffer_rsrc_t pre_rsrc = out_rsrc;
+  const __amdgpu_buffer_rsrc_t routed_out = __builtin_amdgcn_make_buffer_rsrc(
+      Cout, 0, (int)((int64_t)total_rows * n_out * 2), kBufferWord3);
+  __amdgpu_buffer_rsrc_t routed_pre = routed_out;
   if constexpr (KEEP)
-    pre_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+    routed_pre = __builtin_amdgcn_make_buffer_rsrc(
         Pre, 0, (int)((int64_t)total_rows * kPreW * n_out * 2), kBufferWord3);
 
   // ---- consumer ---------------------------------------------------------------------------
@@ -619,6 +650,18 @@ __global__ __launch_bounds__(WAVES * 64, 2) void grouped_gemm_packed_kernel(
     // wait counts stores, as they are older than every load a wait names); rows past the segment
     // or columns past n_out get an out-of-range offset and are dropped by the buffer range check.
     const int hbit = lane >> 5;
+    // output rows: m of the tile walk is row m - row0 of this segment's matrix
+    const bool sh = is_shared(ct);
+    const int row0 = sh ? total_rows : 0;
+    __amdgpu_buffer_rsrc_t out_rsrc = routed_out, pre_rsrc = routed_pre;
+    if constexpr (SHARED) {
+      const int c_rows = sh ? shared.rows : total_rows;
+      out_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+          sh ? shared.c : Cout, 0, (int)((int64_t)c_rows * n_out * 2), kBufferWord3);
+      if constexpr (KEEP)
+        pre_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            sh ? shared.pre : Pre, 0, (int)((int64_t)c_rows * kPreW * n_out * 2), kBufferWord3);
+    }
     if (wave_live) {
       constexpr bool SW = EPI == NT_MOE_EPI_SWIGLU;
       constexpr int CPR = kWB * (SW ? 2 : 4);  // 16-byte chunks per row of the wave's columns
@@ -661,7 +704,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void grouped_gemm_packed_kernel(
               const int nb = ct.nt * kTileBlocks + wv * kWB + rb;
               const int col = SW ? nb * 16 + 8 * hbit : nb * 32 + 16 * st + 8 * hbit;
               const bool ok = j_ok && m_lane < ct.seg_end && nb < NB && col < n_out;
-              const int64_t prow = (int64_t)m_lane * kPreW * n_out;
+              const int64_t prow = (int64_t)(m_lane - row0) * kPreW * n_out;
 #pragma unroll
               for (int h = 0; h < (SW ? 2 : 1); ++h) {
                 const int e0 = SW ? 8 * h : 8 * st;
@@ -694,7 +737,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void grouped_gemm_packed_kernel(
             const int m = ct.m0 + (jb + j) * 32 + pass * RPH + r;
             const int col = col0 + q * 8;
             const uint32_t voff = (j_ok && m < ct.seg_end && col < n_out)
-                                      ? (uint32_t)(((int64_t)m * n_out + col) * 2)
+                                      ? (uint32_t)(((int64_t)(m - row0) * n_out + col) * 2)
                                       : 0x80000000u;
             __builtin_amdgcn_raw_buffer_store_b128(val, out_rsrc, voff, 0, 0);
           }
@@ -734,24 +777,27 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(const uint16_t* __res
       *reinterpret_cast<const u32x4*>(w + (s * R + row) * (int64_t)K + k0);
 }
 
-template <int EPI, bool GATHER, int WAVES, bool KEEP = false, bool EDGE = false>
+template <int EPI, bool GATHER, int WAVES, bool KEEP = false, bool EDGE = false,
+          bool SHARED = false>
 hipError_t launch_packed(const uint16_t* a, int64_t ld_a, int64_t a_rows, const int32_t* src_row,
                          const int32_t* seg_offsets, int S, int64_t total_rows,
                          const uint16_t* wp, int K, int n_out, uint16_t* c, hipStream_t stream,
-                         uint16_t* pre = nullptr) {
+                         uint16_t* pre = nullptr, const SharedSegment& shared = SharedSegment{}) {
   using Gm = Geo<WAVES>;
   const int NB = (EPI == NT_MOE_EPI_SWIGLU ? 2 * n_out : n_out) / 32;
   const int64_t n_tiles = (NB + kTileBlocks - 1) / kTileBlocks;
-  const int64_t upper = ((total_rows + Gm::kBM - 1) / Gm::kBM + S) * n_tiles;
+  const int64_t upper = ((total_rows + Gm::kBM - 1) / Gm::kBM + S +
+                         (SHARED ? (shared.rows + Gm::kBM - 1) / Gm::kBM : 0)) * n_tiles;
   int64_t grid = (int64_t)num_cus() * Gm::kPerCU;
   if (upper < grid) grid = upper;
   grid = ((grid + 7) / 8) * 8;
-  const size_t lds = Gm::lds(S);
-  auto kern = grouped_gemm_packed_kernel<EPI, GATHER, WAVES, KEEP, EDGE>;
+  const size_t lds = Gm::lds(S + (SHARED ? 1 : 0));
+  auto kern = grouped_gemm_packed_kernel<EPI, GATHER, WAVES, KEEP, EDGE, SHARED>;
   hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
   if (err != hipSuccess) return err;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(Gm::kThreads), lds, stream, a, ld_a,
-                     src_row, seg_offsets, S, (int)total_rows, a_rows, wp, K, n_out, c, pre);
+                     src_row, seg_offsets, S, (int)total_rows, a_rows, wp, K, n_out, c, pre,
+                     shared);
   return hipGetLastError();
 }
 
@@ -884,10 +930,11 @@ hipError_t launch_grouped_gemm_bf16_packed_keep(const uint16_t* a, int64_t ld_a,
 }
 
 // The routed product and the shared expert's (one segment of shared_rows rows, no gather, the same
-// epilogue): one launch where the routed rows are few, else one after the other. Past 2048 shared
-// rows (top-1 and top-2 routing over many experts) also one after the other: the shared tiles
-// are then too much work for the kernel for few rows (d 2048, 3072 wide, 3001 rows alone 125 us
-// against 47) to hide under the routed weight stream.
+// epilogue): one launch of the kernel for few rows where the routed rows are few, one of the tiled
+// kernel where the two have the same shape, else one after the other. Past 2048 shared rows (top-1
+// and top-2 routing over many experts) the shared tiles are too much work for the kernel for few
+// rows (d 2048, 3072 wide, 3001 rows alone 125 us against 47) to hide under the routed weight
+// stream.
 hipError_t launch_grouped_gemm_bf16_packed_shared(const FewPart& routed, const int32_t* seg_offsets,
                                                   int num_segments, int64_t total_rows,
                                                   const FewPart& shared, int64_t shared_rows,
@@ -897,6 +944,39 @@ hipError_t launch_grouped_gemm_bf16_packed_shared(const FewPart& routed, const i
       few_rows(num_segments, total_rows, routed.K, routed.n_out, epilogue))
     return launch_grouped_gemm_bf16_few(routed, seg_offsets, num_segments, total_rows, &shared,
                                         shared_rows, epilogue, stream);
+  // equal shapes, and room for one more segment: the shared expert ends the tile list (the up
+  // projections are instantiated for gathered rows, as every caller has them)
+  const bool same = shared.K == routed.K && shared.n_out == routed.n_out &&
+                    (routed.src_row || epilogue == NT_MOE_EPI_NONE);
+  if (same && !use_pp() && total_rows > 0 && num_segments < NT_MOE_MAX_SEGMENTS &&
+      total_rows + shared_rows < ((int64_t)1 << 31)) {
+    const SharedSegment seg{shared.a, shared.ld_a, shared.w, shared.c, shared.pre,
+                            (int)shared_rows};
+    const bool edge = packed_edge(routed.K, routed.n_out, epilogue);
+    auto go = [&](auto epi_c, auto keep_c) {
+      constexpr int EPI = decltype(epi_c)::value;
+      constexpr bool KEEP = decltype(keep_c)::value;
+      auto run = [&](auto gather_c, auto edge_c) {
+        return launch_packed<EPI, decltype(gather_c)::value, 4, KEEP, decltype(edge_c)::value, true>(
+            routed.a, routed.ld_a, routed.a_rows, routed.src_row, seg_offsets, num_segments,
+            total_rows, routed.w, routed.K, routed.n_out, routed.c, stream, routed.pre, seg);
+      };
+      constexpr std::true_type yes{};
+      constexpr std::false_type no{};
+      if constexpr (EPI == NT_MOE_EPI_NONE)
+        if (!routed.src_row) return edge ? run(no, yes) : run(no, no);
+      return edge ? run(yes, yes) : run(yes, no);
+    };
+    constexpr std::integral_constant<int, NT_MOE_EPI_SWIGLU> swiglu{};
+    constexpr std::integral_constant<int, NT_MOE_EPI_RELU2> relu2{};
+    constexpr std::integral_constant<int, NT_MOE_EPI_NONE> none{};
+    const bool keep = routed.pre != nullptr;
+    if (epilogue == NT_MOE_EPI_SWIGLU)
+      return keep ? go(swiglu, std::true_type()) : go(swiglu, std::false_type());
+    if (epilogue == NT_MOE_EPI_RELU2)
+      return keep ? go(relu2, std::true_type()) : go(relu2, std::false_type());
+    return go(none, std::false_type());
+  }
   auto one = [&](const FewPart& p, const int32_t* offsets, int segments, int64_t rows) {
     return p.pre ? launch_grouped_gemm_bf16_packed_keep(p.a, p.ld_a, p.a_rows, p.src_row, offsets,
                                                         segments, rows, p.w, p.K, p.n_out,

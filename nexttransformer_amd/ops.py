@@ -1394,7 +1394,12 @@ def moe_backward(grad_out, grad_aux, x, w_router_t, bw, state, *, top_k,
     # u_r = g_t W2 (the rows gathered by the GEMM), before the routing weight: the activation
     # backward then applies it, so no [A, d] rows of w_r g_t are written and y is not read again
     h = state["h"]
-    u = bw.w2t(g, src, offsets, A)
+    dhs = None
+    if sh and bw.w2t.packed and bw.shared["w2t"].packed:  # one call for both
+        u, _, dhs, _ = grouped_gemm_packed_shared.raw(g, src, offsets, bw.w2t.w, nat.EPI_NONE, A, g,
+                                                      bw.shared["w2t"].w, False)
+    else:
+        u = bw.w2t(g, src, offsets, A)
     mark("dgrad_down")
     dfc1, wh, gw = act_bwd_rows.raw(fc1, h, u, state["perm_w"], activation)
     mark("act_bwd")
@@ -1408,7 +1413,8 @@ def moe_backward(grad_out, grad_aux, x, w_router_t, bw, state, *, top_k,
         fc1s = state.get("shared_fc1")
         if fc1s is None:  # not kept by the forward
             fc1s = bw.shared_w1_proj(x, None, seg, T)
-        dhs = sb["w2t"](g, None, seg, T)
+        if dhs is None:
+            dhs = sb["w2t"](g, None, seg, T)
         dfc1s = act_bwd.raw(fc1s, dhs, activation)
         mark("shared")
     dlogits = router_bwd_rows.raw(state["logits"], ids, state["weights"], gw, cdest,

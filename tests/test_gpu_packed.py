@@ -413,3 +413,41 @@ def test_few_rows_with_shared_expert_equal_the_tiled_kernel(counts, K, n_out, K_
     if keep:
         assert torch.equal(pre, ref_pre) and torch.equal(pres, ref_pres)
     assert torch.equal(ops.grouped_gemm_packed(a, src, off, pw, epilogue, rows), ref)
+
+
+# the shared expert as the tile list's last segment (same shape, more rows than the kernel for few
+# rows takes): full and partial N tiles, odd and even K-step counts, shared rows of one tile, at
+# and past a tile's 128 rows, more than the routed ones; empty and ragged routed segments; rows
+# past the last segment; one segment
+@pytest.mark.parametrize("counts,tail", [([300, 0, 129, 1, 513], 0), ([700], 0), ([200, 333], 70),
+                                         ([128] * 9, 0)], ids=str)
+@pytest.mark.parametrize("K,n_out", [(256, 256), (320, 320), (1280, 320), (512, 128)])
+@pytest.mark.parametrize("T", [1, 128, 130, 3000])
+@pytest.mark.parametrize("epilogue", [0, 1, 2], ids=["swiglu", "relu2", "none"])
+@pytest.mark.parametrize("gather", [False, True])
+def test_shared_segment_equals_two_products(counts, tail, K, n_out, T, epilogue, gather):
+    """Bit for bit the two products apart, outputs and kept pre-activations."""
+    from nexttransformer_amd import _native as nat
+    from nexttransformer_amd import ops
+    g = torch.Generator().manual_seed(K + T)
+    f = 2 if epilogue == nat.EPI_SWIGLU else 1
+    S, rows = len(counts), sum(counts) + tail
+    off = torch.tensor([0] + counts).cumsum(0).to(torch.int32).cuda()
+    mk = lambda *s: torch.randn(s, generator=g).to(torch.bfloat16).cuda()
+    a = mk(400 if gather else rows, K)
+    src = torch.randint(0, 400, (rows,), generator=g, dtype=torch.int32).cuda() if gather else None
+    xs, pw = mk(T, K), ops.pack_expert_weights(mk(S, f * n_out, K), epilogue)
+    pws = ops.pack_expert_weights(mk(1, f * n_out, K), epilogue)
+    seg = torch.tensor([0, T], dtype=torch.int32).cuda()
+    used = sum(counts)
+    for keep in ([False, True] if epilogue != nat.EPI_NONE else [False]):
+        c, pre, cs, pres = ops.grouped_gemm_packed_shared(a, src, off, pw, epilogue, rows, xs, pws,
+                                                          keep)
+        if keep:
+            ref, ref_pre = ops.grouped_gemm_packed_keep(a, src, off, pw, epilogue, rows)
+            ref_s, ref_pres = ops.grouped_gemm_packed_keep(xs, None, seg, pws, epilogue, T)
+            assert torch.equal(pre[:used], ref_pre[:used]) and torch.equal(pres, ref_pres)
+        else:
+            ref = ops.grouped_gemm_packed(a, src, off, pw, epilogue, rows)
+            ref_s = ops.grouped_gemm_packed(xs, None, seg, pws, epilogue, T)
+        assert torch.equal(c[:used], ref[:used]) and torch.equal(cs, ref_s)
