@@ -4,6 +4,7 @@ The library is built in-tree by `nexttransformer_amd.build` (or `__graft_entry__
 There is no fallback: if the library is missing, every op raises.
 """
 import ctypes
+import importlib.util
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libnt_moe.so"
@@ -116,6 +117,26 @@ def load():
         raise NativeLibraryMissing(f"{LIB_PATH}: ABI {lib.nt_moe_abi_version()} != {ABI_VERSION}")
     _LIB = lib
     return lib
+
+
+_HOST = None
+
+
+def host():
+    """The native host path, the module nt_moe_host (cached); NativeLibraryMissing without it."""
+    global _HOST
+    if _HOST is None:
+        load()
+        path = LIB_PATH.with_name("nt_moe_host.so")
+        if not path.exists():
+            raise NativeLibraryMissing(
+                f"{path} is missing: build it with `python -m nexttransformer_amd.build`")
+        import torch  # noqa: F401  (the module's symbols come from torch's libraries)
+        spec = importlib.util.spec_from_file_location("nt_moe_host", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _HOST = module
+    return _HOST
 
 
 def check(status, what):

@@ -1,4 +1,6 @@
-"""Compiles the gfx950 HIP kernels and the C-ABI shim into nexttransformer_amd/_lib/libnt_moe.so.
+"""Compiles the gfx950 HIP kernels and the C-ABI shim into nexttransformer_amd/_lib/libnt_moe.so, and
+the native host path (csrc/host.cpp, a Python module over torch's C++ API) into nt_moe_host.so
+beside it.
 
     python -m nexttransformer_amd.build [-v]
 
@@ -11,6 +13,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -18,6 +21,7 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 LIB = PKG / "_lib" / "libnt_moe.so"
+HOST = PKG / "_lib" / "nt_moe_host.so"
 ARCH = "gfx950"
 
 FLAGS = [
@@ -50,22 +54,52 @@ def _compile(src, verbose):
     return obj
 
 
-def build(verbose=False, jobs=None):
-    """Compile every kernel source and link libnt_moe.so; returns the library path."""
-    BUILD.mkdir(parents=True, exist_ok=True)
-    LIB.parent.mkdir(parents=True, exist_ok=True)
-    srcs = sources()
-    jobs = jobs or min(len(srcs), int(os.environ.get("MAX_JOBS", "8")))
-    with ThreadPoolExecutor(max_workers=jobs) as pool:
-        objs = list(pool.map(lambda s: _compile(s, verbose), srcs))
-    tmp = LIB.with_suffix(".so.tmp")
-    cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
+def _compile_host(verbose):
+    """csrc/host.cpp -> object (host code only, so the host compiler)."""
+    import torch
+    root = Path(torch.__file__).resolve().parent
+    obj = BUILD / "host.o"
+    cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{ROOT / 'include'}", f"-isystem{root / 'include'}",
+           f"-isystem{root / 'include' / 'torch' / 'csrc' / 'api' / 'include'}",
+           f"-isystem{sysconfig.get_paths()['include']}", "-c", str(CSRC / "host.cpp"), "-o", str(obj)]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"the host compiler failed for host.cpp:\n{proc.stderr}")
+    return obj, root / "lib"
+
+
+def _link(cmd, lib, verbose):
+    tmp = lib.with_suffix(".so.tmp")
+    cmd = [*cmd, "-o", str(tmp)]
     if verbose:
         print(" ".join(cmd), flush=True)
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stderr}")
-    os.replace(tmp, LIB)
+    os.replace(tmp, lib)
+
+
+def build(verbose=False, jobs=None):
+    """Compile every source and link libnt_moe.so and nt_moe_host.so; returns the former's path."""
+    BUILD.mkdir(parents=True, exist_ok=True)
+    LIB.parent.mkdir(parents=True, exist_ok=True)
+    srcs = sources()
+    jobs = jobs or min(len(srcs) + 1, int(os.environ.get("MAX_JOBS", "8")))
+    # the longest compilation first
+    srcs.sort(key=lambda p: p.stat().st_size, reverse=True)
+    srcs.sort(key=lambda p: p.stem != "grouped_gemm_packed")
+    with ThreadPoolExecutor(max_workers=jobs) as pool:
+        objs = pool.map(lambda s: _compile(s, verbose), srcs)
+        host, torch_lib = pool.submit(_compile_host, verbose).result()
+        objs = sorted(map(str, objs))
+    _link([hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs], LIB, verbose)
+    _link([shutil.which("g++") or "c++", "-shared", str(host), f"-L{torch_lib}", "-lc10",
+           "-ltorch_cpu", "-ltorch_python", "-ltorch", f"-L{LIB.parent}", f"-l:{LIB.name}",
+           "-Wl,-rpath,$ORIGIN"], HOST, verbose)
     return LIB
 
 

@@ -47,6 +47,7 @@ Weight caches: the bf16 / packed / fp8 operands are rebuilt when a master's addr
 counter changes. An update that does not bump the counter (a write through .data, or into the
 storage from outside PyTorch) must be followed by invalidate_weights().
 """
+import array
 import math
 
 import torch
@@ -239,6 +240,9 @@ class MoELayer(nn.Module):
     forward(hidden [..., d]) -> (out [..., d] in hidden's dtype, aux_loss fp32 scalar).
     """
 
+    _all_tables = None  # the parameter tables of every master, in the masters' order
+    _pool_bytes = None  # the pools' addresses and their slices' (_pool_slices)
+
     def __init__(self, recipe, layer_number: int, pg_collection=None, *, device=None,
                  aux_grad="inject", expert_grad="accumulate"):
         super().__init__()
@@ -337,6 +341,8 @@ class MoELayer(nn.Module):
         set (zero_grad with set_to_none), each takes its slice of `grad`; when every .grad is
         still its slice of one such stack (same storage, consecutive, contiguous), the new
         gradients are added to that stack in one pass; otherwise tensor by tensor."""
+        if nat.host().give_grads(params, grad):
+            return
         if all(p.grad is None for p in params):
             for p, v in zip(params, grad.unbind(0)):
                 if p.requires_grad:
@@ -384,11 +390,33 @@ class MoELayer(nn.Module):
             return [t["weight"] for t in router + shared]
         return [t["weight"] for t in router + pooled + shared]
 
+    def _pool_slices(self):
+        """The addresses of expert i's fc1 and fc2 weights on slice i of their pools (the masters'
+        order), as int64 bytes; made anew when a pool has moved."""
+        pools = (self._fc1_pool, self._fc2_pool)
+        b1, b2 = (p.data_ptr() for p in pools)
+        if self._pool_bytes is None or self._pool_bytes[0] != (b1, b2):
+            s1, s2 = (p.stride(0) * p.element_size() for p in pools)
+            self._pool_bytes = (b1, b2), array.array(
+                "q", [x for i in range(pools[0].shape[0])
+                      for x in (b1 + i * s1, b2 + i * s2)]).tobytes()
+        return self._pool_bytes[1]
+
     def _masters_key(self):
         """Identifies the current values of every master: the tensors' addresses and version
         counters. The pooled expert weights share their pool's version counter (an in-place
         update of any of them bumps it), so while they all sit on their pool slices one
         version stands for each pool."""
+        if self._all_tables is None:
+            self._masters()
+            self._all_tables = sum(self._param_tables, [])
+        found = nat.host().masters(self._all_tables) if self.router.weight.is_cuda else None
+        if found is not None:  # the addresses and versions as bytes, read natively
+            ptrs, versions = found
+            slices = self._pool_slices()
+            self._pools_placed = (ptrs[8:8 + len(slices)] == slices and self._fc1_pool.device
+                                  == self._all_tables[1]["weight"].device)
+            return ptrs, versions
         masters = self._masters()
         ptrs = tuple(p.data_ptr() for p in masters)
         pools = (self._fc1_pool, self._fc2_pool)
@@ -453,7 +481,6 @@ class MoELayer(nn.Module):
             out["shared_w2"] = fc2(g["shared_w2"], r.shared_expert_width)
         return out
 
-    @torch.no_grad()
     def packed_weights(self, keep_plain=False):
         """Device weights the kernels read, rebuilt only when a master tensor changed:
         router_t fp32 [dp, E]; w1 [E, rows, dp]; w2 [E, dp, Hp]; shared_w1/2 [1, ...];
@@ -470,123 +497,128 @@ class MoELayer(nn.Module):
         """
         key = self._masters_key()
         if key != self._pack_key or (keep_plain and "w1_plain" not in self._packed):
-            r = self.recipe
-            fp8 = r.expert_dtype == "fp8"
-            align = 128 if fp8 else 64
-            dp = _round_up(r.width, align)
-            gated = r.activation == "swiglu"
-            dtype = torch.float32 if fp8 else torch.bfloat16
-            # The packed-weight GEMM (fragment-ordered weights streamed into registers) for a
-            # projection when its K and width qualify for every expert kind (routed, shared) and
-            # the weights live on the GPU; fp8 always. (The T3 cell: both projections packed,
-            # the down projection's K = 320 on the kernel's odd K-step path.)
-            widths = [r.expert_width] + ([r.shared_expert_width] if self.shared_experts else [])
-            on_gpu = self.router.weight.is_cuda
-            # Training (keep_plain) rebuilds these after every update. Where the conversion
-            # pass writes the packed layout itself (bf16, no padding, on the GPU) packing costs
-            # nothing extra; elsewhere it is a second pass, worth it only for even K-step counts.
-            fused = (not fp8 and on_gpu and dp == r.width
-                     and all(_round_up(h, align) == h for h in widths))
-            extra_pass = keep_plain and not fused
-            pk_up = fp8 or (on_gpu and all(ops.prefers_packed(
-                dp, _round_up(h, align), nat.EPI_SWIGLU if gated else nat.EPI_RELU2,
-                repacked_each_step=extra_pass) for h in widths))
-            pk_down = fp8 or (on_gpu and all(
-                ops.prefers_packed(_round_up(h, align), dp, nat.EPI_NONE,
-                                   repacked_each_step=extra_pass) for h in widths))
-
-            def stack(experts, hidden, pools=(None, None), need_w1=False):
-                hp = _round_up(hidden, align)
-                if not fp8 and hp == hidden and dp == r.width and self.router.weight.is_cuda:
-                    # one pass over each fp32 master stack writes what the kernels read: the
-                    # packed or plain weights and, for the backward, the transposes (packed
-                    # when their dgrad projection takes the packed GEMM)
-                    up = nat.EPI_SWIGLU if gated else nat.EPI_RELU2
-                    rows1 = (2 if gated else 1) * hidden
-                    t1 = keep_plain and ops.prefers_packed(rows1, r.width, nat.EPI_NONE,
-                                                           repacked_each_step=False)
-                    t2 = keep_plain and ops.prefers_packed(r.width, hidden, nat.EPI_NONE,
-                                                           repacked_each_step=False)
-                    # the pools themselves when the key found every weight on its slice (no
-                    # per-expert attribute walk: at 256 experts that costs 0.4 ms of host time)
-                    placed = pools[0] is not None and self._pools_placed
-                    src1 = pools[0] if placed else _stacked(
-                        pools[0], [e.linear_fc1.weight for e in experts])
-                    src2 = pools[1] if placed else _stacked(
-                        pools[1], [e.linear_fc2.weight for e in experts])
-                    w1, w1t, w1p, w1tp = ops.convert_pack_expert_weights.raw(
-                        src1, up, not pk_up or need_w1, keep_plain and not t1, pk_up, t1)
-                    w2, w2t, w2p, w2tp = ops.convert_pack_expert_weights.raw(
-                        src2, nat.EPI_NONE, not pk_down, keep_plain and not t2, pk_down, t2)
-                    some = lambda t: t if t.numel() else None
-                    plain.append((some(w1), some(w2), some(w1t), some(w2t), some(w1tp),
-                                  some(w2tp)))
-                    return (w1p if pk_up else w1, None, w2p if pk_down else w2, None)
-                if hp == hidden and dp == r.width:
-                    w1 = torch.stack([e.linear_fc1.weight.detach() for e in experts]).to(dtype)
-                    w2 = torch.stack([e.linear_fc2.weight.detach() for e in experts]).to(dtype)
-                else:
-                    n = len(experts)
-                    dev = experts[0].linear_fc1.weight.device
-                    w1 = torch.zeros(n, (2 if gated else 1) * hp, dp, device=dev, dtype=dtype)
-                    w2 = torch.zeros(n, dp, hp, device=dev, dtype=dtype)
-                    for i, e in enumerate(experts):
-                        fc1 = e.linear_fc1.weight.detach()
-                        if gated:
-                            w1[i, :hidden, :r.width] = fc1[:hidden]
-                            w1[i, hp:hp + hidden, :r.width] = fc1[hidden:]
-                        else:
-                            w1[i, :hidden, :r.width] = fc1
-                        w2[i, :r.width, :hidden] = e.linear_fc2.weight.detach()
-                if not fp8:
-                    up = nat.EPI_SWIGLU if gated else nat.EPI_RELU2
-                    w1, w2 = w1.contiguous(), w2.contiguous()
-                    plain.append((w1, w2, None, None, None, None))
-                    return (ops.pack_expert_weights.raw(w1, up) if pk_up else w1, None,
-                            ops.pack_expert_weights.raw(w2, nat.EPI_NONE) if pk_down else w2, None)
-                w1q, w1s = ops.quantize_fp8_blockwise(w1.contiguous())
-                w2q, w2s = ops.quantize_fp8_blockwise(w2.contiguous())
-                up = nat.EPI_SWIGLU if gated else nat.EPI_RELU2
-                return (ops.pack_expert_weights_fp8(w1q, up), w1s,
-                        ops.pack_expert_weights_fp8(w2q, nat.EPI_NONE), w2s)
-
-            plain = []  # the bf16 [E, rows, cols] stacks before packing (for the backward)
-            packed = dict(shared_w1=None, shared_w2=None,
-                          shared_w1_scale=None, shared_w2_scale=None,
-                          packed=True if fp8 else (pk_up, pk_down))
-            (packed["w1"], packed["w1_scale"], packed["w2"],
-             packed["w2_scale"]) = stack(list(self.experts.local_experts), r.expert_width,
-                                         (self._fc1_pool, self._fc2_pool))
-            if self.shared_experts is not None:
-                (packed["shared_w1"], packed["shared_w1_scale"], packed["shared_w2"],
-                 packed["shared_w2_scale"]) = stack([self.shared_experts], r.shared_expert_width,
-                                                     need_w1=True)
-            if keep_plain and not fp8:
-                (packed["w1_plain"], packed["w2_plain"], packed["w1_t"], packed["w2_t"],
-                 packed["w1_t_packed"], packed["w2_t_packed"]) = plain[0]
-                (packed["shared_w1_plain"], packed["shared_w2_plain"], _, packed["shared_w2_t"],
-                 _, packed["shared_w2_t_packed"]) = plain[1] if len(plain) > 1 else (None,) * 6
-            # the router's operands after the expert conversions, whose GPU time then covers
-            # this host work: w_router_t and, for the backward, the first operand in one kernel
-            rw = self.router.weight.detach()
-            packed["first"] = None
-            if on_gpu:
-                want_first = keep_plain and not fp8
-                sw1 = packed.get("shared_w1_plain") if want_first else None
-                if rw.dtype != torch.float32 or rw.stride(1) != 1:
-                    rw = rw.float().contiguous()
-                packed["router_t"], first = ops.router_operands.raw(
-                    rw, dp, None if sw1 is None else sw1[0], want_first)
-                if want_first:
-                    packed["first"] = first
-            else:
-                router_t = torch.zeros(dp, r.routed_experts, device=rw.device,
-                                       dtype=torch.float32)
-                router_t[:r.width] = rw.t()
-                packed["router_t"] = router_t
-            self._packed = packed
+            with torch.no_grad():
+                self._rebuild_operands(keep_plain)
             self._pack_key = key
         return self._packed
+
+    def _rebuild_operands(self, keep_plain):
+        """packed_weights' operands from the masters' present values."""
+        r = self.recipe
+        fp8 = r.expert_dtype == "fp8"
+        align = 128 if fp8 else 64
+        dp = _round_up(r.width, align)
+        gated = r.activation == "swiglu"
+        dtype = torch.float32 if fp8 else torch.bfloat16
+        # The packed-weight GEMM (fragment-ordered weights streamed into registers) for a
+        # projection when its K and width qualify for every expert kind (routed, shared) and
+        # the weights live on the GPU; fp8 always. (The T3 cell: both projections packed,
+        # the down projection's K = 320 on the kernel's odd K-step path.)
+        widths = [r.expert_width] + ([r.shared_expert_width] if self.shared_experts else [])
+        on_gpu = self.router.weight.is_cuda
+        # Training (keep_plain) rebuilds these after every update. Where the conversion
+        # pass writes the packed layout itself (bf16, no padding, on the GPU) packing costs
+        # nothing extra; elsewhere it is a second pass, worth it only for even K-step counts.
+        fused = (not fp8 and on_gpu and dp == r.width
+                 and all(_round_up(h, align) == h for h in widths))
+        extra_pass = keep_plain and not fused
+        pk_up = fp8 or (on_gpu and all(ops.prefers_packed(
+            dp, _round_up(h, align), nat.EPI_SWIGLU if gated else nat.EPI_RELU2,
+            repacked_each_step=extra_pass) for h in widths))
+        pk_down = fp8 or (on_gpu and all(
+            ops.prefers_packed(_round_up(h, align), dp, nat.EPI_NONE,
+                               repacked_each_step=extra_pass) for h in widths))
+
+        def stack(experts, hidden, pools=(None, None), need_w1=False):
+            hp = _round_up(hidden, align)
+            if not fp8 and hp == hidden and dp == r.width and self.router.weight.is_cuda:
+                # one pass over each fp32 master stack writes what the kernels read: the
+                # packed or plain weights and, for the backward, the transposes (packed
+                # when their dgrad projection takes the packed GEMM)
+                up = nat.EPI_SWIGLU if gated else nat.EPI_RELU2
+                rows1 = (2 if gated else 1) * hidden
+                t1 = keep_plain and ops.prefers_packed(rows1, r.width, nat.EPI_NONE,
+                                                       repacked_each_step=False)
+                t2 = keep_plain and ops.prefers_packed(r.width, hidden, nat.EPI_NONE,
+                                                       repacked_each_step=False)
+                # the pools themselves when the key found every weight on its slice (no
+                # per-expert attribute walk: at 256 experts that costs 0.4 ms of host time)
+                placed = pools[0] is not None and self._pools_placed
+                src1 = pools[0] if placed else _stacked(
+                    pools[0], [e.linear_fc1.weight for e in experts])
+                src2 = pools[1] if placed else _stacked(
+                    pools[1], [e.linear_fc2.weight for e in experts])
+                w1, w1t, w1p, w1tp = ops.convert_pack_expert_weights.raw(
+                    src1, up, not pk_up or need_w1, keep_plain and not t1, pk_up, t1)
+                w2, w2t, w2p, w2tp = ops.convert_pack_expert_weights.raw(
+                    src2, nat.EPI_NONE, not pk_down, keep_plain and not t2, pk_down, t2)
+                some = lambda t: t if t.numel() else None
+                plain.append((some(w1), some(w2), some(w1t), some(w2t), some(w1tp),
+                              some(w2tp)))
+                return (w1p if pk_up else w1, None, w2p if pk_down else w2, None)
+            if hp == hidden and dp == r.width:
+                w1 = torch.stack([e.linear_fc1.weight.detach() for e in experts]).to(dtype)
+                w2 = torch.stack([e.linear_fc2.weight.detach() for e in experts]).to(dtype)
+            else:
+                n = len(experts)
+                dev = experts[0].linear_fc1.weight.device
+                w1 = torch.zeros(n, (2 if gated else 1) * hp, dp, device=dev, dtype=dtype)
+                w2 = torch.zeros(n, dp, hp, device=dev, dtype=dtype)
+                for i, e in enumerate(experts):
+                    fc1 = e.linear_fc1.weight.detach()
+                    if gated:
+                        w1[i, :hidden, :r.width] = fc1[:hidden]
+                        w1[i, hp:hp + hidden, :r.width] = fc1[hidden:]
+                    else:
+                        w1[i, :hidden, :r.width] = fc1
+                    w2[i, :r.width, :hidden] = e.linear_fc2.weight.detach()
+            if not fp8:
+                up = nat.EPI_SWIGLU if gated else nat.EPI_RELU2
+                w1, w2 = w1.contiguous(), w2.contiguous()
+                plain.append((w1, w2, None, None, None, None))
+                return (ops.pack_expert_weights.raw(w1, up) if pk_up else w1, None,
+                        ops.pack_expert_weights.raw(w2, nat.EPI_NONE) if pk_down else w2, None)
+            w1q, w1s = ops.quantize_fp8_blockwise(w1.contiguous())
+            w2q, w2s = ops.quantize_fp8_blockwise(w2.contiguous())
+            up = nat.EPI_SWIGLU if gated else nat.EPI_RELU2
+            return (ops.pack_expert_weights_fp8(w1q, up), w1s,
+                    ops.pack_expert_weights_fp8(w2q, nat.EPI_NONE), w2s)
+
+        plain = []  # the bf16 [E, rows, cols] stacks before packing (for the backward)
+        packed = dict(shared_w1=None, shared_w2=None,
+                      shared_w1_scale=None, shared_w2_scale=None,
+                      packed=True if fp8 else (pk_up, pk_down))
+        (packed["w1"], packed["w1_scale"], packed["w2"],
+         packed["w2_scale"]) = stack(list(self.experts.local_experts), r.expert_width,
+                                     (self._fc1_pool, self._fc2_pool))
+        if self.shared_experts is not None:
+            (packed["shared_w1"], packed["shared_w1_scale"], packed["shared_w2"],
+             packed["shared_w2_scale"]) = stack([self.shared_experts], r.shared_expert_width,
+                                                 need_w1=True)
+        if keep_plain and not fp8:
+            (packed["w1_plain"], packed["w2_plain"], packed["w1_t"], packed["w2_t"],
+             packed["w1_t_packed"], packed["w2_t_packed"]) = plain[0]
+            (packed["shared_w1_plain"], packed["shared_w2_plain"], _, packed["shared_w2_t"],
+             _, packed["shared_w2_t_packed"]) = plain[1] if len(plain) > 1 else (None,) * 6
+        # the router's operands after the expert conversions, whose GPU time then covers
+        # this host work: w_router_t and, for the backward, the first operand in one kernel
+        rw = self.router.weight.detach()
+        packed["first"] = None
+        if on_gpu:
+            want_first = keep_plain and not fp8
+            sw1 = packed.get("shared_w1_plain") if want_first else None
+            if rw.dtype != torch.float32 or rw.stride(1) != 1:
+                rw = rw.float().contiguous()
+            packed["router_t"], first = ops.router_operands.raw(
+                rw, dp, None if sw1 is None else sw1[0], want_first)
+            if want_first:
+                packed["first"] = first
+        else:
+            router_t = torch.zeros(dp, r.routed_experts, device=rw.device,
+                                   dtype=torch.float32)
+            router_t[:r.width] = rw.t()
+            packed["router_t"] = router_t
+        self._packed = packed
 
     # -- forward ---------------------------------------------------------------------------
 

@@ -21,6 +21,15 @@ def _stream(device):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
+def _native_call(fn, args, device):
+    """fn(*args, stream) of the native host path: its result, or None where it does not take these
+    arguments (the caller then goes through the ops)."""
+    r = fn(*args, torch.cuda.current_stream(device).cuda_stream)
+    if r is not None and len(r) == 2:
+        nat.check(*r)
+    return r
+
+
 def _require(cond, message):
     if not cond:
         raise ValueError(message)
@@ -760,6 +769,29 @@ def _whole_batch_segment(T, device):
     return seg
 
 
+def _native_forward(x, w_router_t, w1, w2, top_k, score_fn, activation, aux_coeff, z_coeff,
+                    logit_bias, shared_w1, shared_w2, want_logits, keep):
+    """moe_forward on packed bf16 weights through the native host path: the same calls on the same
+    buffers, or None where that path does not take the arguments (the ops then do or refuse)."""
+    if not x.is_cuda:
+        return None
+    seg = None if shared_w1 is None else _whole_batch_segment(x.shape[0], x.device)
+    r = _native_call(nat.host().forward, (
+        x, w_router_t, logit_bias, w1, w2, shared_w1, shared_w2, seg, top_k, score_fn,
+        nat.EPI_SWIGLU if activation == nat.ACT_SWIGLU else nat.EPI_RELU2, aux_coeff, z_coeff,
+        want_logits, keep), x.device)
+    if r is None:
+        return None
+    (out, aux, logits, ids, w, pp, zp, counts, offsets, src, perm_w, cdest, cw, h, y, fc1, hs,
+     fc1s) = r
+    state = dict(logits=logits, ids=ids, weights=w, counts=counts, offsets=offsets, src_row=src,
+                 perm_w=perm_w, combine_dest=cdest, combine_w=cw)
+    if keep:
+        state.update(h=h, y=y, shared_h=hs, prob_partial=pp, z_partial=zp, fc1=fc1,
+                     shared_fc1=fc1s)
+    return out, aux, state
+
+
 def moe_forward(x, w_router_t, w1, w2, *, top_k, score_fn=nat.SCORE_SOFTMAX,
                 activation=nat.ACT_SWIGLU, aux_coeff=0.01, z_coeff=0.001, logit_bias=None,
                 shared_w1=None, shared_w2=None, want_logits=False, permute_rows=False,
@@ -789,6 +821,12 @@ def moe_forward(x, w_router_t, w1, w2, *, top_k, score_fn=nat.SCORE_SOFTMAX,
     T = x.shape[0]
     E = w_router_t.shape[1]
     A = T * top_k
+    if (T > 0 and mark is None and not permute_rows and w1.dtype == torch.bfloat16
+            and packed in (True, (True, True))):
+        fast = _native_forward(x, w_router_t, w1, w2, top_k, score_fn, activation, aux_coeff,
+                               z_coeff, logit_bias, shared_w1, shared_w2, want_logits, keep)
+        if fast is not None:
+            return fast
     mark = mark or (lambda name: None)
     if T == 0:
         dev = x.device
@@ -1348,6 +1386,35 @@ def _unit_weights(T, k, device):
     return t
 
 
+def _native_backward(g, grad_aux, x, w_router_t, bw, state, top_k, score_fn, activation,
+                     aux_coeff, z_coeff, weight_grads_fp32):
+    """moe_backward with packed dgrad weights and kept pre-activations through the native host
+    path, or None where it does not take them."""
+    fc1, fc1s = state.get("fc1"), state.get("shared_fc1")
+    sh = bw.shared_w1 is not None
+    if not (x.is_cuda and fc1 is not None and bw.w1t.packed and bw.w2t.packed
+            and (not sh or (fc1s is not None and bw.shared["w2t"].packed))):
+        return None
+    T, d = x.shape
+    E = w_router_t.shape[1]
+    dev = x.device
+    h, hs = state["h"], state["shared_h"] if sh else None
+    wf, (Fs, Ep, Kc) = bw.first(w_router_t)
+    rows = T * top_k // E
+    r = _native_call(nat.host().backward, (
+        g, grad_aux, x, bw.w1t.w, bw.w2t.w, bw.shared["w2t"].w if sh else None, wf, fc1, h,
+        state["perm_w"], state["src_row"], state["offsets"], state["combine_dest"], state["ids"],
+        state["weights"], state["logits"], state["counts"], state["prob_partial"],
+        state["z_partial"], fc1s if sh else None, hs, _unit_weights(T, top_k, dev),
+        _whole_batch_segment(T, dev), Fs, Ep, activation, score_fn, aux_coeff, z_coeff,
+        wgrad_splits(E, fc1.shape[1], d, rows, dev), wgrad_splits(E, d, h.shape[1], rows, dev),
+        wgrad_splits(1, 2 * Ep, d, T, dev), wgrad_splits(1, Fs, d, T, dev) if sh else 1,
+        wgrad_splits(1, d, hs.shape[1], T, dev) if sh else 1, weight_grads_fp32), dev)
+    if r is None:
+        return None
+    return dict(zip(("x", "router", "w1", "w2", "shared_w1", "shared_w2"), r))
+
+
 def moe_backward(grad_out, grad_aux, x, w_router_t, bw, state, *, top_k,
                  score_fn=nat.SCORE_SOFTMAX, activation=nat.ACT_SWIGLU, aux_coeff=0.01,
                  z_coeff=0.001, mark=None, weight_grads_fp32=False):
@@ -1372,6 +1439,12 @@ def moe_backward(grad_out, grad_aux, x, w_router_t, bw, state, *, top_k,
     carries g to about 2^-17 |g|; the router gradients are checked against fp64), the last
     two split along T in fixed order. `mark(name)` as in moe_forward.
     """
+    if mark is None and x.shape[0] > 0:
+        fast = _native_backward(grad_out.to(torch.bfloat16).contiguous(), grad_aux, x, w_router_t,
+                                bw, state, top_k, score_fn, activation, aux_coeff, z_coeff,
+                                weight_grads_fp32)
+        if fast is not None:
+            return fast
     mark = mark or (lambda name: None)
     T, d = x.shape
     E = w_router_t.shape[1]

@@ -248,3 +248,60 @@ def test_plugin_ffn_forward():
     ref = _oracle_for(module.engine, x)
     assert y.shape == x.shape and torch.is_tensor(module.last_aux)
     assert rel_l2(y.float().reshape(-1, 128), ref["out"]) <= BF16_TOL
+
+
+@pytest.mark.parametrize("T", [1, 65, 700])
+@pytest.mark.parametrize("E,k,d,H,act,score,Hs", [
+    (8, 2, 256, 512, 0, 0, 0), (32, 4, 1024, 512, 0, 1, 512), (16, 3, 320, 320, 1, 0, 320),
+    (16, 2, 256, 256, 1, 1, 448)])
+def test_native_host_path_equals_the_ops(T, E, k, d, H, act, score, Hs):
+    """moe_forward and moe_backward through the native host path (no mark) against the same calls
+    through the ops (any mark): every output bit for bit, forward with and without keep, logits
+    and bias, backward with and without an aux gradient, in fp32 and bf16, on strided rows."""
+    from nexttransformer_amd import ops
+    g = torch.Generator().manual_seed(T + E)
+    mk = lambda *s, std=0.05: (torch.randn(s, generator=g) * std).cuda()
+    f = 2 if act == 0 else 1
+    x = mk(T, 2 * d, std=1.0).to(torch.bfloat16)[:, :d]
+    wr, bias = mk(d, E, std=0.1), mk(E)
+    w1, w2 = mk(E, f * H, d).bfloat16(), mk(E, d, H).bfloat16()
+    s1, s2 = (mk(1, f * Hs, d).bfloat16(), mk(1, d, Hs).bfloat16()) if Hs else (None, None)
+    epi = act
+    pk = lambda w, e: None if w is None else ops.pack_expert_weights(w, e)
+    kw = dict(top_k=k, score_fn=score, activation=act, packed=True, shared_w1=pk(s1, epi),
+              shared_w2=pk(s2, 2))
+    stages = []
+    for bias_, want, keep in ((None, False, False), (bias, True, True)):
+        args = dict(kw, logit_bias=bias_, want_logits=want, keep=keep)
+        fast = ops.moe_forward(x, wr, pk(w1, epi), pk(w2, 2), **args)
+        slow = ops.moe_forward(x, wr, pk(w1, epi), pk(w2, 2), mark=stages.append, **args)
+        assert torch.equal(fast[0], slow[0]) and torch.equal(fast[1], slow[1])
+        assert fast[2].keys() == slow[2].keys()
+        for n, t in slow[2].items():
+            assert (t is None and fast[2][n] is None) or torch.equal(t, fast[2][n]), n
+    assert stages.count("combine") == 2
+    go = mk(T, d, std=1.0).to(torch.bfloat16)
+    for aux, wide in ((None, False), (torch.tensor([1.0, 0.5, 0.0]).cuda(), True)):
+        bw = ops.backward_weights(w1, w2, s1, s2, wr)
+        args = dict(top_k=k, score_fn=score, activation=act, weight_grads_fp32=wide)
+        a = ops.moe_backward(go, aux, x, wr, bw, fast[2], **args)
+        b = ops.moe_backward(go, aux, x, wr, bw, slow[2], mark=stages.append, **args)
+        for n, t in b.items():
+            assert (t is None and a[n] is None) or torch.equal(t, a[n]), n
+
+
+def test_native_host_path_refuses_what_the_ops_refuse():
+    from nexttransformer_amd import ops
+    x = torch.randn(4, 256).cuda()
+    wr = torch.randn(256, 8).cuda()
+    w1, w2 = torch.zeros(8, 1024, 256).cuda().bfloat16(), torch.zeros(8, 256, 512).cuda().bfloat16()
+    call = lambda x, wr, w1, w2, **kw: ops.moe_forward(x, wr, w1, w2, top_k=2, packed=True, **kw)
+    xb = x.bfloat16()
+    call(xb, wr, w1, w2)
+    for args, kw in (((x, wr, w1, w2), {}), ((xb, wr.bfloat16(), w1, w2), {}),
+                     ((xb, wr.t(), w1, w2), {}), ((xb, wr, w1[:, :, ::2], w2), {}),
+                     ((xb, wr, w1, w2), dict(logit_bias=torch.zeros(7).cuda())),
+                     ((xb.t().contiguous().t(), wr, w1, w2), {}),
+                     ((xb[:, :64], wr[:64].contiguous(), w1[:, :, :64].contiguous(), w2), {})):
+        with pytest.raises(ValueError):
+            call(*args, **kw)
