@@ -11,8 +11,8 @@
 // as the packed bf16 kernel's tile.
 //   * Wave w owns the tile's packed 32-row weight block w against all of its token blocks (up to
 //     8 accumulators); the weights are private to the wave, so they skip LDS (1 KB loads, one
-//     step ahead; two steps ahead in tiles of 128 rows and fewer, which are bound by the weight
-//     stream and have the registers to spare).
+//     step ahead; two steps ahead in tiles of 64 to 192 rows, which have the registers to spare:
+//     at 224 rows five would spill).
 //   * Token rows go through LDS in a ring of two steps (direct-to-LDS loads, 16-byte chunks
 //     XOR-swizzled by row as in the packed bf16 kernel), one barrier per step.
 //   * The scale of a 128 x 128 weight block is an fp32 number, not a power of two, so each step's
@@ -23,9 +23,12 @@
 // Two workgroups per CU: one's barriers, start and stores run under the other's products. A
 // segment's rows are dealt evenly to its tiles in multiples of 32, so a segment of 260 rows is
 // two tiles of 128 and 132 and not 256 and 4.
+// The tile is instantiated for each number of 32-row blocks: with 1, 2, 4, 6 and 8 only (and two
+// steps ahead up to 4) a tile of 9 / 2 blocks multiplied a sixth for padding, 4096 tokens below
+// 569 / 350 us against 536 / 342, the forward 1110 against 1082.
 //
 // Measured, us up / down projection, that kernel -> this one (128 experts, top-8, d 4096, H 1536;
-// outputs bit-identical): 4096 tokens (256 rows per expert) 2285 / 1265 -> 569 / 350 (1450 / 1180
+// outputs bit-identical): 4096 tokens (256 rows per expert) 2285 / 1265 -> 536 / 342 (1540 / 1200
 // TFLOP/s), 1024 tokens 677 / 390 -> 300 / 194, 256 tokens 279 / 183 -> 278 / 163, 64 tokens 260 /
 // 156 -> 268 / 154. At 1024 tokens and fewer the time is the weight stream's.
 #include <math.h>
@@ -68,7 +71,7 @@ struct F8Args {
 template <int EPI, int NJ>
 __device__ __forceinline__ void fp8_tile(const F8Args& p, unsigned char* smem, int s, int nt,
                                          int m0, int m_end) {
-  constexpr int D = NJ == 2 || NJ == 4 ? 2 : 1;  // weight steps in flight beyond the current one
+  constexpr int D = NJ == 1 || NJ >= 7 ? 1 : 2;  // weight steps in flight beyond the current one
   constexpr int kStage = NJ * 32 * kKB;
   constexpr bool SW = EPI == NT_MOE_EPI_SWIGLU;
   const int lane = lane_id(), wave = wave_id();
@@ -337,9 +340,12 @@ __global__ __launch_bounds__(256, 2) void fp8_tiled_gemm_kernel(F8Args p) {
   m0 = __builtin_amdgcn_readfirstlane(m0);
   m_end = __builtin_amdgcn_readfirstlane(m_end);
   const int rows = m_end - m0;
-  if (rows > 192) fp8_tile<EPI, 8>(p, smem, s, nt, m0, m_end);
-  else if (rows > 128) fp8_tile<EPI, 6>(p, smem, s, nt, m0, m_end);
-  else if (rows > 64) fp8_tile<EPI, 4>(p, smem, s, nt, m0, m_end);
+  if (rows > 224) fp8_tile<EPI, 8>(p, smem, s, nt, m0, m_end);
+  else if (rows > 192) fp8_tile<EPI, 7>(p, smem, s, nt, m0, m_end);
+  else if (rows > 160) fp8_tile<EPI, 6>(p, smem, s, nt, m0, m_end);
+  else if (rows > 128) fp8_tile<EPI, 5>(p, smem, s, nt, m0, m_end);
+  else if (rows > 96) fp8_tile<EPI, 4>(p, smem, s, nt, m0, m_end);
+  else if (rows > 64) fp8_tile<EPI, 3>(p, smem, s, nt, m0, m_end);
   else if (rows > 32) fp8_tile<EPI, 2>(p, smem, s, nt, m0, m_end);
   else fp8_tile<EPI, 1>(p, smem, s, nt, m0, m_end);
 }

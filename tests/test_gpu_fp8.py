@@ -174,7 +174,7 @@ def test_fp8_layer_config5_full_size():
     assert rel_l2(out[tokens].float(), ref["out"]) <= FP8_LAYER_TOL
 
 
-# segment lengths at the edges of the tiled kernel's row variants (32, 64, 128, 192, 256 rows), of
+# segment lengths at the edges of the tiled kernel's row variants (every 32 rows up to 256), of
 # its even split into tiles (257, 300, 513) and an empty one; K = 1 to 7 steps of its rings, and
 # one K past its limit (the streaming kernel's)
 @pytest.mark.parametrize("K", [128, 256, 384, 512, 896, 8320])
@@ -186,7 +186,8 @@ def test_fp8_many_rows_equal_the_streaming_kernel(K, epilogue, gather):
     from nexttransformer_amd import _native as nat
     from nexttransformer_amd import ops
     g = torch.Generator().manual_seed(K + epilogue)
-    counts = [1, 32, 33, 0, 64, 65, 128, 129, 192, 193, 256, 257, 300, 513]
+    counts = [1, 32, 33, 0, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 225, 256, 257, 300,
+              513]
     S, n_out, rows = len(counts), 128, sum(counts)
     R = 2 * n_out if epilogue == nat.EPI_SWIGLU else n_out
     a_rows = 700 if gather else rows
