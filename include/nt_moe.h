@@ -415,7 +415,16 @@ int nt_moe_grouped_gemm_fp8_packed(const uint8_t* a, int64_t ld_a, int64_t a_row
  *   lb = aux_coeff * E / (k * T^2) * sum_e (sum_t s_te) * counts[e]
  *   z  = z_coeff * mean_t logsumexp(logits_t)^2
  *   aux_out fp32 [3] = {lb + z, lb, z}
+ * nt_moe_combine_aux_load also writes counts as int64 to load [E] (last_load,
+ * megatron_moe.py:143,149) from the workgroup that computes the losses: a conversion launch of its
+ * own took 4 us of a decode pass. load needs aux_out; NULL: not written.
  */
+int nt_moe_combine_aux_load(const uint16_t* y, const int32_t* combine_dest, const float* combine_w,
+                            int64_t T, int32_t d, int32_t k, const uint16_t* shared_y,
+                            int64_t ld_shared, uint16_t* out, int64_t ld_out,
+                            const float* prob_partial, const float* z_partial,
+                            const int32_t* counts, int32_t E, float aux_coeff, float z_coeff,
+                            float* aux_out, int64_t* load, nt_moe_stream_t stream);
 int nt_moe_combine_aux(const uint16_t* y, const int32_t* combine_dest, const float* combine_w,
                        int64_t T, int32_t d, int32_t k, const uint16_t* shared_y,
                        int64_t ld_shared, uint16_t* out, int64_t ld_out,

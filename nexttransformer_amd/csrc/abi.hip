@@ -1039,6 +1039,17 @@ int nt_moe_combine_aux(const uint16_t* y, const int32_t* combine_dest, const flo
                        const float* prob_partial, const float* z_partial,
                        const int32_t* counts, int32_t E, float aux_coeff, float z_coeff,
                        float* aux_out, nt_moe_stream_t stream) {
+  return nt_moe_combine_aux_load(y, combine_dest, combine_w, T, d, k, shared_y, ld_shared, out,
+                                 ld_out, prob_partial, z_partial, counts, E, aux_coeff, z_coeff,
+                                 aux_out, nullptr, stream);
+}
+
+int nt_moe_combine_aux_load(const uint16_t* y, const int32_t* combine_dest, const float* combine_w,
+                            int64_t T, int32_t d, int32_t k, const uint16_t* shared_y,
+                            int64_t ld_shared, uint16_t* out, int64_t ld_out,
+                            const float* prob_partial, const float* z_partial,
+                            const int32_t* counts, int32_t E, float aux_coeff, float z_coeff,
+                            float* aux_out, int64_t* load, nt_moe_stream_t stream) {
   int rc = check_route_shape(T, k, E);
   if (rc) return rc;
   NT_REQUIRE(d > 0 && d % 8 == 0, "combine: d must be a positive multiple of 8, got %d", d);
@@ -1050,9 +1061,10 @@ int nt_moe_combine_aux(const uint16_t* y, const int32_t* combine_dest, const flo
     NT_REQUIRE(aligned16(y) && aligned16(out), "combine: y and out must be 16-byte aligned");
   }
   if (aux_out) NT_REQUIRE(counts && (T == 0 || (prob_partial && z_partial)), "combine: null aux input");
+  NT_REQUIRE(!load || aux_out, "combine: load needs aux_out");
   hipError_t err = launch_combine_aux(y, combine_dest, combine_w, T, d, k, shared_y, ld_shared,
                                       out, ld_out, prob_partial, z_partial, counts, E, aux_coeff,
-                                      z_coeff, aux_out, reinterpret_cast<hipStream_t>(stream));
+                                      z_coeff, aux_out, load, reinterpret_cast<hipStream_t>(stream));
   return launched(err, "combine_aux");
 }
 

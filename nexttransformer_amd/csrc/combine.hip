@@ -143,11 +143,15 @@ constexpr int kAuxThreads = 256;
 __device__ void aux_block(const float* __restrict__ prob_partial,
                           const float* __restrict__ z_partial, int nblk,
                           const int32_t* __restrict__ counts, int E, int P, int k, int64_t T,
-                          float aux_coeff, float z_coeff, float* __restrict__ aux_out) {
+                          float aux_coeff, float z_coeff, float* __restrict__ aux_out,
+                          int64_t* __restrict__ load) {
   __shared__ double red[kAuxThreads];
   __shared__ double zred[kAuxThreads];
   const int tid = threadIdx.x;
   const int e = tid / P, p = tid - (tid / P) * P;
+  // last_load, here rather than in a conversion launch (E <= kAuxThreads): one token of 32
+  // experts 63 -> 53 us a pass, 48 tokens of 256 experts 105 -> 100
+  if (load && tid < E) load[tid] = counts[tid];
   double s = 0.0;
   if (e < E) {
 #pragma unroll 8
@@ -191,6 +195,7 @@ struct AuxArgs {
   int nblk, E, P;
   float aux_coeff, z_coeff;
   float* aux_out;  // null: no aux workgroup
+  int64_t* load;   // [E], counts as 64-bit numbers; may be null
 };
 
 // The combine grid plus, when aux.aux_out is set, one last workgroup that computes the losses
@@ -204,7 +209,7 @@ __global__ __launch_bounds__(256) void combine_aux_kernel(
   const int combine_blocks = (int)gridDim.x - (aux.aux_out ? 1 : 0);
   if ((int)blockIdx.x == combine_blocks) {
     aux_block(aux.prob_partial, aux.z_partial, aux.nblk, aux.counts, aux.E, aux.P, k, T,
-              aux.aux_coeff, aux.z_coeff, aux.aux_out);
+              aux.aux_coeff, aux.z_coeff, aux.aux_out, aux.load);
     return;
   }
   combine_rows<KMAX, VPC>(y, combine_dest, combine_w, T, d, k, shared_y, ld_shared, out, ld_out,
@@ -218,9 +223,9 @@ hipError_t launch_combine_aux(const uint16_t* y, const int32_t* combine_dest,
                               const uint16_t* shared_y, int64_t ld_shared, uint16_t* out,
                               int64_t ld_out, const float* prob_partial, const float* z_partial,
                               const int32_t* counts, int E, float aux_coeff, float z_coeff,
-                              float* aux_out, hipStream_t stream) {
+                              float* aux_out, int64_t* load, hipStream_t stream) {
   AuxArgs aux{prob_partial, z_partial, counts, ceil_div(T, kRouteBlock), E, 1, aux_coeff,
-              z_coeff, aux_out};
+              z_coeff, aux_out, load};
   while (aux.P * 2 * E <= kAuxThreads) aux.P *= 2;
   // persistent waves, as many as stay resident at the variant's register use (each then takes
   // several tokens), or one per token

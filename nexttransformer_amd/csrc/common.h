@@ -164,7 +164,7 @@ hipError_t launch_combine_aux(const uint16_t* y, const int32_t* combine_dest,
                               const uint16_t* shared_y, int64_t ld_shared, uint16_t* out,
                               int64_t ld_out, const float* prob_partial, const float* z_partial,
                               const int32_t* counts, int E, float aux_coeff, float z_coeff,
-                              float* aux_out, hipStream_t stream);
+                              float* aux_out, int64_t* load, hipStream_t stream);
 
 hipError_t launch_quantize_fp8_rowwise(const uint16_t* x, int64_t ld_x, int64_t rows, int d,
                                        uint8_t* q, int64_t ld_q, float* scale, hipStream_t stream);

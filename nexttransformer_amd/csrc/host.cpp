@@ -144,7 +144,8 @@ int64_t route_blocks(int64_t T) { return (T + NT_MOE_ROUTE_BLOCK - 1) / NT_MOE_R
 // forward(x, w_router_t, bias | None, w1, w2, shared_w1 | None, shared_w2 | None, segment | None,
 //         top_k, score_fn, up_epilogue, aux_coeff, z_coeff, want_logits, keep, stream)
 // -> (out, aux, logits, ids, weights, prob_partial, z_partial, counts, offsets, src_row, perm_w,
-//     combine_dest, combine_w, h, y, fc1, shared_h, shared_fc1); the last five None without keep.
+//     combine_dest, combine_w, load, h, y, fc1, shared_h, shared_fc1); the last five None without
+//     keep. load: counts as int64.
 PyObject* forward(PyObject*, PyObject* const* argv, Py_ssize_t argc) {
   HANDLE_TH_ERRORS
   constexpr auto BF = at::kBFloat16, F = at::kFloat, I = at::kInt;
@@ -227,15 +228,15 @@ PyObject* forward(PyObject*, PyObject* const* argv, Py_ssize_t argc) {
                                            bfw(y), st),
            "ntmoe::grouped_gemm_packed");
     }
-    Tensor out = mk({T, D}, BF), aux = mk({3}, F);
-    must(nt_moe_combine_aux(bf(y), i32(cdest), f32(cw), T, (int32_t)D, (int32_t)k,
-                            sh ? bf(ys) : nullptr, sh ? D : 0, bfw(out), D, f32(pp), f32(zp),
-                            i32(counts), (int32_t)E, (float)aux_coeff, (float)z_coeff, f32(aux),
-                            st),
+    Tensor out = mk({T, D}, BF), aux = mk({3}, F), load = mk({E}, at::kLong);
+    must(nt_moe_combine_aux_load(bf(y), i32(cdest), f32(cw), T, (int32_t)D, (int32_t)k,
+                                 sh ? bf(ys) : nullptr, sh ? D : 0, bfw(out), D, f32(pp), f32(zp),
+                                 i32(counts), (int32_t)E, (float)aux_coeff, (float)z_coeff,
+                                 f32(aux), static_cast<int64_t*>(load.data_ptr()), st),
          "ntmoe::combine_aux");
-    r = {out, aux, logits, ids, w, pp, zp, counts, offsets, src, perm_w, cdest, cw};
+    r = {out, aux, logits, ids, w, pp, zp, counts, offsets, src, perm_w, cdest, cw, load};
     if (keep) r.insert(r.end(), {h, y, fc1, hs, fc1s});
-    else r.resize(18);
+    else r.resize(19);
   } catch (const Failed& f) {
     return failed(f);
   }

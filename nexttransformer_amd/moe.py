@@ -198,7 +198,7 @@ class _MoETrain(torch.autograd.Function):
             activation=cfg["activation"], aux_coeff=cfg["aux_coeff"], z_coeff=cfg["z_coeff"],
             logit_bias=layer.logit_bias, shared_w1=w["shared_w1"], shared_w2=w["shared_w2"],
             want_logits=True, packed=w["packed"], keep=True)
-        cfg["counts"] = state["counts"]
+        cfg["load"] = state["load"]
         ctx.cfg, ctx.state, ctx.x, ctx.w = cfg, state, x, w
         # an output the loss does not use gets None, not a zero-filled gradient
         ctx.set_materialize_grads(False)
@@ -281,21 +281,13 @@ class MoELayer(nn.Module):
         # Optional fixed per-expert logit bias [E] fp32 added after the gating GEMM (not a
         # parameter; None = no bias, the reference router): used to impose a routing skew.
         self.register_buffer("logit_bias", None)
-        self._last_counts = None
+        # Per-expert token counts of the last forward, int64 [E] (None before the first).
+        self.last_load = None
         self.last_aux_loss = None
         self.last_aux_parts = None
         self._pack_key = None
         self._packed = None
         self.reset_parameters()
-
-    @property
-    def last_load(self):
-        """Per-expert token counts of the last forward, int64 [E] (None before the first): the
-        kernels' int32 counts, converted on first access rather than in every forward."""
-        c = self._last_counts
-        if c is not None and c.dtype != torch.int64:
-            c = self._last_counts = c.to(torch.int64)
-        return c
 
     # -- initialisation --------------------------------------------------------------------
 
@@ -652,7 +644,7 @@ class MoELayer(nn.Module):
             shared_w2_scale=w["shared_w2_scale"], packed=w["packed"])
         if dp != r.width:
             out = out[:, :r.width]
-        self._last_counts = state["counts"]
+        self.last_load = state["load"]
         self.last_aux_parts = aux
         self.last_aux_loss = aux[0]
         out = out.reshape(hidden.shape).to(hidden.dtype)
@@ -685,7 +677,7 @@ class MoELayer(nn.Module):
         out, aux = _MoETrain.apply(x, cfg, anchor, *masters)
         if dp != r.width:
             out = out[:, :r.width]
-        self._last_counts = cfg["counts"]
+        self.last_load = cfg["load"]
         self.last_aux_parts = aux.detach()
         # "inject": the gradient comes from the backward itself, so the returned value is
         # detached and adding it to a loss changes nothing

@@ -720,6 +720,13 @@ def combine_aux(y: Tensor, combine_dest: Tensor, combine_w: Tensor, shared_y: Op
                 prob_partial: Tensor, z_partial: Tensor, counts: Tensor, aux_coeff: float,
                 z_coeff: float) -> tuple[Tensor, Tensor]:
     """(out [T, d] bf16, aux fp32 [3] = {lb + z, lb, z})."""
+    return _combine_aux(y, combine_dest, combine_w, shared_y, prob_partial, z_partial, counts,
+                        aux_coeff, z_coeff, None)
+
+
+def _combine_aux(y, combine_dest, combine_w, shared_y, prob_partial, z_partial, counts, aux_coeff,
+                 z_coeff, load):
+    """combine_aux; the launch also writes the counts to load, int64 [E], unless that is None."""
     _on_gpu(y, combine_dest, combine_w, shared_y, prob_partial, z_partial, counts)
     _require(y.dtype == torch.bfloat16 and y.dim() == 2 and y.is_contiguous(),
              "combine_aux: y must be contiguous bf16 [A, d]")
@@ -737,11 +744,11 @@ def combine_aux(y: Tensor, combine_dest: Tensor, combine_w: Tensor, shared_y: Op
     dev = y.device
     out = torch.empty(T, d, device=dev, dtype=torch.bfloat16)
     aux = torch.empty(3, device=dev, dtype=torch.float32)
-    st = nat.load().nt_moe_combine_aux(
+    st = nat.load().nt_moe_combine_aux_load(
         ptr(y), ptr(combine_dest), ptr(combine_w), T, d, k, ptr(shared_y),
         shared_y.stride(0) if shared_y is not None else 0, ptr(out), out.stride(0),
         ptr(prob_partial), ptr(z_partial), ptr(counts), E, float(aux_coeff), float(z_coeff),
-        ptr(aux), _stream(dev))
+        ptr(aux), ptr(load), _stream(dev))
     nat.check(st, "ntmoe::combine_aux")
     return out, aux
 
@@ -782,10 +789,10 @@ def _native_forward(x, w_router_t, w1, w2, top_k, score_fn, activation, aux_coef
         want_logits, keep), x.device)
     if r is None:
         return None
-    (out, aux, logits, ids, w, pp, zp, counts, offsets, src, perm_w, cdest, cw, h, y, fc1, hs,
-     fc1s) = r
+    (out, aux, logits, ids, w, pp, zp, counts, offsets, src, perm_w, cdest, cw, load, h, y, fc1,
+     hs, fc1s) = r
     state = dict(logits=logits, ids=ids, weights=w, counts=counts, offsets=offsets, src_row=src,
-                 perm_w=perm_w, combine_dest=cdest, combine_w=cw)
+                 perm_w=perm_w, combine_dest=cdest, combine_w=cw, load=load)
     if keep:
         state.update(h=h, y=y, shared_h=hs, prob_partial=pp, z_partial=zp, fc1=fc1,
                      shared_fc1=fc1s)
@@ -836,7 +843,8 @@ def moe_forward(x, w_router_t, w1, w2, *, top_k, score_fn=nat.SCORE_SOFTMAX,
                      weights=empty(0, top_k, dtype=f32), counts=torch.zeros(E, device=dev, dtype=i32),
                      offsets=torch.zeros(E + 1, device=dev, dtype=i32), src_row=empty(0),
                      perm_w=empty(0, dtype=f32), combine_dest=empty(0, top_k),
-                     combine_w=empty(0, top_k, dtype=f32))
+                     combine_w=empty(0, top_k, dtype=f32),
+                     load=torch.zeros(E, device=dev, dtype=torch.int64))
         return x.new_empty(0, x.shape[1]), torch.zeros(3, device=dev, dtype=f32), state
     if permute_rows:
         logits, ids, w, pp, zp = router.raw(x, w_router_t, logit_bias, top_k, score_fn,
@@ -870,11 +878,12 @@ def moe_forward(x, w_router_t, w1, w2, *, top_k, score_fn=nat.SCORE_SOFTMAX,
             shared_y = grouped_gemm_fp8.raw(hsq, hss, None, seg, shared_w2, shared_w2_scale,
                                         nat.EPI_NONE, T, packed)
             mark("shared")
-        out, aux = combine_aux.raw(y, cdest, cw, shared_y, pp, zp, counts, aux_coeff, z_coeff)
+        load = torch.empty(E, device=x.device, dtype=torch.int64)
+        out, aux = _combine_aux(y, cdest, cw, shared_y, pp, zp, counts, aux_coeff, z_coeff, load)
         mark("combine")
         state = dict(logits=logits, ids=ids, weights=w, counts=counts, offsets=offsets,
                      src_row=src, perm_w=perm_w, combine_dest=cdest, combine_w=cw, x_q=xq,
-                     x_scale=xs)
+                     x_scale=xs, load=load)
         return out, aux, state
     packed_up, packed_down = (packed, packed) if isinstance(packed, bool) else packed
     gemm_up = grouped_gemm_packed.raw if packed_up else grouped_gemm.raw
@@ -920,10 +929,11 @@ def moe_forward(x, w_router_t, w1, w2, *, top_k, score_fn=nat.SCORE_SOFTMAX,
         shared_y = gemm_down(hs, None, seg, shared_w2, nat.EPI_NONE, T)
     if shared_w1 is not None:
         mark("shared")
-    out, aux = combine_aux.raw(y, cdest, cw, shared_y, pp, zp, counts, aux_coeff, z_coeff)
+    load = torch.empty(E, device=x.device, dtype=torch.int64)
+    out, aux = _combine_aux(y, cdest, cw, shared_y, pp, zp, counts, aux_coeff, z_coeff, load)
     mark("combine")
     state = dict(logits=logits, ids=ids, weights=w, counts=counts, offsets=offsets, src_row=src,
-                 perm_w=perm_w, combine_dest=cdest, combine_w=cw)
+                 perm_w=perm_w, combine_dest=cdest, combine_w=cw, load=load)
     if keep:
         state.update(h=h, y=y, shared_h=hs, prob_partial=pp, z_partial=zp, fc1=fc1,
                      shared_fc1=fc1s)

@@ -228,6 +228,21 @@ def test_combine_row_shapes_agree_bit_for_bit(T, k, shared):
     torch.testing.assert_close(wide.cpu().double(), ref, rtol=1e-2, atol=1e-3)
 
 
+@pytest.mark.parametrize("E", [3, 64, 256])
+def test_forward_load_is_the_counts_in_64_bits(E):
+    """The combine launch's int64 counts, next to the int32 ones it reads."""
+    from nexttransformer_amd import ops
+    gen = torch.Generator().manual_seed(E)
+    x = torch.randn(130, 256, generator=gen).to(torch.bfloat16).cuda()
+    wr = torch.randn(256, E, generator=gen).cuda()
+    w = torch.randn(E, 256, 256, generator=gen) * 0.05
+    p = ops.pack_expert_weights(w.to(torch.bfloat16).cuda(), 1)
+    p2 = ops.pack_expert_weights(w.to(torch.bfloat16).cuda(), 2)
+    _, _, st = ops.moe_forward(x, wr, p, p2, top_k=2, activation=1, packed=True)
+    assert st["load"].dtype == torch.int64 and st["load"].shape == (E,)
+    assert torch.equal(st["load"], st["counts"].long()) and int(st["load"].sum()) == 260
+
+
 @pytest.mark.parametrize("gather", [False, True])
 def test_grouped_wgrad_matches_float64(gather):
     """Ragged segments (empty, shorter than one 32-row step, not a multiple of it, long)."""
