@@ -22,13 +22,14 @@ namespace {
 // 85 against 96 us for the T3 cell's combine). Waves are persistent over tokens (t, t + the
 // grid's waves, ...) and walk the items (token, chunk) in order, issuing the next item's k row
 // loads (and its shared-expert chunk) before summing the current one, so 2 (k + 1) VPC vectors
-// per lane are in flight. KMAX bounds k (registers are sized by it).
+// per lane are in flight. With `split` (batches of at most one item per SIMD) each item
+// has a wave of its own. KMAX bounds k (registers are sized by it).
 template <int KMAX, int VPC>
 __device__ __forceinline__ void combine_rows(
     const uint16_t* __restrict__ y, const int32_t* __restrict__ combine_dest,
     const float* __restrict__ combine_w, int64_t T, int d, int k,
     const uint16_t* __restrict__ shared_y, int64_t ld_shared, uint16_t* __restrict__ out,
-    int64_t ld_out, int blocks) {
+    int64_t ld_out, int blocks, bool split) {
   const int lane = lane_id();
   const int vecs = d >> 3;
   const int chunk = 64 * VPC;
@@ -104,19 +105,25 @@ __device__ __forceinline__ void combine_rows(
   };
 
   int64_t t = (int64_t)blockIdx.x * 4 + wave_id();
+  int v0 = 0, vend = vecs, dest;
+  if (split) {
+    const int chunks = (vecs + chunk - 1) / chunk;
+    v0 = (int)(t % chunks) * chunk;
+    vend = v0 + chunk;
+    t /= chunks;
+  }
   if (t >= T) return;
-  int v0 = 0, dest;
   float w;
   u32x4 rows[KMAX][VPC], sh[VPC], nrows[KMAX][VPC], nsh[VPC];
   plan(t, dest, w);
-  load_rows(t, dest, 0, rows, sh);
+  load_rows(t, dest, v0, rows, sh);
   while (t < T) {
     // the next item: the row's next chunk, or the first chunk of the wave's next token
     int64_t tn = t;
     int vn = v0 + chunk, ndest = dest;
     float nw = w;
-    if (vn >= vecs) {
-      tn = t + waves;
+    if (vn >= vend) {
+      tn = split ? T : t + waves;
       vn = 0;
       plan(tn, ndest, nw);
     }
@@ -205,7 +212,7 @@ __global__ __launch_bounds__(256) void combine_aux_kernel(
     const uint16_t* __restrict__ y, const int32_t* __restrict__ combine_dest,
     const float* __restrict__ combine_w, int64_t T, int d, int k,
     const uint16_t* __restrict__ shared_y, int64_t ld_shared, uint16_t* __restrict__ out,
-    int64_t ld_out, AuxArgs aux) {
+    int64_t ld_out, AuxArgs aux, bool split) {
   const int combine_blocks = (int)gridDim.x - (aux.aux_out ? 1 : 0);
   if ((int)blockIdx.x == combine_blocks) {
     aux_block(aux.prob_partial, aux.z_partial, aux.nblk, aux.counts, aux.E, aux.P, k, T,
@@ -213,7 +220,7 @@ __global__ __launch_bounds__(256) void combine_aux_kernel(
     return;
   }
   combine_rows<KMAX, VPC>(y, combine_dest, combine_w, T, d, k, shared_y, ld_shared, out, ld_out,
-                          combine_blocks);
+                          combine_blocks, split);
 }
 
 }  // namespace
@@ -229,13 +236,19 @@ hipError_t launch_combine_aux(const uint16_t* y, const int32_t* combine_dest,
   while (aux.P * 2 * E <= kAuxThreads) aux.P *= 2;
   // persistent waves, as many as stay resident at the variant's register use (each then takes
   // several tokens), or one per token
-  int64_t blocks = (T + 3) / 4;
+  const bool two = (d / 8) % 128 == 0;  // rows of whole 2-vector chunks
   const int per_cu = k <= 2 ? 7 : (k <= 4 ? 4 : 3);
   const int64_t cap = (int64_t)num_cus() * per_cu;
+  // One wave per chunk while each has a SIMD of its own (a token's chunks one after another are a
+  // chain of latencies): forwards of 48 tokens, d = 1280, top-8 100.7 -> 98.4 us, of 64 tokens, d =
+  // 4096 458 -> 453; past that the waves share SIMDs and lose the next chunk's early loads (777
+  // tokens, d = 2048, 1554 chunks 284.9 -> 286.4).
+  const int64_t chunks = ceil_div(d / 8, two ? 128 : 64);
+  const bool split = chunks > 1 && T * chunks <= 4 * (int64_t)num_cus();
+  int64_t blocks = (T * (split ? chunks : 1) + 3) / 4;
   if (blocks > cap) blocks = cap;
   if (aux_out) ++blocks;
   if (blocks == 0) return hipSuccess;
-  const bool two = (d / 8) % 128 == 0;  // rows of whole 2-vector chunks
   auto kern = two ? (k <= 2 ? combine_aux_kernel<2, 2>
                             : (k <= 4 ? combine_aux_kernel<4, 2>
                                       : combine_aux_kernel<NT_MOE_MAX_TOPK, 2>))
@@ -243,7 +256,7 @@ hipError_t launch_combine_aux(const uint16_t* y, const int32_t* combine_dest,
                             : (k <= 4 ? combine_aux_kernel<4, 1>
                                       : combine_aux_kernel<NT_MOE_MAX_TOPK, 1>));
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, stream, y, combine_dest,
-                     combine_w, T, d, k, shared_y, ld_shared, out, ld_out, aux);
+                     combine_w, T, d, k, shared_y, ld_shared, out, ld_out, aux, split);
   hipError_t err = hipGetLastError();
   return err;
 }

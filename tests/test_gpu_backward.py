@@ -243,6 +243,33 @@ def test_forward_load_is_the_counts_in_64_bits(E):
     assert torch.equal(st["load"], st["counts"].long()) and int(st["load"].sum()) == 260
 
 
+@pytest.mark.parametrize("d", [1280, 1800, 2048])
+def test_combine_of_a_batch_equals_its_parts(d):
+    """One wave per chunk (a small batch) and persistent waves over whole tokens agree bit for bit:
+    batches on both sides of the line (1024 chunks on 256 CUs: 341 tokens at d = 1280, 256 at 1800,
+    512 at 2048), against parts of 100 tokens, which are split, and of 700, which are not."""
+    from nexttransformer_amd import ops
+    E, k, T = 16, 4, 2100
+    gen = torch.Generator().manual_seed(d)
+    y = torch.randn(T * k, d, generator=gen).to(torch.bfloat16).cuda()
+    dest = torch.randperm(T * k, generator=gen).int().view(T, k).cuda()
+    w = torch.rand(T, k, generator=gen).cuda()
+    counts = torch.full((E,), 7, dtype=torch.int32).cuda()
+
+    def combine(lo, hi):  # tokens lo .. hi - 1, their rows brought to the front
+        n = hi - lo
+        rows = y[dest[lo:hi].reshape(-1).long()].contiguous()
+        at = torch.arange(n * k, dtype=torch.int32).view(n, k).cuda()
+        pp, zp = torch.ones((n + 63) // 64, E).cuda(), torch.ones((n + 63) // 64).cuda()
+        return ops.combine_aux(rows, at, w[lo:hi].contiguous(), None, pp, zp, counts, 0.01,
+                               0.001)[0]
+
+    parts = torch.cat([combine(a, a + 100) for a in range(0, T, 100)])
+    assert torch.equal(parts, torch.cat([combine(a, a + 700) for a in range(0, T, 700)]))
+    for n in (1, 255, 256, 257, 341, 342, 512, 513, T):
+        assert torch.equal(combine(0, n), parts[:n]), n
+
+
 @pytest.mark.parametrize("gather", [False, True])
 def test_grouped_wgrad_matches_float64(gather):
     """Ragged segments (empty, shorter than one 32-row step, not a multiple of it, long)."""
