@@ -1499,6 +1499,8 @@ int logit_ranges(int d) {
   return nchunk >= 4 ? 4 : (nchunk >= 2 ? 2 : 1);
 }
 
+bool logits_kernel_takes(int d) { return ceil_div(d, kRouterChunk) <= 16; }
+
 enum RouterPath { kFused = 0, kLogits = 1, kPlanes = 2, kStream = 3 };
 
 // Path for this shape. Up to 128 experts: the fused kernel (top-k in the block, no workspace)
@@ -1535,10 +1537,10 @@ int router_path(int64_t T, int d, int E) {
   };
   if (E > 128 && E <= 256 && blocks * 8 >= 2LL * num_cus())
     return planes_win(10.5 * nchunk, blocks) ? kPlanes : kStream;
-  if (nchunk <= 16 && logit_waves >= 2LL * num_cus())
+  if (logits_kernel_takes(d) && logit_waves >= 2LL * num_cus())
     return planes_win(8.3 * ceil_div(nchunk, logit_ranges(d)), logit_wgs) ? kPlanes : kLogits;
   if (planes_fit) return kPlanes;
-  return nchunk <= 16 ? kLogits : (E <= 128 ? kFused : kStream);
+  return logits_kernel_takes(d) ? kLogits : (E <= 128 ? kFused : kStream);
 }
 
 template <int KMAX>
@@ -1638,11 +1640,13 @@ hipError_t launch_rank_finish(const float* planes, int nchunk, const float* bias
 }  // namespace
 
 // Whether the router ranks over the whole chip (router_rank_kernel, router_finish_kernel, which
-// then also writes the route plan): the shapes on the planes and logits paths.
+// then also writes the route plan): the shapes on the planes path, and those on the logits path
+// that the logits kernel takes (with a router mode forced, the others run a kernel that ranks in
+// its block and writes no plan).
 bool router_small(int64_t T, int d, int E, int k) {
   const int path = router_path(T, d, E);
-  return (path == kPlanes || path == kLogits) && E <= NT_MOE_MAX_EXPERTS &&
-         T * k <= kRankAssignments;
+  return (path == kPlanes || (path == kLogits && logits_kernel_takes(d))) &&
+         E <= NT_MOE_MAX_EXPERTS && T * k <= kRankAssignments;
 }
 
 // Workspace the router uses for this shape: the chunk planes or one T x E logits plane, then (for
@@ -1692,11 +1696,11 @@ hipError_t launch_router(const uint16_t* x, int64_t ld_x, const float* wt, const
     return launch_topk_any(workspace, nchunk, bias, T, E, k, score_fn, logits, topk_ids, topk_w,
                            prob_partial, z_partial, block_counts, stream);
   }
-  if (path == kStream || (path == kPlanes && E > 128 && E <= 256))
+  if (!plan && (path == kStream || (path == kPlanes && E > 128 && E <= 256)))
     return launch_stream(x, ld_x, wt, bias, T, d, E, k, score_fn, logits, topk_ids, topk_w,
                          prob_partial, z_partial, block_counts, stream);
   float* lbuf = logits ? logits : (workspace && workspace_bytes >= plane ? workspace : nullptr);
-  if ((path != kFused || E > 128) && lbuf && nchunk <= 16) {
+  if ((path != kFused || E > 128) && lbuf && logits_kernel_takes(d)) {
     const int ranges = logit_ranges(d);
     const dim3 grid((unsigned)ceil_div(T, kRouteBlock), (unsigned)ceil_div(E, 32));
 #define NT_LOGITS(R)                                                                       \
@@ -1719,6 +1723,7 @@ hipError_t launch_router(const uint16_t* x, int64_t ld_x, const float* wt, const
     return launch_topk_any(lbuf, 1, nullptr, T, E, k, score_fn, nullptr, topk_ids, topk_w,
                            prob_partial, z_partial, block_counts, stream);
   }
+  if (plan) return hipErrorInvalidValue;  // the kernels below write none
   if (E <= 128) {  // the fused kernel: its path, or planes / logits without their buffers
     // (the chunk-per-wave kernel where it fits, unless NT_MOE_ROUTER_MODE=fused)
     if (chunk_router_fits(d, E) && router_mode_override() != 1)

@@ -185,6 +185,57 @@ def test_router_plan_equals_router_then_route_plan(case):
     assert int(got[5].sum()) == case.T * case.k
 
 
+_MODE_CHECK = r"""
+import sys, torch
+sys.path.insert(0, sys.argv[1])
+from nexttransformer_amd import ops
+from oracle import moe_oracle as orc
+from tests.moe_cases import Case, make_router_inputs
+bits = lambda t: t.contiguous().view(torch.int32)
+for i, (T, d, E, k, score, bias) in enumerate([
+        (64, 4096, 128, 8, 0, 0), (130, 4096, 200, 6, 1, 1.2), (64, 2184, 256, 8, 0, 0),
+        (4100, 2176, 96, 2, 0, 0), (16, 4096, 32, 4, 1, 0), (700, 2048, 256, 8, 0, 0.8),
+        (300, 264, 160, 6, 1, 0), (130, 1280, 24, 3, 0, 0)]):
+    case = Case("mode", T, d, E, k, 64, score_fn=score, zipf_bias=bias, seed=40 + i)
+    print(case, flush=True)
+    x, w, b = make_router_inputs(case)
+    ref = orc.router_logits_fixed(x, w, b)
+    ref_ids = orc.topk(ref, k, score)[0]
+    args = (x.cuda(), w.t().contiguous().cuda(), None if b is None else b.cuda(), k, score)
+    for want in (False, True):
+        out = ops.router_plan(*args, want)
+        assert torch.equal(out[1].cpu(), ref_ids)
+        if want:
+            assert torch.equal(bits(out[0].cpu()), bits(ref))
+        for a, c in zip(out[2:5], ops.topk_from_logits(ref.cuda(), k, score)[1:]):
+            # the kernels differ in the order of their sums: 64 terms of one sign at most
+            torch.testing.assert_close(a, c, rtol=64 * 2.0 ** -23, atol=1e-7)
+        for a, c in zip(out[5:], ops.route_plan(out[1], out[2], E, None, False)):
+            assert torch.equal(bits(a), bits(c))
+        router = ops.router(*args, want)
+        assert torch.equal(router[1], out[1]) and torch.equal(bits(router[2]), bits(out[2]))
+print("router modes ok")
+"""
+
+
+@pytest.mark.parametrize("mode", ["fused", "split", "stream"])
+def test_forced_router_modes_write_the_plan(mode):
+    """NT_MOE_ROUTER_MODE (read once per process, so in a child process): every forced path gives
+    the oracle's logits and selection and the plan that route_plan makes of it, on both sides of
+    the 2048 features that the logits kernel takes (past them its shapes run the fused or the
+    streamed kernel) and of 128 experts; the streamed kernel with a ragged last block, a partial
+    last stage and experts that are no multiple of 32."""
+    import os
+    import subprocess
+    import sys
+    from pathlib import Path
+    root = str(Path(__file__).resolve().parents[1])
+    r = subprocess.run([sys.executable, "-c", _MODE_CHECK, root],
+                       env=dict(os.environ, NT_MOE_ROUTER_MODE=mode), capture_output=True,
+                       text=True, timeout=100)
+    assert r.returncode == 0 and "router modes ok" in r.stdout, r.stdout + r.stderr
+
+
 def test_router_plan_empty_batch():
     from nexttransformer_amd import ops
     dev = torch.device("cuda")
