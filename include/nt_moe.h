@@ -433,6 +433,16 @@ int nt_moe_combine_aux(const uint16_t* y, const int32_t* combine_dest, const flo
                        float* aux_out, nt_moe_stream_t stream);
 
 /*
+ * The backward's sum of a token's rows: out_t = first_t + sum_j y[combine_dest[t, j]] (in the
+ * order of combine_dest, in fp32, rounded to bf16 once), that is nt_moe_combine_aux's sum with
+ * every weight one (index_add's transpose of the gather, megatron_moe.py:144). y bf16 [T k, d],
+ * first bf16 [T, d] with row stride ld_first or NULL (zeros), out bf16 [T, d].
+ */
+int nt_moe_sum_rows(const uint16_t* y, const int32_t* combine_dest, int64_t T, int32_t d, int32_t k,
+                    const uint16_t* first, int64_t ld_first, uint16_t* out, int64_t ld_out,
+                    nt_moe_stream_t stream);
+
+/*
  * Backward of the layer (autograd through megatron_moe.py:137-150 and the MCore router and
  * aux losses, megatron_moe.py:43-45,95-100; the reference trains through it, e.g.
  * tests/test_megatron_moe.py:183-197). The grouped dgrad GEMMs use the forward entry points

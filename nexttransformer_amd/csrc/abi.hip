@@ -1033,6 +1033,25 @@ int nt_moe_grouped_gemm_fp8_packed(const uint8_t* a, int64_t ld_a, int64_t a_row
   return launched(err, "grouped_gemm_fp8_packed");
 }
 
+int nt_moe_sum_rows(const uint16_t* y, const int32_t* combine_dest, int64_t T, int32_t d, int32_t k,
+                    const uint16_t* first, int64_t ld_first, uint16_t* out, int64_t ld_out,
+                    nt_moe_stream_t stream) {
+  int rc = check_route_shape(T, k, NT_MOE_MAX_EXPERTS);
+  if (rc) return rc;
+  NT_REQUIRE(d > 0 && d % 8 == 0, "sum_rows: d must be a positive multiple of 8, got %d", d);
+  NT_REQUIRE(ld_out >= d && ld_out % 8 == 0, "sum_rows: ld_out must be >= d and a multiple of 8");
+  NT_REQUIRE(!first || (ld_first >= d && ld_first % 8 == 0 && aligned16(first)),
+             "sum_rows: first needs ld_first >= d, a multiple of 8, 16-byte alignment");
+  if (T == 0) return ok();
+  NT_REQUIRE(y && combine_dest && out, "sum_rows: null buffer");
+  NT_REQUIRE(aligned16(y) && aligned16(out), "sum_rows: y and out must be 16-byte aligned");
+  return launched(launch_combine_aux(y, combine_dest, nullptr, T, d, k, first, ld_first, out,
+                                     ld_out, nullptr, nullptr, nullptr, NT_MOE_MAX_EXPERTS, 0.f,
+                                     0.f, nullptr, nullptr,
+                                     reinterpret_cast<hipStream_t>(stream)),
+                  "sum_rows");
+}
+
 int nt_moe_combine_aux(const uint16_t* y, const int32_t* combine_dest, const float* combine_w,
                        int64_t T, int32_t d, int32_t k, const uint16_t* shared_y,
                        int64_t ld_shared, uint16_t* out, int64_t ld_out,

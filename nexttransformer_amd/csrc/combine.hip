@@ -23,7 +23,8 @@ namespace {
 // grid's waves, ...) and walk the items (token, chunk) in order, issuing the next item's k row
 // loads (and its shared-expert chunk) before summing the current one, so 2 (k + 1) VPC vectors
 // per lane are in flight. With `split` (batches of at most one item per SIMD) each item
-// has a wave of its own. KMAX bounds k (registers are sized by it).
+// has a wave of its own. KMAX bounds k (registers are sized by it). Without combine_w every weight
+// is one (the backward's sum of a token's input-gradient rows).
 template <int KMAX, int VPC>
 __device__ __forceinline__ void combine_rows(
     const uint16_t* __restrict__ y, const int32_t* __restrict__ combine_dest,
@@ -41,7 +42,7 @@ __device__ __forceinline__ void combine_rows(
     w = 0.f;
     if (lane < k && t < T) {
       dest = combine_dest[t * k + lane];
-      w = combine_w[t * k + lane];
+      w = combine_w ? combine_w[t * k + lane] : 1.f;
       dest = dest < 0 ? 0 : (dest >= A ? (int)(A - 1) : dest);
     }
   };

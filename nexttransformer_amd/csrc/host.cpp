@@ -246,9 +246,9 @@ PyObject* forward(PyObject*, PyObject* const* argv, Py_ssize_t argc) {
 
 // backward(g, grad_aux | None, x, w1_t packed, w2_t packed, shared_w2_t packed | None, first,
 //          fc1, h, perm_w, src_row, offsets, combine_dest, ids, weights, logits, counts,
-//          prob_partial, z_partial, shared_fc1 | None, shared_h | None, unit, segment, Fs, Ep,
-//          activation, score_fn, aux_coeff, z_coeff, splits of dW1, dW2, the router's and the
-//          shared expert's two, weight gradients fp32, stream)
+//          shared_fc1 | None, shared_h | None, segment, Fs, Ep, activation, score_fn, aux_coeff,
+//          z_coeff, splits of dW1, dW2, the router's and the shared expert's two, weight gradients
+//          fp32, stream)
 // -> (dx, d router, dW1, dW2, shared dW1 | None, shared dW2 | None)
 PyObject* backward(PyObject*, PyObject* const* argv, Py_ssize_t argc) {
   HANDLE_TH_ERRORS
@@ -260,9 +260,9 @@ PyObject* backward(PyObject*, PyObject* const* argv, Py_ssize_t argc) {
   const Tensor fc1 = a.whole(BF, 2), h = a.whole(BF, 2), perm_w = a.whole(F, 1),
                src = a.whole(I, 1), offsets = a.whole(I, 1), cdest = a.whole(I, 2),
                ids = a.whole(I, 2), w = a.whole(F, 2), logits = a.whole(F, 2),
-               counts = a.whole(I, 1), pp = a.whole(F, 2), zp = a.whole(F, 1);
+               counts = a.whole(I, 1);
   const Tensor fc1s = a.whole(BF, 2, true), hs = a.whole(BF, 2, true);
-  const Tensor unit = a.whole(F, 2), seg = a.whole(I, 1);
+  const Tensor seg = a.whole(I, 1);
   const int64_t Fs = a.integer(), Ep = a.integer(), act = a.integer(), score = a.integer();
   const double aux_coeff = a.number(), z_coeff = a.number();
   const int64_t n1 = a.integer(), n2 = a.integer(), nr = a.integer(), ns1 = a.integer(),
@@ -279,8 +279,7 @@ PyObject* backward(PyObject*, PyObject* const* argv, Py_ssize_t argc) {
       !is(w1t, {E, d, F1}) || !is(w2t, {E, H, d}) || F1 != halves * H || !is(fc1, {A, F1}) ||
       !is(h, {A, H}) || !is(perm_w, {A}) || !is(src, {A}) || !is(offsets, {E + 1}) ||
       !is(cdest, {T, k}) || !is(ids, {T, k}) || !is(w, {T, k}) || !is(logits, {T, E}) ||
-      !is(counts, {E}) || !is(pp, {route_blocks(T), E}) || !is(zp, {route_blocks(T)}) ||
-      !is(unit, {T, k}) || !is(seg, {2}) || !is(first_w, {1, d, Kc}) || sh != fc1s.defined() ||
+      !is(counts, {E}) || !is(seg, {2}) || !is(first_w, {1, d, Kc}) || sh != fc1s.defined() ||
       sh != hs.defined() || Kc < Fs + 3 * Ep || Ep < E || n1 < 1 || n2 < 1 || nr < 1 || ns1 < 1 ||
       ns2 < 1)
     Py_RETURN_NONE;
@@ -353,11 +352,10 @@ PyObject* backward(PyObject*, PyObject* const* argv, Py_ssize_t argc) {
     };
     Tensor wr = wgrad(bf(cat) + Fs + Ep, Kc, 2 * Ep, x, nr, true)[0];
     Tensor d_router = at::add(wr.narrow(0, 0, E), wr.narrow(0, Ep, E));
-    Tensor dx = mk({T, d}, BF), unused = mk({3}, F);
-    must(nt_moe_combine_aux(bf(dxp), i32(cdest), f32(unit), T, (int32_t)d, (int32_t)k, bf(first), d,
-                            bfw(dx), d, f32(pp), f32(zp), i32(counts), (int32_t)E, 0.f, 0.f,
-                            f32(unused), st),
-         "ntmoe::combine_aux");
+    Tensor dx = mk({T, d}, BF);
+    must(nt_moe_sum_rows(bf(dxp), i32(cdest), T, (int32_t)d, (int32_t)k, bf(first), d, bfw(dx), d,
+                         st),
+         "ntmoe::sum_rows");
     const auto wt = wide ? F : BF;
     Tensor dw1 = mk({E, F1, d}, wt), dw2 = mk({E, d, H}, wt), partial;
     const int64_t p1 = n1 > 1 ? n1 * F1 : 0, p2 = n2 > 1 ? n2 * H : 0;

@@ -759,6 +759,34 @@ def _(y, combine_dest, combine_w, shared_y, prob_partial, z_partial, counts, aux
     return y.new_empty((T, y.shape[1])), y.new_empty((3,), dtype=torch.float32)
 
 
+@_custom_op("ntmoe::sum_rows")
+def sum_rows(y: Tensor, combine_dest: Tensor, first: Optional[Tensor]) -> Tensor:
+    """out [T, d] bf16 = first + the token's rows y[combine_dest[t]], summed as combine_aux does
+    with every weight one."""
+    _on_gpu(y, combine_dest, first)
+    _require(y.dtype == torch.bfloat16 and y.dim() == 2 and y.is_contiguous(),
+             "sum_rows: y must be contiguous bf16 [T*k, d]")
+    _require(combine_dest.dtype == torch.int32 and combine_dest.dim() == 2
+             and combine_dest.is_contiguous(), "sum_rows: combine_dest must be contiguous int32 [T, k]")
+    T, k = combine_dest.shape
+    d = y.shape[1]
+    _require(y.shape[0] == T * k, "sum_rows: y must have T*k rows")
+    if first is not None:
+        _require(first.dtype == torch.bfloat16 and first.shape == (T, d) and first.stride(1) == 1,
+                 "sum_rows: first must be bf16 [T, d]")
+    out = torch.empty(T, d, device=y.device, dtype=torch.bfloat16)
+    st = nat.load().nt_moe_sum_rows(ptr(y), ptr(combine_dest), T, d, k, ptr(first),
+                                    first.stride(0) if first is not None else 0, ptr(out),
+                                    out.stride(0), _stream(y.device))
+    nat.check(st, "ntmoe::sum_rows")
+    return out
+
+
+@sum_rows.register_fake
+def _(y, combine_dest, first):
+    return y.new_empty((combine_dest.shape[0], y.shape[1]))
+
+
 # ---------------------------------------------------------------------------------------------
 # the whole layer
 
@@ -1381,21 +1409,6 @@ def backward_weights(w1, w2, shared_w1=None, shared_w2=None, w_router_t=None, **
     return BackwardWeights(w1, w2, shared_w1, shared_w2, w_router_t, **transposes)
 
 
-_unit_cache = {}
-
-
-def _unit_weights(T, k, device):
-    """Cached fp32 ones [T, k] (the unit combine weights of the input-gradient sum), read only;
-    a fill kernel less per backward. Holds the last few shapes."""
-    key = (T, k, device)
-    t = _unit_cache.get(key)
-    if t is None:
-        if len(_unit_cache) >= 8:
-            _unit_cache.clear()
-        t = _unit_cache[key] = torch.ones(T, k, device=device, dtype=torch.float32)
-    return t
-
-
 def _native_backward(g, grad_aux, x, w_router_t, bw, state, top_k, score_fn, activation,
                      aux_coeff, z_coeff, weight_grads_fp32):
     """moe_backward with packed dgrad weights and kept pre-activations through the native host
@@ -1414,8 +1427,7 @@ def _native_backward(g, grad_aux, x, w_router_t, bw, state, top_k, score_fn, act
     r = _native_call(nat.host().backward, (
         g, grad_aux, x, bw.w1t.w, bw.w2t.w, bw.shared["w2t"].w if sh else None, wf, fc1, h,
         state["perm_w"], state["src_row"], state["offsets"], state["combine_dest"], state["ids"],
-        state["weights"], state["logits"], state["counts"], state["prob_partial"],
-        state["z_partial"], fc1s if sh else None, hs, _unit_weights(T, top_k, dev),
+        state["weights"], state["logits"], state["counts"], fc1s if sh else None, hs,
         _whole_batch_segment(T, dev), Fs, Ep, activation, score_fn, aux_coeff, z_coeff,
         wgrad_splits(E, fc1.shape[1], d, rows, dev), wgrad_splits(E, d, h.shape[1], rows, dev),
         wgrad_splits(1, 2 * Ep, d, T, dev), wgrad_splits(1, Fs, d, T, dev) if sh else 1,
@@ -1440,8 +1452,7 @@ def moe_backward(grad_out, grad_aux, x, w_router_t, bw, state, *, top_k,
     the dgrad of both projections (grouped GEMMs; the down projection's on the output gradient's
     gathered rows, before the routing weight), the activation backward with the routing weight and
     its gradient (act_bwd_rows), the router backward (routing-weight, load-balance and
-    z-loss terms), the token-side sum of the k input-gradient rows (the forward's combine kernel
-    with unit weights; its first row, the shared expert's input gradient plus the router's,
+    z-loss terms), the token-side sum of the k input-gradient rows (sum_rows; its first row, the shared expert's input gradient plus the router's,
     grad_logits . Wr, comes from one grouped GEMM over the concatenated K of BackwardWeights'
     `first` operand), and every weight gradient on the grouped_wgrad kernels: g^T (w h) and d_fc1^T x over each
     expert's rows (g and x gathered through src_row), the shared expert's over all T rows and the
@@ -1512,9 +1523,7 @@ def moe_backward(grad_out, grad_aux, x, w_router_t, bw, state, *, top_k,
     wr = grouped_wgrad.raw(g_cat, x, None, seg, T, wgrad_splits(1, 2 * Ep, d, T, x.device), True)[0]
     res["router"] = wr[:E] + wr[Ep:Ep + E]
     mark("router_bwd")
-    res["x"], _ = combine_aux.raw(dxp, cdest, _unit_weights(T, k, x.device), first,
-                                  state["prob_partial"], state["z_partial"], state["counts"],
-                                  0.0, 0.0)
+    res["x"] = sum_rows.raw(dxp, cdest, first)
     mark("dx_sum")
     # expert weight gradients over each expert's rows; the shared expert's over all T rows
     f32 = weight_grads_fp32

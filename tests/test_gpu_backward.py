@@ -691,3 +691,57 @@ def test_router_bwd_rows_equal_slot_order(T, E, k, score_fn):
     aux = torch.tensor([0.5, 1.0, 2.0]).cuda()
     got = ops.router_bwd_rows(logits, ids, w, rows, dest, counts, score_fn, aux, 0.01, 0.001)
     assert torch.equal(got, ops.router_bwd(logits, ids, w, slots, counts, score_fn, aux, 0.01, 0.001))
+
+
+@pytest.mark.parametrize("T,k,d", [(1, 1, 8), (3, 8, 1280), (300, 2, 1800), (513, 3, 2048),
+                                   (2100, 8, 1024)])
+@pytest.mark.parametrize("first", [False, True])
+def test_sum_rows_is_the_combine_with_unit_weights(T, k, d, first):
+    """Bit for bit, on both sides of the line between a wave per chunk and a wave per token, with
+    rows of one- and two-vector chunks and a first row of a wider matrix."""
+    from nexttransformer_amd import ops
+    g = torch.Generator().manual_seed(T + d)
+    y = torch.randn(T * k, d, generator=g).to(torch.bfloat16).cuda()
+    dest = torch.randperm(T * k, generator=g).int().view(T, k).cuda()
+    f = torch.randn(T, d + 8, generator=g).to(torch.bfloat16).cuda()[:, :d] if first else None
+    one = lambda *s: torch.ones(s, device="cuda")
+    counts = torch.ones(8, device="cuda", dtype=torch.int32)
+    nblk = (T + 63) // 64
+    ref, _ = ops.combine_aux(y, dest, one(T, k), f, one(nblk, 8), one(nblk), counts, 0.0, 0.0)
+    assert torch.equal(ops.sum_rows(y, dest, f), ref)
+
+
+@pytest.mark.parametrize("through_ops", [False, True])
+def test_backward_on_a_second_stream_needs_nothing_of_the_first(through_ops):
+    """Two backward passes of a batch size not seen before, on two streams, the first one's work
+    queued behind a long product: the second, which starts at once, reads nothing that the first
+    has yet to write."""
+    from nexttransformer_amd import ops
+    E, k, d, H = 8, 2, 256, 256
+    g = torch.Generator().manual_seed(5)
+    mk = lambda *s, std=0.05: (torch.randn(s, generator=g) * std).cuda()
+    w1, w2, wr = mk(E, 2 * H, d).bfloat16(), mk(E, d, H).bfloat16(), mk(d, E)
+    p1, p2 = ops.pack_expert_weights(w1, 0), ops.pack_expert_weights(w2, 2)
+    bw = ops.backward_weights(w1, w2, None, None, wr)
+    mark = dict(mark=lambda name: None) if through_ops else {}
+
+    def case(T):
+        x, go = mk(T, d, std=1.0).bfloat16(), mk(T, d, std=1.0).bfloat16()
+        state = ops.moe_forward(x, wr, p1, p2, top_k=k, packed=True, want_logits=True, keep=True)[2]
+        return lambda: ops.moe_backward(go, None, x, wr, bw, state, top_k=k, **mark)
+
+    case(77)()  # the weights' operands
+    run = case(1013 if through_ops else 1021)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    big = mk(8192, 8192)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(a):
+        for _ in range(20):
+            big @ big
+        ga = run()
+    with torch.cuda.stream(b):
+        gb = run()
+    torch.cuda.synchronize()
+    ref = run()
+    for n, t in ref.items():
+        assert t is None or (torch.equal(t, ga[n]) and torch.equal(t, gb[n])), n
