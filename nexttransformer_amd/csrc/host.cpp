@@ -143,9 +143,8 @@ int64_t route_blocks(int64_t T) { return (T + NT_MOE_ROUTE_BLOCK - 1) / NT_MOE_R
 
 // forward(x, w_router_t, bias | None, w1, w2, shared_w1 | None, shared_w2 | None, segment | None,
 //         top_k, score_fn, up_epilogue, aux_coeff, z_coeff, want_logits, keep, stream)
-// -> (out, aux, logits, ids, weights, prob_partial, z_partial, counts, offsets, src_row, perm_w,
-//     combine_dest, combine_w, load, h, y, fc1, shared_h, shared_fc1); the last five None without
-//     keep. load: counts as int64.
+// -> (out, aux, logits, ids, weights, counts, offsets, src_row, perm_w, combine_dest, combine_w,
+//     load, h, fc1, shared_h, shared_fc1); the last four None without keep. load: counts as int64.
 PyObject* forward(PyObject*, PyObject* const* argv, Py_ssize_t argc) {
   HANDLE_TH_ERRORS
   constexpr auto BF = at::kBFloat16, F = at::kFloat, I = at::kInt;
@@ -234,9 +233,9 @@ PyObject* forward(PyObject*, PyObject* const* argv, Py_ssize_t argc) {
                                  i32(counts), (int32_t)E, (float)aux_coeff, (float)z_coeff,
                                  f32(aux), static_cast<int64_t*>(load.data_ptr()), st),
          "ntmoe::combine_aux");
-    r = {out, aux, logits, ids, w, pp, zp, counts, offsets, src, perm_w, cdest, cw, load};
-    if (keep) r.insert(r.end(), {h, y, fc1, hs, fc1s});
-    else r.resize(19);
+    r = {out, aux, logits, ids, w, counts, offsets, src, perm_w, cdest, cw, load};
+    if (keep) r.insert(r.end(), {h, fc1, hs, fc1s});
+    else r.resize(16);
   } catch (const Failed& f) {
     return failed(f);
   }

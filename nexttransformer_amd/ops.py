@@ -817,13 +817,12 @@ def _native_forward(x, w_router_t, w1, w2, top_k, score_fn, activation, aux_coef
         want_logits, keep), x.device)
     if r is None:
         return None
-    (out, aux, logits, ids, w, pp, zp, counts, offsets, src, perm_w, cdest, cw, load, h, y, fc1,
-     hs, fc1s) = r
+    (out, aux, logits, ids, w, counts, offsets, src, perm_w, cdest, cw, load, h, fc1, hs,
+     fc1s) = r
     state = dict(logits=logits, ids=ids, weights=w, counts=counts, offsets=offsets, src_row=src,
                  perm_w=perm_w, combine_dest=cdest, combine_w=cw, load=load)
     if keep:
-        state.update(h=h, y=y, shared_h=hs, prob_partial=pp, z_partial=zp, fc1=fc1,
-                     shared_fc1=fc1s)
+        state.update(h=h, shared_h=hs, fc1=fc1, shared_fc1=fc1s)
     return out, aux, state
 
 
@@ -848,10 +847,11 @@ def moe_forward(x, w_router_t, w1, w2, *, top_k, score_fn=nat.SCORE_SOFTMAX,
     h are then quantised per row and both projections run on the fp8 grouped GEMM.
     `mark(name)`, when given, is called after each stage is enqueued (used to place timing
     events on the stream; without permute_rows the router and the route plan are one call, so
-    the "router" stage holds both and "route_plan" is empty). keep (bf16 experts): the state also holds what moe_backward reads
-    (h, the shared expert's h; also y, the router's aux partials and the fc1 pre-activations of
-    the routed and the shared expert from their up projections' launches, with packed weights
-    or plain ones that plain_keep_supported takes; otherwise moe_backward recomputes them).
+    the "router" stage holds both and "route_plan" is empty). keep (bf16 experts): the state also
+    holds what moe_backward reads (h, the shared expert's h and the fc1 pre-activations of the
+    routed and the shared expert from their up projections' launches, with packed weights or
+    plain ones that plain_keep_supported takes; otherwise moe_backward recomputes them). The
+    down projection's rows y are not among them: their block is free once the combine ran.
     """
     T = x.shape[0]
     E = w_router_t.shape[1]
@@ -963,8 +963,7 @@ def moe_forward(x, w_router_t, w1, w2, *, top_k, score_fn=nat.SCORE_SOFTMAX,
     state = dict(logits=logits, ids=ids, weights=w, counts=counts, offsets=offsets, src_row=src,
                  perm_w=perm_w, combine_dest=cdest, combine_w=cw, load=load)
     if keep:
-        state.update(h=h, y=y, shared_h=hs, prob_partial=pp, z_partial=zp, fc1=fc1,
-                     shared_fc1=fc1s)
+        state.update(h=h, shared_h=hs, fc1=fc1, shared_fc1=fc1s)
     return out, aux, state
 
 

@@ -745,3 +745,26 @@ def test_backward_on_a_second_stream_needs_nothing_of_the_first(through_ops):
     ref = run()
     for n, t in ref.items():
         assert t is None or (torch.equal(t, ga[n]) and torch.equal(t, gb[n])), n
+
+
+@pytest.mark.parametrize("through_ops", [False, True])
+def test_forward_for_training_keeps_only_what_the_backward_reads(through_ops):
+    """Memory held between forward and backward: the outputs, h, the pre-activations and the
+    routing tensors, not the down projection's [T k, d] rows (which nothing reads again)."""
+    from nexttransformer_amd import ops
+    T, E, k, d, H = 1024, 8, 4, 1024, 256
+    g = torch.Generator().manual_seed(6)
+    mk = lambda *s, std=0.05: (torch.randn(s, generator=g) * std).cuda()
+    p1 = ops.pack_expert_weights(mk(E, 2 * H, d).bfloat16(), 0)
+    p2 = ops.pack_expert_weights(mk(E, d, H).bfloat16(), 2)
+    x, wr = mk(T, d, std=1.0).bfloat16(), mk(d, E)
+    mark = dict(mark=lambda name: None) if through_ops else {}
+    call = lambda: ops.moe_forward(x, wr, p1, p2, top_k=k, packed=True, want_logits=True,
+                                   keep=True, **mark)
+    call()
+    before = torch.cuda.memory_allocated()
+    out, aux, state = call()
+    held = torch.cuda.memory_allocated() - before
+    kept = 2 * (T * d + T * k * H + T * k * 2 * H) + 4 * (T * E + 8 * T * k)
+    assert held <= kept + (1 << 17), (held, kept)  # (small tensors are rounded up to 512 bytes)
+    assert not any(t is not None and t.shape == (T * k, d) for t in state.values())
