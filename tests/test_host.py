@@ -47,6 +47,20 @@ def test_library_exports_every_declared_symbol(lib):
     assert lib.nt_moe_abi_version() == 1
 
 
+def test_host_module_has_no_thread_local_storage():
+    """A module with a thread-local block that no thread ever touches slows every thread-local
+    access of the process (glibc before 2.39 looks the block up anew each time): no PT_TLS program
+    header in nt_moe_host.so."""
+    import struct
+    from nexttransformer_amd import _native as nat
+    nat.host()
+    elf = nat.LIB_PATH.with_name("nt_moe_host.so").read_bytes()
+    assert elf[:6] == b"\x7fELF\x02\x01"
+    at, size, n = struct.unpack_from("<Q", elf, 32)[0], *struct.unpack_from("<HH", elf, 54)
+    kinds = [struct.unpack_from("<I", elf, at + i * size)[0] for i in range(n)]
+    assert 1 in kinds and 7 not in kinds  # PT_LOAD, PT_TLS
+
+
 def test_header_constants_match_binding():
     from nexttransformer_amd import _native as nat
     text = HEADER.read_text()
