@@ -7,22 +7,23 @@
 // had one K step of weights in flight per wave, eight or sixteen workgroups in all for one token
 // or for the shared expert alone, and a tile list to scan before the first load. Here:
 //   * one workgroup per (segment, 128 packed weight rows): it reads two offsets and leaves if the
-//     segment is empty; nothing is scanned. A segment of more than 128 rows is dealt, in even
-//     chunks of whole 32-row blocks, to the kSplitM workgroups of its weight rows;
+//     segment is empty; nothing is scanned. A segment of more than 128 rows is cut into even chunks
+//     of whole 32-row blocks: its workgroup takes the first one, and the others have workgroups at
+//     the front of the grid, which find theirs by a scan of the offsets;
 //   * wave w streams packed block w of the tile (4 KB per 64-wide K step) into a register ring,
 //     D steps ahead: 6, 4 or 2 for chunks of 32, 64 and 128 rows, as the accumulators allow;
 //   * the chunk's token rows go through LDS in a ring of the same depth (direct-to-LDS copies,
 //     16-byte chunks XOR-swizzled by row), one barrier per step;
 //   * the outputs are transposed through that LDS, so stores write whole row segments.
-// The shared expert is one more range of workgroups ahead of the routed ones (its rows are the
+// The shared expert is one more range of workgroups ahead of the segments' (its rows are the
 // batch, no gather; its widths may differ), so its few tiles overlap the routed weight stream
 // instead of taking two launches on a few CUs.
 //
 // Measured, us up / down, that kernel -> this one (weights not in any cache): T3 cell (256
 // experts, d 1280, H 320) 48 tokens 43 / 35 -> 31 / 29, 512 tokens 46 / 51 -> 40 / 40; 128 experts
 // d 2048 H 768, 48 tokens 146 / 75 -> 134 / 69 (6.0 TB/s), 777 tokens 153 / 87 -> 146 / 85; 32
-// experts d 1024 H 512, 48 tokens 18 / 12 -> 14 / 9. Whole forward at 48 tokens, T3 cell: see the
-// dispatch rule (few_rows).
+// experts d 1024 H 512, 48 tokens 18 / 12 -> 14 / 9. Whole forward at 48 tokens, T3 cell (with the
+// shared expert in the same launches): 185 -> 104 us of GPU time.
 #include <math.h>
 
 #include "common.h"
@@ -216,51 +217,99 @@ __host__ __device__ inline int few_n_tiles(int n_out, int epilogue) {
 // 8's, so the workgroups that read the same token rows share an L2 (777 tokens over 128 experts:
 // up 186 -> 146 us, down 108 -> 85 us); with fewer segments spread = 1: the whole chip takes
 // each one's weight rows.
+// The first tail_blocks workgroups each take one chunk past the first of a segment that has more
+// than one (routing that favours a few experts), weight rows fastest, an eighth of that list per
+// XCD; without such segments they read the offsets and leave. With the segment's own workgroups
+// walking them, 8192 rows of one of 256 experts (K 1280, 320 outputs) took 775 us and 8 x 1024 rows
+// 102; this way both take 21 (the tiled kernel 27), and 32 rows of every expert 46 (45; tiled 54).
+// At the end of the grid they cost the even case 1 us less and the uneven ones up to a quarter more
+// (32 experts, K 1024, 4 x 256 rows: 17.5 us there, 13.9 here, tiled 16.3). One chunk each and no
+// loop: the state of a loop around the tile spills.
 template <int EPI, bool KEEP>
 __global__ __launch_bounds__(256, 3) void few_gemm_kernel(FewPart routed,
                                                           const int32_t* __restrict__ seg_offsets,
-                                                          int S, int total_rows, int split_m,
-                                                          int spread,
+                                                          int S, int total_rows, int spread,
                                                           FewPart shared, int shared_rows,
-                                                          int shared_blocks) {
+                                                          int shared_blocks, int tail_blocks) {
   extern __shared__ __align__(16) unsigned char smem[];
-  int b = blockIdx.x;
-  const bool is_shared = b < shared_blocks;
+  const int tail = (int)blockIdx.x < tail_blocks ? (int)blockIdx.x : -1;
+  int b = (int)blockIdx.x - tail_blocks;
+  const bool is_shared = tail < 0 && b < shared_blocks;
   const FewPart& p = is_shared ? shared : routed;
   const int n_tiles = few_n_tiles(p.n_out, EPI);
-  const uint16_t* w = p.w;
-  int lo, hi, chunk, chunks_by;  // rows, this workgroup's first chunk and its step
+  auto clamped = [&](int o) { return o < 0 ? 0 : (o > total_rows ? total_rows : o); };
+  int s = 0, lo = 0, hi = shared_rows, chunk = 0, chunks, nt;
   if (is_shared) {
-    lo = 0;
-    hi = shared_rows;
     chunk = b / n_tiles;
-    chunks_by = shared_blocks / n_tiles;
-  } else {
+    nt = b % n_tiles;
+    chunks = (hi + kMaxRows - 1) / kMaxRows;
+  } else if (tail < 0) {
     b -= shared_blocks;
     const int first = b % spread;
     b /= spread;
-    const int sc = b / n_tiles, s = sc / split_m * spread + first;
+    s = b / n_tiles * spread + first;
+    nt = b % n_tiles;
     if (s >= S) return;
-    chunk = sc % split_m;
-    chunks_by = split_m;
-    lo = seg_offsets[s];
-    hi = seg_offsets[s + 1];
-    lo = lo < 0 ? 0 : (lo > total_rows ? total_rows : lo);
-    hi = hi < lo ? lo : (hi > total_rows ? total_rows : hi);
-    w += (int64_t)s * (EPI == NT_MOE_EPI_SWIGLU ? 2 : 1) * p.n_out * p.K;
+    lo = clamped(seg_offsets[s]);
+    hi = clamped(seg_offsets[s + 1]);
+    if (hi <= lo) return;
+    chunks = (hi - lo + kMaxRows - 1) / kMaxRows;
+  } else {
+    // Lane l holds segments per l .. per l + per - 1: their chunks past the first, added up over
+    // the lanes; the lane whose share holds the item's chunk finds it among its segments.
+    constexpr int kPer = (NT_MOE_MAX_SEGMENTS + 63) / 64;
+    const int per = (S + 63) / 64, lane = lane_id();
+    int off[kPer + 1], sum = 0;
+#pragma unroll
+    for (int i = 0; i <= kPer; ++i) {
+      const int at = lane * per + i;
+      off[i] = i <= per ? clamped(seg_offsets[at < S ? at : S]) : 0;
+    }
+    auto later = [&](int i) {
+      return i < per && off[i + 1] > off[i] ? (off[i + 1] - off[i] - 1) / kMaxRows : 0;
+    };
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) sum += later(i);
+    int incl = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int u = __shfl_up(incl, o);
+      if (lane >= o) incl += u;
+    }
+    const int64_t all = (int64_t)__builtin_amdgcn_readlane(incl, 63) * n_tiles;
+    const int64_t item = all * (tail % 8) / 8 + tail / 8;
+    if (item >= all * (tail % 8 + 1) / 8) return;
+    const int at = (int)(item / n_tiles);
+    nt = (int)(item % n_tiles);
+    const int k = __builtin_ctzll(__ballot(at < incl));
+    int r = at - (incl - sum), fs = 0, fl = 0, fh = 0, fc = 0, fn = 1;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int n = later(i);
+      if (r >= 0 && r < n) {
+        fs = lane * per + i;
+        fl = off[i];
+        fh = off[i + 1];
+        fc = r + 1;
+        fn = n + 1;
+      }
+      r -= n;
+    }
+    s = __builtin_amdgcn_readlane(fs, k);
+    lo = __builtin_amdgcn_readlane(fl, k);
+    hi = __builtin_amdgcn_readlane(fh, k);
+    chunk = __builtin_amdgcn_readlane(fc, k);
+    chunks = __builtin_amdgcn_readlane(fn, k);
   }
-  const int nt = b % n_tiles;
-  const int blocks = (hi - lo + 31) / 32, chunks = (hi - lo + kMaxRows - 1) / kMaxRows;
-  for (; chunk < chunks; chunk += chunks_by) {
-    const int m0 = lo + 32 * (int)((int64_t)blocks * chunk / chunks);
-    const int end = lo + 32 * (int)((int64_t)blocks * (chunk + 1) / chunks);
-    const int m_end = end < hi ? end : hi;
-    const int rows = m_end - m0;
-    if (rows > 64) few_tile<EPI, KEEP, 4>(p, w, smem, nt, m0, m_end);
-    else if (rows > 32) few_tile<EPI, KEEP, 2>(p, w, smem, nt, m0, m_end);
-    else few_tile<EPI, KEEP, 1>(p, w, smem, nt, m0, m_end);
-    __syncthreads();  // the next chunk's copies reuse the LDS
-  }
+  const uint16_t* w = p.w + (int64_t)s * (EPI == NT_MOE_EPI_SWIGLU ? 2 : 1) * p.n_out * p.K;
+  const int blocks = (hi - lo + 31) / 32;
+  const int m0 = lo + 32 * (int)((int64_t)blocks * chunk / chunks);
+  const int end = lo + 32 * (int)((int64_t)blocks * (chunk + 1) / chunks);
+  const int m_end = end < hi ? end : hi;
+  const int rows = m_end - m0;
+  if (rows > 64) few_tile<EPI, KEEP, 4>(p, w, smem, nt, m0, m_end);
+  else if (rows > 32) few_tile<EPI, KEEP, 2>(p, w, smem, nt, m0, m_end);
+  else few_tile<EPI, KEEP, 1>(p, w, smem, nt, m0, m_end);
 }
 
 constexpr size_t few_lds() {
@@ -273,20 +322,20 @@ static_assert(few_lds() >= (size_t)kMaxRows * 256 && few_lds() >= 32u * kRowByte
 template <int EPI, bool KEEP>
 hipError_t launch_few(const FewPart& routed, const int32_t* seg_offsets, int S, int64_t total_rows,
                       const FewPart* shared, int64_t shared_rows, hipStream_t stream) {
-  // Workgroups per (segment, weight rows): enough for a segment of four times the mean.
-  const int64_t mean = (total_rows + S - 1) / S;
-  const int64_t want = (4 * mean + kMaxRows - 1) / kMaxRows;
-  const int split_m = (int)(want > 4 ? 4 : want);
+  const int n_tiles = few_n_tiles(routed.n_out, EPI);
   const int64_t sh = shared && shared_rows > 0
                          ? (shared_rows + kMaxRows - 1) / kMaxRows * few_n_tiles(shared->n_out, EPI)
                          : 0;
   const int spread = S >= 8 ? 8 : 1;
-  const int64_t grid =
-      sh + ((int64_t)S + spread - 1) / spread * spread * few_n_tiles(routed.n_out, EPI) * split_m;
+  // A workgroup for every chunk past the first that there can be (the segments' rows are not known
+  // here): n segments of r rows in all have at most (r - 1) / kMaxRows of them.
+  const int64_t tail = ((total_rows - 1) / kMaxRows * n_tiles + 7) / 8 * 8;
+  const int64_t grid = sh + ((int64_t)S + spread - 1) / spread * spread * n_tiles + tail;
   if (grid >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
   auto kern = few_gemm_kernel<EPI, KEEP>;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), few_lds(), stream, routed, seg_offsets,
-                     S, (int)total_rows, split_m, spread, shared ? *shared : routed, (int)shared_rows, (int)sh);
+                     S, (int)total_rows, spread, shared ? *shared : routed, (int)shared_rows,
+                     (int)sh, (int)tail);
   return hipGetLastError();
 }
 

@@ -451,3 +451,82 @@ def test_shared_segment_equals_two_products(counts, tail, K, n_out, T, epilogue,
             ref = ops.grouped_gemm_packed(a, src, off, pw, epilogue, rows)
             ref_s = ops.grouped_gemm_packed(xs, None, seg, pws, epilogue, T)
         assert torch.equal(c[:used], ref[:used]) and torch.equal(cs, ref_s)
+
+
+def _uneven(S, long, total):
+    """Segment counts: the given long segments by index, the other rows two to a segment."""
+    counts = [long.get(i, 0) for i in range(S)]
+    left, i = total - sum(counts), 0
+    while left > 0:
+        if i not in long:
+            counts[i] += min(2, left)
+            left -= 2
+        i = (i + 3) % S
+    return counts
+
+
+# within the rule's 32 rows per segment on average: one segment with nearly all rows, first, last
+# and in the middle; several long ones around the 128-row chunk; the segment counts at the edges of
+# the workgroups' order (7, 8, 9) and of the lanes' shares (64, 65, 512)
+@pytest.mark.parametrize("S,long", [(7, {0: 129}), (8, {7: 200}), (9, {4: 257, 8: 25}),
+                                    (64, {0: 2048}), (64, {63: 1921}), (65, {31: 128, 32: 129, 64: 255, 1: 385}),
+                                    (130, {0: 300, 2: 300, 3: 300, 129: 300, 65: 640}),
+                                    (512, {511: 4000, 0: 130, 8: 129, 15: 1000, 16: 128, 300: 7000})],
+                         ids=str)
+@pytest.mark.parametrize("epilogue", [0, 1, 2], ids=["swiglu", "relu2", "none"])
+@pytest.mark.parametrize("gather", [False, True])
+def test_few_rows_with_long_segments_equal_the_tiled_kernel(S, long, epilogue, gather):
+    """Bit for bit, every row: the chunks past a segment's first are dealt to workgroups of their
+    own, with and without the shared expert in the launch."""
+    from nexttransformer_amd import _native as nat
+    from nexttransformer_amd import ops
+    K, n_out, T = 256, 192, 150  # (SwiGLU three and the others one and a half tiles of weight rows)
+    g = torch.Generator().manual_seed(S + epilogue)
+    counts = _uneven(S, long, min(32 * S, sum(long.values()) + S))
+    f = 2 if epilogue == nat.EPI_SWIGLU else 1
+    rows = sum(counts)
+    assert rows <= 32 * S
+    off = torch.tensor([0] + counts).cumsum(0).to(torch.int32).cuda()
+    mk = lambda *s: torch.randn(s, generator=g).to(torch.bfloat16).cuda()
+    a = mk(T if gather else rows, K)
+    src = torch.randint(0, T, (rows,), generator=g, dtype=torch.int32).cuda() if gather else None
+    w, ws, xs = mk(S, f * n_out, K), mk(1, f * n_out, K), mk(T, K)
+    pw, pws = ops.pack_expert_weights(w, epilogue), ops.pack_expert_weights(ws, epilogue)
+    ref = ops.grouped_gemm(a, src, off, w, epilogue, rows)
+    assert torch.equal(ops.grouped_gemm_packed(a, src, off, pw, epilogue, rows), ref)
+    keep = epilogue != nat.EPI_NONE
+    c, pre, cs, _ = ops.grouped_gemm_packed_shared(a, src, off, pw, epilogue, rows, xs, pws, keep)
+    assert torch.equal(c, ref)
+    seg = torch.tensor([0, T], dtype=torch.int32).cuda()
+    assert torch.equal(cs, ops.grouped_gemm(xs, None, seg, ws, epilogue, T))
+    if keep:
+        assert torch.equal(pre, ops.grouped_gemm_keep(a, src, off, w, epilogue, rows)[1])
+
+
+def test_few_rows_of_one_expert_take_no_longer_than_of_all():
+    """All rows of a batch in one of 256 experts read one expert's weights instead of 256 and
+    spread over the chip: no slower than four times the even batch (half as long when measured;
+    sixteen times as long where one workgroup per weight rows walks them)."""
+    from nexttransformer_amd import ops
+    S, K, n_out, rows = 256, 1280, 320, 8192
+    a = torch.randn(rows, K, device="cuda").to(torch.bfloat16)
+    w = ops.pack_expert_weights((torch.randn(S, n_out, K, device="cuda") * 0.05).to(torch.bfloat16), 2)
+    even = torch.arange(0, rows + 1, rows // S, dtype=torch.int32, device="cuda")
+    one = torch.full_like(even, rows)
+    one[0] = 0
+
+    def us(off):
+        times = []
+        for _ in range(7):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            torch.cuda.synchronize()
+            start.record()
+            for _ in range(10):
+                ops.grouped_gemm_packed(a, None, off, w, 2, rows)
+            end.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(end) * 100)
+        return sorted(times)[3]
+
+    us(even)
+    assert us(one) <= 4 * us(even)
