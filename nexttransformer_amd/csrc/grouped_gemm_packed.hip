@@ -851,6 +851,7 @@ static bool packed_edge(int K, int n_out, int epilogue) {
 // the extreme; 169 -> 165, 54 -> 55), but for the 128-expert down projection with all 6216 rows
 // in 8 or 16 experts (32 -> 36 and 33 -> 38).
 static bool few_rows(int num_segments, int64_t total_rows, int K, int n_out, int epilogue) {
+  if (use_pp() || packed_waves() != 4) return false;  // a switch names the kernel for every size
   const int64_t weights = (int64_t)(epilogue == NT_MOE_EPI_SWIGLU ? 2 : 1) * n_out * K * 2;
   return total_rows <= (weights >= (1 << 20) ? 64 : 32) * (int64_t)num_segments;
 }
@@ -952,7 +953,7 @@ hipError_t launch_grouped_gemm_bf16_packed_shared(const FewPart& routed, const i
   // projections are instantiated for gathered rows, as every caller has them)
   const bool same = shared.K == routed.K && shared.n_out == routed.n_out &&
                     (routed.src_row || epilogue == NT_MOE_EPI_NONE);
-  if (same && !use_pp() && total_rows > 0 && num_segments < NT_MOE_MAX_SEGMENTS &&
+  if (same && !use_pp() && packed_waves() == 4 && total_rows > 0 && num_segments < NT_MOE_MAX_SEGMENTS &&
       total_rows + shared_rows < ((int64_t)1 << 31)) {
     const SharedSegment seg{shared.a, shared.ld_a, shared.w, shared.c, shared.pre,
                             (int)shared_rows};

@@ -286,6 +286,52 @@ def test_256_tile_kernels_match_plain(switch):
     assert r.returncode == 0 and "variant ok" in r.stdout, r.stdout + r.stderr
 
 
+_KERNEL_CHECK = r"""
+import sys, torch
+sys.path.insert(0, sys.argv[1])
+from nexttransformer_amd import ops
+from torch.profiler import ProfilerActivity, profile
+def names(fn):
+    fn(); torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        fn(); torch.cuda.synchronize()
+    return [e.key for e in p.key_averages() if "ntmoe" in e.key]
+w = ops.pack_expert_weights(torch.zeros(8, 512, 512, device="cuda", dtype=torch.bfloat16), 2)
+for rows in (8, 200, 4000):
+    off = torch.tensor([0, 1] + [rows] * 7, dtype=torch.int32).cuda()
+    a = torch.zeros(rows, 512, device="cuda", dtype=torch.bfloat16)
+    seg = torch.tensor([0, rows], dtype=torch.int32).cuda()
+    print("one", rows, names(lambda: ops.grouped_gemm_packed(a, None, off, w, 2, rows)))
+    print("shared", rows, names(lambda: ops.grouped_gemm_packed_shared(a, None, off, w, 2, rows, a,
+                                                                       w[:1], False)))
+"""
+
+
+@pytest.mark.parametrize("switch,short,long", [
+    ("NT_MOE_GEMM_PP=1", "grouped_gemm_pp_kernel<", "grouped_gemm_pp_kernel<"),
+    ("NT_MOE_PACKED_WAVES=8", "grouped_gemm_packed_kernel<2, false, 8,",
+     "grouped_gemm_packed_kernel<2, false, 8,"),
+    ("NT_MOE_GEMM_PP=0", "few_gemm_kernel<", "grouped_gemm_packed_kernel<2, false, 4,")])
+def test_a_kernel_switch_holds_for_every_size(switch, short, long):
+    """The packed entry points run the kernel that a switch names for few rows, too, and for the
+    shared expert beside them; without one the kernel for few rows takes the short segments."""
+    import os
+    import subprocess
+    import sys
+    from pathlib import Path
+    root = str(Path(__file__).resolve().parents[1])
+    name, value = switch.split("=")
+    r = subprocess.run([sys.executable, "-c", _KERNEL_CHECK, root],
+                       env=dict(os.environ, **{name: value}), capture_output=True, text=True,
+                       timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
+    lines = [l for l in r.stdout.splitlines() if l.startswith(("one", "shared"))]
+    assert len(lines) == 6
+    for line in lines:
+        want = long if line.split()[1] == "4000" else short
+        assert line.count("ntmoe::(anonymous") - line.count("SharedSegment") == line.count(want) > 0, line
+
+
 PACKED_CASES = [
     Case("cfg1-shape", 512, 256, 8, 2, 512),
     Case("ragged-T1000-E32-k4", 1000, 1024, 32, 4, 512, seed=1),
