@@ -1061,12 +1061,14 @@ __device__ __forceinline__ float row_sum(float v) {
 // logit becomes NaN, which is never taken), all lane exchanges as DPP moves: the list insertions,
 // LDS re-reads and permutes of rank_token are a chain of latencies that nothing hides in a small
 // batch (one token of 256 experts, planes summed here too: 18.6 us that way, 10.3 us this way;
-// of 32 experts 5.3 and 3.4 us). Same bits.
+// of 32 experts 5.3 and 3.4 us). Same bits. scores may be plane 0 itself (so neither is
+// __restrict__): a workgroup reads the planes of its own tokens only, all of it before the barrier
+// that its stores follow.
 template <int KMAX, int NPL>
 __global__ __launch_bounds__(256) void router_rank_kernel(
-    const float* __restrict__ planes, int nchunk, const float* __restrict__ bias, int64_t T, int E,
-    int k, int score_fn, float* __restrict__ logits, int32_t* __restrict__ topk_ids,
-    float* __restrict__ topk_w, float* __restrict__ scores, float* __restrict__ z,
+    const float* planes, int nchunk, const float* __restrict__ bias, int64_t T, int E, int k,
+    int score_fn, float* __restrict__ logits, int32_t* __restrict__ topk_ids,
+    float* __restrict__ topk_w, float* scores, float* __restrict__ z,
     uint8_t* __restrict__ block_counts) {
   __shared__ __align__(16) float rows[kRankTokens][NPL * 16 + 1];
   __shared__ int cnt[NT_MOE_MAX_EXPERTS];
