@@ -351,10 +351,22 @@ hipError_t launch_grouped_gemm_fp8(const uint8_t* a, int64_t ld_a, int64_t a_row
   const int n_tiles = ceil_div(n_out, per_block);
   const dim3 grid((unsigned)((int64_t)num_segments * n_tiles));
   if (total_rows == 0) return hipSuccess;
-  // The tiled kernel from 16 rows per segment on the up projection (278 us against 279 there; 8
-  // rows 273 against 267, 32 rows 286 against 411) and from 4 on the others, whose row-wide
-  // stores also pay for fewer rows (4 rows 154 us against 156, 8 rows 157 against 168).
-  const int64_t few = epilogue == NT_MOE_EPI_SWIGLU ? 16 : 4;
+  // The tiled kernel from 16 rows per segment on with SwiGLU and from 4 on with the others, whose
+  // row-wide stores also pay for fewer rows, while the chip has more than one weight tile per CU:
+  // it is then bound by the weights (us, streaming / tiled, randomly routed rows: SwiGLU 128
+  // experts K 4096 H 1536 16 rows 298 / 302, 20 rows 312 / 301; 64 experts K 2048 H 1024 16 rows
+  // 59 / 54; ReLU^2 of the first 4 rows 146 / 148, 8 rows 152 / 149, of the second 29.5 / 28.1;
+  // down projections 169 / 160 and 35.7 / 30.5 at 4). With a tile per CU or fewer a wave's chain of
+  // K steps is the time, and the streaming kernel keeps more of it in flight until an expert's rows
+  // exceed its 32 a pass: SwiGLU K 1024 H 512, 32 experts 16 rows 11.1 / 12.8, 20 rows 15.0 / 12.7;
+  // K 4096 H 1024, 16 experts 33 / 39 and 51 / 39; ReLU^2 K 1024 H 512, 32 experts 4 rows 8.5 /
+  // 10.9, 16 rows 10.2 / 11.0, 20 rows 14.7 / 11.0; no activation K 4096, 64 experts x 512 columns
+  // 34 / 40 and 52 / 40. Short chains are the stores' time again: ReLU^2 K 256 6.6 / 6.0, no
+  // activation K 512 9.0 / 8.4 and K 1024 9.4 / 8.2 (16 experts), 10.7 / 10.7 (32), at 4 rows.
+  const bool chain = (int64_t)num_segments * (epilogue == NT_MOE_EPI_SWIGLU ? 2 : 1) * n_out / 128 <=
+                         num_cus() &&
+                     K > (epilogue == NT_MOE_EPI_NONE ? 1024 : 512);
+  const int64_t few = chain ? 20 : (epilogue == NT_MOE_EPI_SWIGLU ? 16 : 4);
   if (packed && total_rows >= few * num_segments &&
       fp8_tiled_supported(ld_a, a_rows, total_rows, K, c))
     return launch_grouped_gemm_fp8_tiled(a, ld_a, a_rows, a_scale, src_row, seg_offsets,

@@ -202,3 +202,47 @@ def test_fp8_many_rows_equal_the_streaming_kernel(K, epilogue, gather):
     tiled = ops.grouped_gemm_fp8(aq, as_, src, seg, ops.pack_expert_weights_fp8(wq, epilogue), ws,
                                  epilogue, rows, True)
     assert torch.equal(plain, tiled)
+
+
+_KERNEL_CHECK = r"""
+import sys, torch
+sys.path.insert(0, sys.argv[1])
+from nexttransformer_amd import ops
+from torch.profiler import ProfilerActivity, profile
+cus = torch.cuda.get_device_properties(0).multi_processor_count
+for epi, K, n_out, S, line in [(0, 1024, 512, cus // 8, 20), (0, 512, 512, cus // 8, 16),
+                               (0, 1024, 512, cus // 8 + 1, 16), (1, 1024, 1024, cus // 8, 20),
+                               (1, 512, 1024, cus // 8, 4), (1, 1024, 1024, cus // 8 + 1, 4),
+                               (2, 1152, 256, cus // 2, 20), (2, 1024, 256, cus // 2, 4),
+                               (2, 1152, 256, cus // 2 + 1, 4)]:
+    g = torch.Generator(device="cuda").manual_seed(K + S)
+    R = 2 * n_out if epi == 0 else n_out
+    wq, ws = ops.quantize_fp8_blockwise(torch.randn(S, R, K, device="cuda", generator=g) * 0.05)
+    wp = ops.pack_expert_weights_fp8(wq, epi)
+    for rows in (line * S - 1, line * S):
+        a, sc = ops.quantize_fp8_rowwise(torch.randn(rows, K, device="cuda", generator=g).bfloat16())
+        cuts = torch.randint(0, rows + 1, (S - 1,), device="cuda", generator=g).sort().values
+        off = torch.cat([cuts.new_zeros(1), cuts, cuts.new_full((1,), rows)]).int()
+        print("case", epi, K, S, rows, flush=True)
+        plain = ops.grouped_gemm_fp8(a, sc, None, off, wq, ws, epi, rows, False)
+        torch.cuda.synchronize()
+        with profile(activities=[ProfilerActivity.CUDA]) as p:
+            c = ops.grouped_gemm_fp8(a, sc, None, off, wp, ws, epi, rows, True)
+            torch.cuda.synchronize()
+        assert torch.equal(c, plain)
+        names = [e.key for e in p.key_averages() if "fp8" in e.key]
+        assert len(names) == 1 and ("tiled" in names[0]) == (rows >= line * S), (rows, names)
+print("lines ok")
+"""
+
+
+def test_fp8_kernels_on_both_sides_of_their_lines():
+    """Which kernel runs one row below and at each line of the dispatch (rows per segment, by the
+    weight tiles per CU, the K steps and the epilogue), and the same bits on both sides."""
+    import subprocess
+    import sys
+    from pathlib import Path
+    root = str(Path(__file__).resolve().parents[1])
+    r = subprocess.run([sys.executable, "-c", _KERNEL_CHECK, root], capture_output=True, text=True,
+                       timeout=100)
+    assert r.returncode == 0 and "lines ok" in r.stdout, r.stdout + r.stderr
