@@ -790,17 +790,41 @@ def _(y, combine_dest, first):
 # ---------------------------------------------------------------------------------------------
 # the whole layer
 
-_SEGMENTS = {}
+_SEGMENT_ROWS = 65536  # batches of up to so many tokens share one table per device (512 KB)
+_SEGMENT_TABLES = {}  # device -> int32 {[0, 0], [0, 1], ...}
+_SEGMENTS = {}        # (T, device) -> its row of the table
+_LONG_SEGMENTS = {}   # (T, device) -> a tensor of its own
 
 
 def _whole_batch_segment(T, device):
-    """Device tensor [0, T]: the shared expert's single segment (cached: no per-call upload)."""
+    """Device tensor [0, T]: the shared expert's single segment. A row of a table that is made once
+    per device, by a synchronous copy, and never changed or freed: any number of batch sizes,
+    streams, threads and captured graphs read it, and a new size needs no upload of its own.
+    Batches past the table: a tensor each, the first 64 sizes kept. Only plain tensors are kept
+    (under a fake or tracing mode the factories make others)."""
     key = (T, device)
     seg = _SEGMENTS.get(key)
+    if seg is not None:
+        return seg
+    if T <= _SEGMENT_ROWS:
+        table = _SEGMENT_TABLES.get(device)
+        if table is None:
+            rows = torch.zeros(_SEGMENT_ROWS + 1, 2, dtype=torch.int32)
+            rows[:, 1] = torch.arange(_SEGMENT_ROWS + 1, dtype=torch.int32)
+            table = rows.to(device)
+            if type(table) is torch.Tensor:
+                table = _SEGMENT_TABLES.setdefault(device, table)
+        seg = table[T]
+        if type(seg) is torch.Tensor:
+            if len(_SEGMENTS) >= 1024:  # (frees the views, not the table)
+                _SEGMENTS.clear()
+            _SEGMENTS[key] = seg
+        return seg
+    seg = _LONG_SEGMENTS.get(key)
     if seg is None:
         seg = torch.tensor([0, T], device=device, dtype=torch.int32)
-        if len(_SEGMENTS) < 64:
-            _SEGMENTS[key] = seg
+        if len(_LONG_SEGMENTS) < 64 and type(seg) is torch.Tensor:
+            _LONG_SEGMENTS[key] = seg
     return seg
 
 

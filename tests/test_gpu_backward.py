@@ -768,3 +768,31 @@ def test_forward_for_training_keeps_only_what_the_backward_reads(through_ops):
     kept = 2 * (T * d + T * k * H + T * k * 2 * H) + 4 * (T * E + 8 * T * k)
     assert held <= kept + (1 << 17), (held, kept)  # (small tensors are rounded up to 512 bytes)
     assert not any(t is not None and t.shape == (T * k, d) for t in state.values())
+
+
+def test_new_batch_sizes_need_no_synchronisation():
+    """Forward and backward of more batch sizes than a small cache holds, each for the first time,
+    without a synchronising call (an upload of the shared expert's segment would be one)."""
+    from nexttransformer_amd import ops
+    E, k, d, H = 8, 2, 256, 256
+    g = torch.Generator().manual_seed(8)
+    mk = lambda *s, std=0.05: (torch.randn(s, generator=g) * std).cuda()
+    w1, w2, s1, s2 = (mk(*s).bfloat16() for s in ((E, 2 * H, d), (E, d, H), (1, 2 * H, d), (1, d, H)))
+    wr, p = mk(d, E), ops.pack_expert_weights
+    bw = ops.backward_weights(w1, w2, s1, s2, wr)
+    kw = dict(top_k=k, packed=True, shared_w1=p(s1, 0), shared_w2=p(s2, 2))
+    p1, p2, xs = p(w1, 0), p(w2, 2), mk(400, d, std=1.0).bfloat16()
+
+    def both(T):
+        x = xs[:T]
+        state = ops.moe_forward(x, wr, p1, p2, want_logits=True, keep=True, **kw)[2]
+        return ops.moe_backward(x, None, x, wr, bw, state, top_k=k)["x"]
+
+    both(300)
+    torch.cuda.synchronize()
+    torch.cuda.set_sync_debug_mode("error")
+    try:
+        for T in range(150, 250):
+            both(T)
+    finally:
+        torch.cuda.set_sync_debug_mode("default")

@@ -158,6 +158,26 @@ def test_ops_reject_cpu_tensors():
         ops.grouped_wgrad(x, x, None, torch.zeros(2, dtype=torch.int32), 4)
 
 
+def test_whole_batch_segments_are_rows_of_one_table_and_plain_tensors():
+    """[0, T] for any number of batch sizes without a tensor each, and nothing kept of a fake
+    mode's tensors."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from nexttransformer_amd import ops
+    cpu = torch.device("cpu")
+    with FakeTensorMode():
+        ops._whole_batch_segment(5, cpu)
+        ops._whole_batch_segment(ops._SEGMENT_ROWS + 5, cpu)
+    sizes = [0, 1, 5, ops._SEGMENT_ROWS, ops._SEGMENT_ROWS + 1, ops._SEGMENT_ROWS + 5]
+    for T in sizes + list(range(1000, 2200)) + sizes:
+        seg = ops._whole_batch_segment(T, cpu)
+        assert type(seg) is torch.Tensor and seg.tolist() == [0, T] and seg.is_contiguous(), T
+    table = ops._SEGMENT_TABLES[cpu]
+    for T in (1, 700, 1999, ops._SEGMENT_ROWS):
+        seg = ops._whole_batch_segment(T, cpu)
+        assert seg.data_ptr() == table.data_ptr() + 8 * T
+    assert len(ops._SEGMENTS) <= 1024
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     from nexttransformer_amd import _native
     monkeypatch.setattr(_native, "LIB_PATH", tmp_path / "missing.so")
