@@ -5,6 +5,8 @@ There is no fallback: if the library is missing, every op raises.
 """
 import ctypes
 import importlib.util
+import sys
+import warnings
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libnt_moe.so"
@@ -122,11 +124,35 @@ def load():
     return lib
 
 
+class _OpsOnly:
+    """In the host module's place where that was built for another torch: it takes no call, so
+    every caller goes through the ops (the same kernels, issued from Python)."""
+
+    @staticmethod
+    def forward(*args):
+        return None
+
+    backward = masters = forward
+
+    @staticmethod
+    def give_grads(*args):
+        return False
+
+
+def host_marker():
+    """What nt_moe_host.so holds when it was built for the running torch and Python: it uses torch's
+    C++ classes, whose layout is one version's own."""
+    import torch
+    return (f"nt_moe_host for torch {torch.__version__}, Python {sys.version_info[0]}."
+            f"{sys.version_info[1]};").encode()
+
+
 _HOST = None
 
 
 def host():
-    """The native host path, the module nt_moe_host (cached); NativeLibraryMissing without it."""
+    """The native host path, the module nt_moe_host (cached). NativeLibraryMissing without it; built
+    for another torch or Python it is not loaded, with a warning, and the ops do its work."""
     global _HOST
     if _HOST is None:
         load()
@@ -134,7 +160,11 @@ def host():
         if not path.exists():
             raise NativeLibraryMissing(
                 f"{path} is missing: build it with `python -m nexttransformer_amd.build`")
-        import torch  # noqa: F401  (the module's symbols come from torch's libraries)
+        if host_marker() not in path.read_bytes():
+            warnings.warn(f"{path} was built for another torch or Python: small batches are slower "
+                          "until `python -m nexttransformer_amd.build` has run", RuntimeWarning)
+            _HOST = _OpsOnly()
+            return _HOST
         spec = importlib.util.spec_from_file_location("nt_moe_host", path)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)

@@ -61,9 +61,11 @@ def _compile_host(verbose):
     glibc's slow way (each torch.empty 1.1 -> 1.4 us, a small fp8 forward through the ops 91 -> 101
     us once the module was loaded)."""
     import torch
+    from nexttransformer_amd._native import host_marker
     root = Path(torch.__file__).resolve().parent
     obj = BUILD / "host.o"
     cmd = [shutil.which("g++") or "c++", "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-fvisibility=hidden",
+           f'-DNT_MOE_HOST_MARKER="{host_marker().decode()}"',
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            f"-I{ROOT / 'include'}", f"-isystem{root / 'include'}",
            f"-isystem{root / 'include' / 'torch' / 'csrc' / 'api' / 'include'}",

@@ -447,6 +447,9 @@ PyMethodDef methods[] = {
      METH_FASTCALL, "Hands each parameter its slice of a gradient stack."},
     {nullptr, nullptr, 0, nullptr}};
 
+// Read from the file before it is loaded (_native.host).
+__attribute__((used)) const char marker[] = NT_MOE_HOST_MARKER;
+
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "nt_moe_host",
                       "Native host path of the MoE layer", -1, methods};
 

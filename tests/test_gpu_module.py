@@ -305,3 +305,36 @@ def test_native_host_path_refuses_what_the_ops_refuse():
                      ((xb[:, :64], wr[:64].contiguous(), w1[:, :, :64].contiguous(), w2), {})):
         with pytest.raises(ValueError):
             call(*args, **kw)
+
+
+@pytest.mark.parametrize("expert_grad", ["accumulate", "autograd"])
+def test_training_without_the_host_module_gives_the_same_bits(monkeypatch, expert_grad):
+    """Two steps with an update between, through the native host path and (in its absence) through
+    the ops alone: outputs, load and every gradient."""
+    from nexttransformer_amd import _native as nat
+    from nexttransformer_amd.moe import MoELayer
+    from nexttransformer_amd.moe_recipe import MoERecipe
+
+    def steps():
+        layer = MoELayer(MoERecipe(layers=2, width=256, heads=4, sequence_len=64,
+                                   global_batch_tokens=256, routed_experts=8, top_k=2,
+                                   expert_width=256, activation="swiglu", shared_experts=1,
+                                   shared_expert_width=128, allow_any_expert_width=True), 1,
+                         expert_grad=expert_grad)
+        opt = torch.optim.SGD(layer.parameters(), lr=0.5)
+        got = []
+        for i in range(2):
+            g = torch.Generator().manual_seed(i)
+            x = torch.randn(130, 256, generator=g).to(torch.bfloat16).cuda().requires_grad_()
+            opt.zero_grad()
+            out, aux = layer(x)
+            out.backward(torch.randn(130, 256, generator=g).to(torch.bfloat16).cuda())
+            got += [out.detach(), aux.detach(), layer.last_load, x.grad]
+            got += [p.grad.clone() for p in layer.parameters()]
+            opt.step()
+        return got
+
+    native = steps()
+    monkeypatch.setattr(nat, "_HOST", nat._OpsOnly())
+    for a, b in zip(native, steps()):
+        assert torch.equal(a, b)

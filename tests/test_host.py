@@ -186,6 +186,26 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
         _native.load()
 
 
+def test_host_module_of_another_torch_is_not_loaded(monkeypatch, tmp_path):
+    """A module built for another torch or Python would read torch's objects by the wrong layout:
+    a warning instead, and every call goes through the ops. A missing one still raises."""
+    from nexttransformer_amd import _native as nat
+    nat.load()
+    built = nat.LIB_PATH.with_name("nt_moe_host.so").read_bytes()
+    assert built.count(nat.host_marker()) == 1
+    monkeypatch.setattr(nat, "LIB_PATH", tmp_path / "libnt_moe.so")
+    monkeypatch.setattr(nat, "_HOST", None)
+    with pytest.raises(nat.NativeLibraryMissing):
+        nat.host()
+    marker = nat.host_marker()
+    (tmp_path / "nt_moe_host.so").write_bytes(built.replace(marker, marker.replace(b"torch ", b"torch 9")))
+    with pytest.warns(RuntimeWarning, match="another torch"):
+        h = nat.host()
+    assert h.forward(1, 2) is None and h.backward() is None and h.masters([]) is None
+    assert h.give_grads([], None) is False
+    assert nat.host() is h
+
+
 # ---------------------------------------------------------------------------------------------
 # recipe
 
