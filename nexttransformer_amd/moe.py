@@ -289,6 +289,14 @@ class MoELayer(nn.Module):
         self._packed = None
         self.reset_parameters()
 
+    def __setstate__(self, state):
+        """Layers pickled when the load was kept as int32 counts and converted on access."""
+        if "last_load" not in state:
+            state = dict(state)
+            counts = state.pop("_last_counts", None)
+            state["last_load"] = None if counts is None else counts.to(torch.int64)
+        super().__setstate__(state)
+
     # -- initialisation --------------------------------------------------------------------
 
     @torch.no_grad()

@@ -428,6 +428,30 @@ def test_module_state_dict_round_trip_and_repack():
     assert not repacked["w2"][3][:, 16:].any()
 
 
+def test_pickled_layers_keep_their_load(tmp_path):
+    """A layer saved as a whole: its load comes back, also from files that hold the int32 counts of
+    earlier builds, and the copy's master tables are its own parameters'."""
+    import copy
+    import pickle
+    from nexttransformer_amd.moe import MoELayer
+    layer = MoELayer(small_recipe(), 1, device="cpu")
+    layer._masters_key()
+    for saved in (None, torch.arange(8)):
+        layer.last_load = saved
+        for other in (copy.deepcopy(layer), pickle.loads(pickle.dumps(layer))):
+            assert (saved is None and other.last_load is None) or torch.equal(other.last_load, saved)
+            assert other._masters()[1] is other.experts.local_experts[0].linear_fc1.weight
+            assert other._all_tables[0] is other.router._parameters
+        old = dict(layer.__dict__)
+        del old["last_load"], old["_all_tables"]
+        old["_last_counts"] = None if saved is None else saved.int()
+        other = MoELayer.__new__(MoELayer)
+        other.__setstate__(old)
+        assert "_last_counts" not in other.__dict__ and "_last_counts" in old
+        assert (saved is None and other.last_load is None) or (
+            torch.equal(other.last_load, saved) and other.last_load.dtype == torch.int64)
+
+
 @pytest.mark.parametrize("activation", ["swiglu", "relu2"])
 def test_padded_packing_computes_the_same_layer(activation):
     """Widths that are not multiples of 64 are zero-padded for the GEMM tiles; the padded
