@@ -338,3 +338,141 @@ def test_training_without_the_host_module_gives_the_same_bits(monkeypatch, exper
     monkeypatch.setattr(nat, "_HOST", nat._OpsOnly())
     for a, b in zip(native, steps()):
         assert torch.equal(a, b)
+
+
+def _small_calls(T=65, E=8, k=2, d=256, H=256):
+    """(forward(x, **kw), backward(state, **kw), x) on packed bf16 operands with a shared expert."""
+    from nexttransformer_amd import ops
+    g = torch.Generator().manual_seed(T)
+    mk = lambda *s, std=0.05: (torch.randn(s, generator=g) * std).cuda()
+    w1, w2, s1, s2 = (mk(*s).bfloat16() for s in ((E, 2 * H, d), (E, d, H), (1, 2 * H, d), (1, d, H)))
+    x, go, wr, p = mk(T, d, std=1.0).bfloat16(), mk(T, d, std=1.0).bfloat16(), mk(d, E), ops.pack_expert_weights
+    p1, p2 = p(w1, 0), p(w2, 2)
+    kw = dict(top_k=k, packed=True, shared_w1=p(s1, 0), shared_w2=p(s2, 2))
+    bw = ops.backward_weights(w1, w2, s1, s2, wr)
+    forward = lambda x, **more: ops.moe_forward(x, wr, p1, p2, want_logits=True, keep=True, **kw, **more)
+    backward = lambda x, state, **more: ops.moe_backward(go, None, x, wr, bw, state, top_k=k, **more)
+    return forward, backward, x
+
+
+def _count_native(monkeypatch):
+    """A list that takes, per call of the host module's forward and backward, whether it did the
+    work."""
+    from types import SimpleNamespace
+    from nexttransformer_amd import _native as nat
+    host, calls = nat.host(), []
+
+    def counted(name):
+        def call(*args):
+            r = getattr(host, name)(*args)
+            calls.append((name, r is not None))
+            return r
+        return call
+
+    monkeypatch.setattr(nat, "_HOST", SimpleNamespace(
+        forward=counted("forward"), backward=counted("backward"), masters=host.masters,
+        give_grads=host.give_grads))
+    return calls
+
+
+def test_native_host_path_is_taken(monkeypatch):
+    """By the ops on packed operands and by the layer, inference and training; not with a mark."""
+    from nexttransformer_amd.moe import MoELayer
+    from nexttransformer_amd.moe_recipe import MoERecipe
+    calls = _count_native(monkeypatch)
+    forward, backward, x = _small_calls()
+    backward(x, forward(x)[2])
+    assert calls == [("forward", True), ("backward", True)]
+    mark = dict(mark=lambda name: None)
+    backward(x, forward(x, **mark)[2], **mark)
+    assert len(calls) == 2
+    layer = MoELayer(MoERecipe(layers=2, width=256, heads=4, sequence_len=64, global_batch_tokens=256,
+                               routed_experts=8, top_k=2, expert_width=256, activation="swiglu",
+                               shared_experts=0, allow_any_expert_width=True), 1)
+    with torch.no_grad():
+        layer(x)
+    layer(x.requires_grad_())[0].sum().backward()
+    assert calls[2:] == [("forward", True), ("forward", True), ("backward", True)]
+
+
+def test_native_host_path_leaves_wrapped_tensors_to_the_ops(monkeypatch):
+    """A tensor subclass and a dispatch mode: the ops, with the same results, and the mode sees
+    their factory calls. Under functorch's vmap and grad: refused before anything is launched, as
+    the ops refuse a tensor without storage."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    calls = _count_native(monkeypatch)
+    forward, backward, x = _small_calls()
+    out, aux, state = forward(x)
+    grads = backward(x, state)
+
+    class Sub(torch.Tensor):
+        pass
+
+    class Seen(TorchDispatchMode):
+        names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    def check(r):
+        assert torch.equal(r[0], out) and torch.equal(r[1], aux)
+        for n, t in state.items():
+            assert torch.equal(t, r[2][n]), n
+
+    def check_grads(g):
+        for n, t in grads.items():
+            assert torch.equal(t, g[n]), n
+
+    del calls[:]
+    check(forward(x.as_subclass(Sub)))
+    check_grads(backward(x.as_subclass(Sub), state))
+    with Seen() as seen:
+        r = forward(x)
+        g = backward(x, state)
+    check(r)
+    check_grads(g)
+    assert any("empty" in n for n in seen.names)
+    assert calls == [("forward", False), ("backward", False)] * 2
+    del calls[:]
+    with pytest.raises(RuntimeError):
+        torch.vmap(lambda v: forward(v)[0])(torch.stack([x, x]))
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda v: forward(v)[0].float().sum())(x)
+    assert all(not taken for _, taken in calls)
+
+
+def test_native_host_path_from_two_threads():
+    """Two threads, a stream and inputs each (the calls run without the GIL): what each gets alone."""
+    import threading
+    work = [_small_calls(T=T) for T in (33, 130)]
+    alone = []
+    for forward, backward, x in work:
+        out, aux, state = forward(x)
+        alone.append((out, aux, backward(x, state)))
+    torch.cuda.synchronize()
+    failed = []
+
+    def run(i):
+        try:
+            forward, backward, x = work[i]
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                got = []
+                for _ in range(40):
+                    out, aux, state = forward(x)
+                    got.append((out, aux, backward(x, state)))
+            stream.synchronize()
+            for out, aux, grads in got:
+                assert torch.equal(out, alone[i][0]) and torch.equal(aux, alone[i][1])
+                for n, t in alone[i][2].items():
+                    assert torch.equal(t, grads[n]), n
+        except BaseException as e:  # noqa: BLE001
+            failed.append(e)
+
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
