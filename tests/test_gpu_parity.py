@@ -88,8 +88,9 @@ VARIANTS = ([(v, E, T, 1024) for v in ("no-buffers", "workspace", "logits-buffer
 def test_router_variants_bit_exact_via_abi(variant, E, T, d):
     """Raw C-ABI calls that reach each router kernel (on a 256-CU part): with neither workspace
     nor a logits buffer the fused kernel (top-k in the block; one, two and four expert blocks);
-    with the workspace the chunk planes (T = 512) or the logits kernel + top-k (T = 4096); with
-    only a logits buffer the logits kernel. All follow the same order: identical bits."""
+    with the workspace the chunk planes or the logits kernel, ranked over the whole chip; with
+    only a logits buffer the logits kernel and the 64-token top-k. All follow the same order:
+    identical bits."""
     import ctypes
     from nexttransformer_amd import _native as nat
     case = Case("variant", T, d, E, 4, 64, seed=11)
@@ -123,10 +124,43 @@ def test_router_variants_bit_exact_via_abi(variant, E, T, d):
     torch.testing.assert_close(pp.cpu().double().sum(0), s_.sum(0), rtol=1e-5, atol=1e-5)
 
 
-# The streamed router (129-256 experts, at least 64 token blocks): E not a multiple of 32, a
-# partial last 64-feature stage (d = 1032) and a one-chunk d, a ragged last token block, bias,
-# sigmoid, top-6 and top-8.
+@pytest.mark.parametrize("T,d,E,k,whole", [(512, 1024, 64, 4, False), (300, 640, 30, 3, False),
+                                           (100, 1280, 256, 8, False), (9000, 2176, 128, 8, True)])
+def test_summed_planes_and_the_block_top_k_bit_exact(T, d, E, k, whole):
+    """The chunk planes summed in a pass of their own (experts in fours, or by the top-k) and ranked
+    64 tokens to a block: with a workspace of the planes alone, as callers sized it before the
+    ranking kept its scores there, or for more selections than are ranked over the whole chip."""
+    import ctypes
+    from nexttransformer_amd import _native as nat
+    lib = nat.load()
+    cpu, g = gpu_inputs(Case("planes", T, d, E, k, 64, seed=12))
+    nblk, chunks = (T + 63) // 64, (d + 127) // 128
+    mk = lambda *s, dt=torch.float32: torch.empty(s, device="cuda", dtype=dt)
+    logits, ids, w, pp, zp = mk(T, E), mk(T, k, dt=torch.int32), mk(T, k), mk(nblk, E), mk(nblk)
+    need = lib.nt_moe_router_workspace_bytes(T, d, E, k) if whole else 4 * T * E * chunks
+    assert need >= 4 * T * E * chunks
+    ws = mk(need, dt=torch.uint8)
+    nat.check(lib.nt_moe_router_fwd(
+        nat.ptr(g["x"]), d, nat.ptr(g["wt"]), None, T, d, E, k, 1, nat.ptr(logits), nat.ptr(ids),
+        nat.ptr(w), nat.ptr(pp), nat.ptr(zp), nat.ptr(ws), need,
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "router")
+    torch.cuda.synchronize()
+    ref = orc.router_logits_fixed(cpu["x"], cpu["router"])
+    assert torch.equal(logits.cpu().view(torch.int32), ref.view(torch.int32))
+    ref_ids, ref_w = orc.topk(ref, k, 1)
+    assert torch.equal(ids.cpu(), ref_ids)
+    torch.testing.assert_close(w.cpu(), ref_w, rtol=2e-6, atol=2e-7)
+    s_ = orc.full_scores(ref, 1)
+    torch.testing.assert_close(pp.cpu().double().sum(0), s_.sum(0), rtol=1e-5, atol=1e-5)
+
+
+# 129-256 experts, at least 64 token blocks: E not a multiple of 32, a partial last 64-feature stage
+# (d = 1032) and a one-chunk d, a ragged last token block, bias, sigmoid, top-6 and top-8. The
+# first is the streamed router's; on a 256-CU part the others' sizes are the chunk planes' (the
+# streamed kernel at small sizes: test_forced_router_modes_write_the_plan).
 STREAM = [
+    Case("stream-T8260-d1032-E200-k8-sigmoid-bias", 8260, 1032, 200, 8, 64, score_fn=1,
+         zipf_bias=0.8, seed=20),
     Case("stream-T4100-d1032-E200-k8-sigmoid-bias", 4100, 1032, 200, 8, 64, score_fn=1,
          zipf_bias=0.8, seed=21),
     Case("stream-T4096-d1280-E256-k8", 4096, 1280, 256, 8, 64, seed=22),
@@ -161,6 +195,7 @@ ROUTER_PLAN = SMALL + MID + STREAM + [
     Case("t3-T16384-d1280-E256-k8", 16384, 1280, 256, 8, 64, seed=24),
     Case("E64-T16400-d2048-k8-zipf", 16400, 2048, 64, 8, 64, zipf_bias=1.2, seed=25),
     Case("E128-T8192-d2048-k8-sigmoid", 8192, 2048, 128, 8, 64, score_fn=1, seed=26),
+    Case("E128-T9000-d2176-k8", 9000, 2176, 128, 8, 64, seed=27),
 ]
 
 
