@@ -74,24 +74,37 @@ def set_aux_loss_scale(scale, *, device="cpu"):
     _aux_loss_scale = torch.tensor(float(scale), dtype=torch.float32, device=device)
 
 
-_injected_cache = {}  # device -> (the scale tensor it was made from, its version, gradient)
+_injected_cache = {}  # (device, stream) -> (the scale tensor it was made from, its version, gradient)
 
 
 def _injected_aux_grad(device):
     """{lb + z, lb, z} gradient [3] on `device` that an "inject" backward adds: (scale, 0, 0).
-    Made once per device while the scale set by set_aux_loss_scale stays the same unmodified
-    tensor (two small kernels less per backward); callers must not modify it."""
+    Made once per device and stream (its fill is not yet done for another stream's readers) while
+    the scale set by set_aux_loss_scale stays the same unmodified tensor (two small kernels less
+    per backward); callers must not modify it. A captured graph takes one made before it on any
+    stream, and keeps none of its own making, whose fill runs only when the graph does."""
     s = _aux_loss_scale
     ver = None if s is None else s._version
-    hit = _injected_cache.get(device)
-    if hit is not None and hit[0] is s and hit[1] == ver:
+    same = lambda hit: hit is not None and hit[0] is s and hit[1] == ver
+    gpu = device.type == "cuda"
+    key = (device, torch.cuda.current_stream(device).cuda_stream if gpu else None)
+    hit = _injected_cache.get(key)
+    if same(hit):
         return hit[2]
+    capturing = gpu and torch.cuda.is_current_stream_capturing()
+    if capturing:
+        for (dev, _), hit in list(_injected_cache.items()):
+            if dev == device and same(hit):
+                return hit[2]
     g = torch.zeros(3, device=device, dtype=torch.float32)
     if s is None:
         g[0] = 1.0
     else:
         g[0] = s.to(device, non_blocking=True)
-    _injected_cache[device] = (s, ver, g)
+    if not capturing:
+        if len(_injected_cache) >= 64:  # (each was made and read on its own stream only)
+            _injected_cache.clear()
+        _injected_cache[key] = (s, ver, g)
     return g
 
 

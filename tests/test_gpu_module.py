@@ -476,3 +476,54 @@ def test_native_host_path_from_two_threads():
     for t in threads:
         t.join()
     assert not failed, failed
+
+
+def test_injected_aux_gradient_is_made_on_the_stream_that_reads_it():
+    """Training on two streams after a new aux-loss scale, the first one's work queued behind a long
+    product: the second's router gradient holds the scale, and so does a captured graph's."""
+    from nexttransformer_amd import moe
+    from nexttransformer_amd.moe import MoELayer, set_aux_loss_scale
+    from nexttransformer_amd.moe_recipe import MoERecipe
+    layer = MoELayer(MoERecipe(layers=2, width=256, heads=4, sequence_len=64, global_batch_tokens=256,
+                               routed_experts=8, top_k=2, expert_width=256, activation="swiglu",
+                               shared_experts=0, aux_loss_coeff=3.0, allow_any_expert_width=True), 1)
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(130, 256, generator=g).to(torch.bfloat16).cuda()
+    go = torch.zeros_like(x)
+
+    def grad():
+        out, _ = layer(x)
+        return torch.autograd.grad(out, layer.router.weight, go)[0]
+
+    try:
+        set_aux_loss_scale(0.25)
+        quarter = grad()
+        set_aux_loss_scale(0.5)
+        a, b = torch.cuda.Stream(), torch.cuda.Stream()
+        big = torch.randn(8192, 8192, device="cuda")
+        torch.cuda.synchronize()
+        with torch.cuda.stream(a):
+            for _ in range(20):
+                big @ big
+            ga = grad()
+        with torch.cuda.stream(b):
+            gb = grad()
+        torch.cuda.synchronize()
+        half = grad()
+        assert torch.equal(ga, half) and torch.equal(gb, half)
+        assert float((half - 2 * quarter).norm() / half.norm()) < 1e-3 and float(half.norm()) > 0
+        # a stream of its own captures: it takes the gradient made before
+        made = {k: v[2] for k, v in moe._injected_cache.items()}
+        side = torch.cuda.Stream()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            inside = moe._injected_aux_grad(x.device)
+            read = inside * 2
+        assert any(inside is t for t in made.values())
+        assert {k: v[2] for k, v in moe._injected_cache.items()}.keys() == made.keys()
+        for _ in range(3):
+            graph.replay()
+            torch.cuda.synchronize()
+            assert read.tolist() == [1.0, 0.0, 0.0]
+    finally:
+        moe._aux_loss_scale = None
