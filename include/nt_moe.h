@@ -86,8 +86,10 @@ const char* nt_moe_last_error(void);
  *   prob_partial fp32 [ceil(T/64), E]: per 64-token block, sum over its tokens of the
  *                full score s_te (softmax over all E, or sigmoid normalised over all E)
  *   z_partial   fp32 [ceil(T/64)]: per block, sum of logsumexp(logits_t)^2
- *   workspace   nt_moe_router_workspace_bytes(T, d, E, k) bytes; may be smaller (or NULL)
- *               for E <= 256, which then takes a single-kernel path (slower for small T);
+ *   workspace   nt_moe_router_workspace_bytes(T, d, E, k) bytes: ceil(d / 128) planes of 4 T E
+ *               bytes where the features are split over the chip (T <= 8192, and longer batches
+ *               of d > 2048; 512 MB at most), one plane or none elsewhere; may be smaller (or
+ *               NULL) for E <= 256, which then takes a single-kernel path (slower for small T);
  *               E > 256 needs it (or logits, with d <= 2048)
  */
 size_t nt_moe_router_workspace_bytes(int64_t T, int32_t d, int32_t E, int32_t k);

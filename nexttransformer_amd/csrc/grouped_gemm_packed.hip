@@ -939,7 +939,10 @@ hipError_t launch_grouped_gemm_bf16_packed_keep(const uint16_t* a, int64_t ld_a,
 // kernel where the two have the same shape, else one after the other. Past 2048 shared rows (top-1
 // and top-2 routing over many experts) the shared tiles are too much work for the kernel for few
 // rows (d 2048, 3072 wide, 3001 rows alone 125 us against 47) to hide under the routed weight
-// stream.
+// stream. Whole forwards at 2048 tokens, apart -> in one launch: 128 experts d 2048 top-1 and top-2
+// with a shared expert of twice the width 361 -> 296 and 380 -> 318 us, 256 experts d 2048 top-2
+// 341 -> 275, d 1280 top-1 206 -> 139, 32 experts d 1024 top-1 with one of four times the width
+// 121 -> 82 (router and combine included in both).
 hipError_t launch_grouped_gemm_bf16_packed_shared(const FewPart& routed, const int32_t* seg_offsets,
                                                   int num_segments, int64_t total_rows,
                                                   const FewPart& shared, int64_t shared_rows,

@@ -1517,7 +1517,11 @@ enum RouterPath { kFused = 0, kLogits = 1, kPlanes = 2, kStream = 3 };
 // writing and summing the planes), while the logits and the streamed kernel take whole rounds of
 // 64-token workgroups (8.3 and 10.5 us per 128-feature chunk of a workgroup's range). Router and
 // plan with want_logits, E = 256, d = 1280: 4095 tokens streamed 130 us, planes 72; 8192 tokens
-// 128 and 118; 3001 tokens logits 69, planes 63, but 2048 tokens (one full round) 44 and 51.
+// 128 and 118; 3001 tokens logits 69, planes 63, but 2048 tokens (one full round) 44 and 51. The
+// two rates were fitted there and hold elsewhere: over 8 to 256 experts, d 256 to 4096 and 1 to 8192
+// tokens (420 calls) none took longer than by the rule without them and the 64-token top-k.
+// The price is workspace: up to 512 MB of planes (84 MB at 8192 tokens of d 1280, 256 experts) on
+// shapes whose streamed kernel needs none.
 constexpr int64_t kPlanesTokens = 8192;  // (T k <= kRankAssignments for every k)
 
 int router_path(int64_t T, int d, int E) {

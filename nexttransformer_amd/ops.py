@@ -952,7 +952,7 @@ def moe_forward(x, w_router_t, w1, w2, *, top_k, score_fn=nat.SCORE_SOFTMAX,
         return gemm_up(a, rows_src, offs, w, up_epi, rows), None
 
     # A packed projection of the routed and the shared expert is one call: one launch for short
-    # segments (the T3 cell, 48 tokens: 43 + 28 us up, 44 + 11 down as four launches).
+    # segments and for equal shapes.
     shared_y = hs = fc1s = None
     both_up = shared_w1 is not None and packed_up and not permute_rows
     both_down = shared_w1 is not None and packed_down
