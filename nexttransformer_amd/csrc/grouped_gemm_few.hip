@@ -8,8 +8,8 @@
 // or for the shared expert alone, and a tile list to scan before the first load. Here:
 //   * one workgroup per (segment, 128 packed weight rows): it reads two offsets and leaves if the
 //     segment is empty; nothing is scanned. A segment of more than 128 rows is cut into even chunks
-//     of whole 32-row blocks: its workgroup takes the first one, and the others have workgroups at
-//     the front of the grid, which find theirs by a scan of the offsets;
+//     of whole 32-row blocks: its workgroup takes the first one, and the others have workgroups of
+//     their own, which find theirs by a scan of the offsets;
 //   * wave w streams packed block w of the tile (4 KB per 64-wide K step) into a register ring,
 //     D steps ahead: 6, 4 or 2 for chunks of 32, 64 and 128 rows, as the accumulators allow;
 //   * the chunk's token rows go through LDS in a ring of the same depth (direct-to-LDS copies,
@@ -217,14 +217,18 @@ __host__ __device__ inline int few_n_tiles(int n_out, int epilogue) {
 // 8's, so the workgroups that read the same token rows share an L2 (777 tokens over 128 experts:
 // up 186 -> 146 us, down 108 -> 85 us); with fewer segments spread = 1: the whole chip takes
 // each one's weight rows.
-// The first tail_blocks workgroups each take one chunk past the first of a segment that has more
-// than one (routing that favours a few experts), weight rows fastest, an eighth of that list per
-// XCD; without such segments they read the offsets and leave. With the segment's own workgroups
-// walking them, 8192 rows of one of 256 experts (K 1280, 320 outputs) took 775 us and 8 x 1024 rows
-// 102; this way both take 21 (the tiled kernel 27), and 32 rows of every expert 46 (45; tiled 54).
-// At the end of the grid they cost the even case 1 us less and the uneven ones up to a quarter more
-// (32 experts, K 1024, 4 x 256 rows: 17.5 us there, 13.9 here, tiled 16.3). One chunk each and no
-// loop: the state of a loop around the tile spills.
+// tail_blocks workgroups each take one chunk past the first of a segment that has more than one
+// (routing that favours a few experts), weight rows fastest, an eighth of that list per XCD; without
+// such segments they read the offsets and leave. With the segment's own workgroups walking those
+// chunks, 8192 rows of one of 256 experts (K 1280, 320 outputs) took 775 us and 8 x 1024 rows 102;
+// this way both take 21 (the tiled kernel 27), and 32 rows of every expert 46 (45; tiled 54). One
+// chunk each and no loop: the state of a loop around the tile spills. The first kFront of them lead
+// the grid, so long segments start at once (at its end 32 experts, K 1024, 4 x 256 rows take 17.5 us,
+// in front 14.0, tiled 16.3; 128 experts, K 2048, lognormal rows 180, 171 and 171); the others end
+// it: all in front would keep the even case's workgroups out of the CUs for an offset read (777
+// tokens of 128 experts, 576 and 768 of them, 287.8 -> 291.2 us a forward).
+constexpr int kFront = 256;
+
 template <int EPI, bool KEEP>
 __global__ __launch_bounds__(256, 3) void few_gemm_kernel(FewPart routed,
                                                           const int32_t* __restrict__ seg_offsets,
@@ -232,8 +236,10 @@ __global__ __launch_bounds__(256, 3) void few_gemm_kernel(FewPart routed,
                                                           FewPart shared, int shared_rows,
                                                           int shared_blocks, int tail_blocks) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const int tail = (int)blockIdx.x < tail_blocks ? (int)blockIdx.x : -1;
-  int b = (int)blockIdx.x - tail_blocks;
+  const int front = tail_blocks < kFront ? tail_blocks : kFront;
+  const int own = (int)gridDim.x - tail_blocks;  // workgroups of the shared expert and the segments
+  int b = (int)blockIdx.x - front;
+  const int tail = b < 0 ? (int)blockIdx.x : (b < own ? -1 : (int)blockIdx.x - own);
   const bool is_shared = tail < 0 && b < shared_blocks;
   const FewPart& p = is_shared ? shared : routed;
   const int n_tiles = few_n_tiles(p.n_out, EPI);

@@ -848,8 +848,8 @@ static bool packed_edge(int K, int n_out, int epilogue) {
 // workgroup's start and stores weigh more than its stream (0.8 MB at 48 rows 48 / 53 -> 52 / 55).
 // Uneven routing does not turn that round: with the mean at 32 rows and 49, lognormal and Zipf
 // popularities up to all rows in top-k experts are as fast or faster (68 -> 51 us, 27 -> 21 at
-// the extreme; 169 -> 165, 54 -> 55), but for the 128-expert down projection with all 6216 rows
-// in 8 or 16 experts (32 -> 36 and 33 -> 38).
+// the extreme; 169 -> 164, 55 -> 54), but for the 128-expert down projection with all 6216 rows
+// in 8 or 16 experts (32 -> 36 and 33 -> 42).
 static bool few_rows(int num_segments, int64_t total_rows, int K, int n_out, int epilogue) {
   if (use_pp() || packed_waves() != 4) return false;  // a switch names the kernel for every size
   const int64_t weights = (int64_t)(epilogue == NT_MOE_EPI_SWIGLU ? 2 : 1) * n_out * K * 2;
