@@ -672,7 +672,10 @@ def main():
                     "bytes_per_launch": up_bytes, "experts_touched": touched,
                     "avg_launch_ms": round(up_ms, 5), "launches_timed": len(ev)}
     else:
-        up_flop = 2.0 * A * case.d * F
+        # packed weights: the shared expert's up projection is part of the same call
+        with_shared = bool(case.shared_H) and g["packed"][0] and not args.permute_rows
+        Fs = (2 if case.activation == 0 else 1) * case.shared_H if with_shared else 0
+        up_flop = 2.0 * case.d * (A * F + case.T * Fs)
         achieved = up_flop / (up_ms * 1e-3) / 1e12
         # the plain-weight entry point takes the 256x256 kernel when K >= 128 and the output
         # width is a multiple of 8 (nt_moe_grouped_gemm_bf16)
@@ -680,7 +683,8 @@ def main():
         plain = "grouped_gemm_t256_kernel" if case.d >= 128 and n_out % 8 == 0 else "grouped_gemm_kernel"
         epi = "SwiGLU" if case.activation == 0 else "ReLU^2"
         roofline = {"kernel": ("grouped_gemm_packed_kernel" if g["packed"][0] else plain)
-                              + f" (up-projection + {epi} epilogue)",
+                              + f" (up-projection + {epi} epilogue"
+                              + (", routed and shared expert)" if with_shared else ")"),
                     "bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK_BF16_TFLOPS,
                     "unit": "TFLOP/s", "frac": round(achieved / PEAK_BF16_TFLOPS, 4),
                     "traffic": load_traffic(f"config{args.config}"),
