@@ -809,8 +809,8 @@ def _whole_batch_segment(T, device):
     if T <= _SEGMENT_ROWS:
         table = _SEGMENT_TABLES.get(device)
         if table is None:
-            rows = torch.zeros(_SEGMENT_ROWS + 1, 2, dtype=torch.int32)
-            rows[:, 1] = torch.arange(_SEGMENT_ROWS + 1, dtype=torch.int32)
+            rows = torch.zeros(_SEGMENT_ROWS + 1, 2, dtype=torch.int32, device="cpu")
+            rows[:, 1] = torch.arange(_SEGMENT_ROWS + 1, dtype=torch.int32, device="cpu")
             table = rows.to(device)
             if type(table) is torch.Tensor:
                 table = _SEGMENT_TABLES.setdefault(device, table)

@@ -160,13 +160,15 @@ def test_ops_reject_cpu_tensors():
 
 def test_whole_batch_segments_are_rows_of_one_table_and_plain_tensors():
     """[0, T] for any number of batch sizes without a tensor each, and nothing kept of a fake
-    mode's tensors."""
+    mode's tensors; made on the host whatever the default device."""
     from torch._subclasses.fake_tensor import FakeTensorMode
     from nexttransformer_amd import ops
     cpu = torch.device("cpu")
     with FakeTensorMode():
         ops._whole_batch_segment(5, cpu)
         ops._whole_batch_segment(ops._SEGMENT_ROWS + 5, cpu)
+    with torch.device("meta"):
+        assert ops._whole_batch_segment(9, cpu).tolist() == [0, 9]
     sizes = [0, 1, 5, ops._SEGMENT_ROWS, ops._SEGMENT_ROWS + 1, ops._SEGMENT_ROWS + 5]
     for T in sizes + list(range(1000, 2200)) + sizes:
         seg = ops._whole_batch_segment(T, cpu)
